@@ -239,9 +239,10 @@ int         sl_set_raster_config(sl_context* ctx, int config);
  * with more than 4 * partRecords records is split into parts of about
  * partRecords records (at most 1024 parts) rasterised by separate workgroups
  * and merged exactly.  By default batches with point or line draws split
- * with parts of 256 records; sl_set_raster_split(n > 0) splits every such
- * batch with parts of n records, 0 turns the split off.  Results never
- * depend on it. */
+ * with parts of 256 records; sl_set_raster_split(n > 0) splits these and
+ * wireframe batches with parts of n records, 0 turns the split off.  Batches
+ * of filled triangles alone never split (their raster's work items are 8x8
+ * pixel blocks).  Results never depend on it. */
 int         sl_set_raster_split(sl_context* ctx, uint32_t partRecords);
 #define SL_RASTER_SPLIT_DEFAULT 0xFFFFFFFFu   /* sl_set_raster_split: back to the default policy */
 /* Occupancy (no counterpart in the reference): caps the raster workgroups
@@ -249,13 +250,11 @@ int         sl_set_raster_split(sl_context* ctx, uint32_t partRecords);
  * kernel's registers and LDS allow) by giving each workgroup that share of
  * the CU's LDS.  Results never depend on it. */
 int         sl_set_raster_occupancy(sl_context* ctx, uint32_t workgroupsPerCU);
-/* Depth rejection (no counterpart in the reference): with enable non-zero,
- * batches of filled triangles without a visibility attachment use the
- * raster variant that skips, for each wave of a tile holding 64 or more
- * records, the records whose depth provably fails a LESS / LESS_EQUAL test
- * at every pixel the wave owns (R_FLOAT depth targets only; such records
- * only count their depth tests).  Off by default: it pays off where depth
- * complexity is high.  Results never depend on it. */
+/* Depth rejection (no counterpart in the reference): the raster of batches
+ * of filled triangles skips, for each 8x8 pixel block, the records whose depth
+ * provably fails a LESS / LESS_EQUAL test at every pixel of the block (such
+ * records only count their depth tests), whatever this switch says: it is
+ * kept for callers that set it, and results never depended on it. */
 int         sl_set_raster_depth_reject(sl_context* ctx, int enable);
 int         sl_get_raster_config(const sl_context* ctx, int config, int* tileW, int* tileH, int* segments);
 

@@ -62,7 +62,8 @@ SL_HD int ilog2i(int v) { int r = 0; while ((1 << r) < v) ++r; return r; }
 // value x86 cvttss2si produces for the reference's (int32_t) casts.
 SL_HD int32_t f2i(float f)
 {
-    return (f >= -2147483648.0f && f < 2147483648.0f) ? (int32_t)f : INT32_MIN;
+    // (-2^31 itself converts to INT32_MIN too: one comparison serves both ends)
+    return (fabsf(f) < 2147483648.0f) ? (int32_t)f : INT32_MIN;
 }
 
 SL_HD float rcpf(float x) { return 1.0f / x; }
@@ -463,6 +464,7 @@ struct RasterParams
     float clearDepthValue;
     int32_t extra;                // some draw of the batch draws wireframe triangles, lines or points
     int32_t mrt;                  // some draw of the batch has several fragment outputs
+    int32_t blend;                // some draw of the batch with outputs blends them
     FrameCtrl* ctrl;
     // heavy-tile split (items == nullptr: one workgroup per tile, tileOrder)
     const RasterItem* items;      // whole tiles and parts of split tiles, parts first

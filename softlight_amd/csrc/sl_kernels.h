@@ -30,17 +30,20 @@ hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const Fram
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items = nullptr,
                           uint32_t* itemCount = nullptr, uint32_t* partDone = nullptr, uint32_t partRecs = 1,
                           uint32_t splitAbove = 0, uint32_t maxParts = 0);
-// reject: the filled-triangle variants (plain and debug) with depth rejection (k_raster AUX bit 4)
-hipError_t launch_raster(const RasterParams& p, int numTiles, int cfg, bool debug, hipStream_t s, bool reject = false);
-// k_raster of one colour format (CF: 0 none, 1 8-bit/packed, 2 float) and
-// variant (AUX bits, see k_raster) on tile configuration `cfg`; defined in
-// sl_raster_impl.h and instantiated in the sl_raster_*.hip units.
+hipError_t launch_raster(const RasterParams& p, int numTiles, int cfg, bool debug, hipStream_t s);
+// k_raster (batches with wireframe, line or point records) of one colour
+// format (CF: 0 none, 1 8-bit/packed, 2 float) and variant (AUX bits, see
+// k_raster) on tile configuration `cfg`; defined in sl_raster_impl.h and
+// instantiated in the sl_raster_m*.hip units.
 template <int CF, int AUX>
 void launch_raster_cfg(const RasterParams& p, int grid, int cfg, hipStream_t s);
+// k_raster_wave (batches of filled triangles, no split) of one colour format
+// and variant, on tiles of 2^shx x 2^shy pixels; defined in sl_raster_wave.h.
+template <int CF, int AUX>
+void launch_raster_wave_cfg(const RasterParams& p, int numTiles, int shx, int shy, hipStream_t s);
 // The heavy-tile split's first pass (k_raster MODE 1) on tile configuration
-// `cfg`, over the parts of split tiles; EXTRA: the batch holds wireframe,
-// line or point records.
-template <int EXTRA>
+// `cfg`, over the parts of split tiles (CF 0: it touches no colour).
+template <int CF>
 void launch_raster_depth_cfg(const RasterParams& p, int grid, int cfg, hipStream_t s);
 hipError_t launch_raster_depth(const RasterParams& p, int grid, int cfg, hipStream_t s);
 

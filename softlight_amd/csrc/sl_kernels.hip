@@ -2086,71 +2086,75 @@ hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const Fram
 hipError_t launch_raster_depth(const RasterParams& p, int grid, int cfg, hipStream_t s)
 {
     (void)hipGetLastError();   // drop a stale error from an earlier call
-    if (p.extra) launch_raster_depth_cfg<1>(p, grid, cfg, s);
-    else launch_raster_depth_cfg<0>(p, grid, cfg, s);
+    launch_raster_depth_cfg<0>(p, grid, cfg, s);
     return hipGetLastError();
 }
 
-hipError_t launch_raster(const RasterParams& p, int numTiles, int cfg, bool debug, hipStream_t s, bool reject)
+// Batches of filled triangles: k_raster_wave.
+static hipError_t launch_raster_wave(const RasterParams& p, int cf, int numTiles, int cfg, bool debug, hipStream_t s)
+{
+    const int shx = ilog2i(kTileConfigs[cfg].tileW), shy = ilog2i(kTileConfigs[cfg].tileH);
+    const bool bl = p.blend != 0;
+    if (p.vis != nullptr)
+    {
+        // the visibility attachment is only built for RGBA32F colour targets
+        // and single-output programs
+        if (cf != 2 || p.mrt) return hipErrorInvalidValue;
+        if (debug) launch_raster_wave_cfg<2, 35>(p, numTiles, shx, shy, s);
+        else if (bl) launch_raster_wave_cfg<2, 34>(p, numTiles, shx, shy, s);
+        else launch_raster_wave_cfg<2, 2>(p, numTiles, shx, shy, s);
+    }
+    else if (p.mrt)
+    {
+        if (cf == 0) return hipErrorInvalidValue;   // outputs need colour attachment 0
+        if (debug && cf == 1) launch_raster_wave_cfg<1, 41>(p, numTiles, shx, shy, s);
+        else if (debug) launch_raster_wave_cfg<2, 41>(p, numTiles, shx, shy, s);
+        else if (cf == 1 && bl) launch_raster_wave_cfg<1, 40>(p, numTiles, shx, shy, s);
+        else if (cf == 1) launch_raster_wave_cfg<1, 8>(p, numTiles, shx, shy, s);
+        else if (bl) launch_raster_wave_cfg<2, 40>(p, numTiles, shx, shy, s);
+        else launch_raster_wave_cfg<2, 8>(p, numTiles, shx, shy, s);
+    }
+    else if (cf == 0)
+    {
+        if (debug) launch_raster_wave_cfg<0, 1>(p, numTiles, shx, shy, s);
+        else launch_raster_wave_cfg<0, 0>(p, numTiles, shx, shy, s);
+    }
+    else if (cf == 1)
+    {
+        if (debug) launch_raster_wave_cfg<1, 33>(p, numTiles, shx, shy, s);
+        else if (bl) launch_raster_wave_cfg<1, 32>(p, numTiles, shx, shy, s);
+        else launch_raster_wave_cfg<1, 0>(p, numTiles, shx, shy, s);
+    }
+    else
+    {
+        if (debug) launch_raster_wave_cfg<2, 33>(p, numTiles, shx, shy, s);
+        else if (bl) launch_raster_wave_cfg<2, 32>(p, numTiles, shx, shy, s);
+        else launch_raster_wave_cfg<2, 0>(p, numTiles, shx, shy, s);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_raster(const RasterParams& p, int numTiles, int cfg, bool debug, hipStream_t s)
 {
     (void)hipGetLastError();   // drop a stale error from an earlier call
     const bool floatColor = p.colorType == SL_COLOR_R_FLOAT || p.colorType == SL_COLOR_RG_FLOAT ||
                             p.colorType == SL_COLOR_RGB_FLOAT || p.colorType == SL_COLOR_RGBA_FLOAT;
     const int cf = (p.color == nullptr) ? 0 : (floatColor ? 2 : 1);
-    if (p.vis != nullptr)
-    {
-        // the visibility attachment is only built for RGBA32F colour targets
-        // and filled triangles
-        if (cf != 2 || p.extra || p.mrt) return hipErrorInvalidValue;
-        if (debug) launch_raster_cfg<2, 3>(p, numTiles, cfg, s);
-        else launch_raster_cfg<2, 2>(p, numTiles, cfg, s);
-    }
-    else if (p.mrt)
+    if (!p.extra) return launch_raster_wave(p, cf, numTiles, cfg, debug, s);
+    if (p.vis != nullptr) return hipErrorInvalidValue;   // built for filled triangles only
+    if (p.mrt)
     {
         if (cf == 0) return hipErrorInvalidValue;   // outputs need colour attachment 0
-        if (debug)
-        {
-            if (cf == 1) launch_raster_cfg<1, 13>(p, numTiles, cfg, s);
-            else launch_raster_cfg<2, 13>(p, numTiles, cfg, s);
-        }
-        else
-        {
-            if (cf == 1) launch_raster_cfg<1, 12>(p, numTiles, cfg, s);
-            else launch_raster_cfg<2, 12>(p, numTiles, cfg, s);
-        }
-    }
-    else if (p.extra)
-    {
-        if (debug)
-        {
-            if (cf == 0) launch_raster_cfg<0, 5>(p, numTiles, cfg, s);
-            else if (cf == 1) launch_raster_cfg<1, 5>(p, numTiles, cfg, s);
-            else launch_raster_cfg<2, 5>(p, numTiles, cfg, s);
-        }
-        else
-        {
-            if (cf == 0) launch_raster_cfg<0, 4>(p, numTiles, cfg, s);
-            else if (cf == 1) launch_raster_cfg<1, 4>(p, numTiles, cfg, s);
-            else launch_raster_cfg<2, 4>(p, numTiles, cfg, s);
-        }
-    }
-    else if (debug && reject)
-    {
-        if (cf == 0) launch_raster_cfg<0, 17>(p, numTiles, cfg, s);
-        else if (cf == 1) launch_raster_cfg<1, 17>(p, numTiles, cfg, s);
-        else launch_raster_cfg<2, 17>(p, numTiles, cfg, s);
+        if (debug && cf == 1) launch_raster_cfg<1, 9>(p, numTiles, cfg, s);
+        else if (debug) launch_raster_cfg<2, 9>(p, numTiles, cfg, s);
+        else if (cf == 1) launch_raster_cfg<1, 8>(p, numTiles, cfg, s);
+        else launch_raster_cfg<2, 8>(p, numTiles, cfg, s);
     }
     else if (debug)
     {
         if (cf == 0) launch_raster_cfg<0, 1>(p, numTiles, cfg, s);
         else if (cf == 1) launch_raster_cfg<1, 1>(p, numTiles, cfg, s);
         else launch_raster_cfg<2, 1>(p, numTiles, cfg, s);
-    }
-    else if (reject)
-    {
-        if (cf == 0) launch_raster_cfg<0, 16>(p, numTiles, cfg, s);
-        else if (cf == 1) launch_raster_cfg<1, 16>(p, numTiles, cfg, s);
-        else launch_raster_cfg<2, 16>(p, numTiles, cfg, s);
     }
     else
     {

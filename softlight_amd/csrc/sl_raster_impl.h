@@ -27,8 +27,6 @@ namespace {
 // Catch-up distances up to kStepLimit groups are stepped; longer ones use the
 // binade jump (one out-of-line copy for the three barycentric components).
 constexpr int kStepLimit = 256;
-// Depth rejection (AUX bit 4) runs on tiles (or parts) of at least this many records.
-constexpr int kHizMinRecs = 64;
 
 __device__ __noinline__ float3 recur_advance3(float3 s, float3 d, int k)
 {
@@ -323,13 +321,10 @@ constexpr uint32_t kNoPending = 0xFFFFFFFFu;
 // miss its rows with one uniform test) and never touches another wave's
 // pixels, so no workgroup barrier is needed between records.
 //
-// AUX bit 0: debug buffers (last primitive, depth-pass count); bit 1: the
-// visibility attachment; bit 2: the batch holds wireframe, line or point
-// records (the variants without it carry only the filled-triangle code);
-// bit 3: the batch has draws with several fragment outputs (launched with
-// bit 2 set); bit 4: depth rejection of records that fail every depth test
-// in a wave (filled triangles, LESS / LESS_EQUAL; results are identical with
-// it and without it).
+// Launched for batches that hold wireframe, line or point records (filled
+// triangles among them); batches of filled triangles run k_raster_wave.
+// AUX bit 0: debug buffers (last primitive, depth-pass count); bit 3: the
+// batch has draws with several fragment outputs.
 //
 // Heavy tiles (RasterParams::items): a workgroup takes a work item, a whole
 // tile or one part of a split tile's record list.  MODE 1 walks a part from
@@ -344,10 +339,7 @@ template <int CF, int AUX, int TW, int TH, int SEGS, int MODE>
 __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
 {
     constexpr bool DBG = (AUX & 1) != 0;
-    constexpr bool VIS = (AUX & 2) != 0;
-    constexpr bool EXTRA = (AUX & 4) != 0;
     constexpr bool MRT = (AUX & 8) != 0;
-    constexpr bool HIZ = (AUX & 16) != 0;
     constexpr int NT = TH * 4 * SEGS;       // lanes: rows x segments x 4 phases
     constexpr int NW = NT / 64;             // waves, each owning TH / NW rows
     constexpr int SW = TW / SEGS;           // segment width (columns)
@@ -358,7 +350,6 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
     __shared__ float4 sColF[CF == 2 ? TH : 1][TW];
     __shared__ uint32_t sLast[DBG ? TH : 1][TW];
     __shared__ uint32_t sCount[DBG ? TH : 1][TW];
-    __shared__ float4 sVis[VIS ? TH : 1][TW];
     __shared__ uint32_t sPend[TH][TW];                  // pending fragment's record, or kNoPending
     __shared__ float sPendS[3][TH][TW];                 // its barycentric values
 
@@ -413,7 +404,6 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
                 sLast[r][c] = P.clearDepth ? 0u : (inb ? P.dbgLast[gi] : 0u);
                 sCount[r][c] = P.clearDepth ? 0u : (inb ? P.dbgCount[gi] : 0u);
             }
-            if (VIS) sVis[r][c] = (P.clearDepth || !inb) ? make_float4(0.f, 0.f, 0.f, 0.f) : P.vis[gi];
             sPend[r][c] = kNoPending;
         }
     };
@@ -463,7 +453,6 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
         const bool have = shade<MRT>(P, QD, qhw, Q.bc3, Q.state, prid, sPendS[0][r][c], sPendS[1][r][c], sPendS[2][r][c], out, wv,
                                 (uint64_t)(y0 + r) * P.W + (x0 + c), SL_BLEND_OFF);
         if (have) blend_into<CF>(&sCol8[CF == 1 ? r : 0][CF == 1 ? c : 0], &sColF[CF == 2 ? r : 0][CF == 2 ? c : 0], SL_BLEND_OFF, out, P.colorComps, P.colorPacked);
-        if (VIS) sVis[r][c] = make_float4(__uint_as_float(Q.seq), wv.x, wv.y, wv.z);
     };
 
     // lane = (row, segment, phase): the lane owns the columns x = phase (mod 4)
@@ -482,9 +471,6 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
     // one batch ahead) are issued before the current batch is processed, so
     // their latency hides behind the raster work.
     constexpr int kBatch = 16;
-    // depth rejection (below) on tiles of at least kHizMinRecs records:
-    // lighter tiles reject too little to pay for the bound's reduction
-    const bool hiz = HIZ && !P.depthHalf && range.y - range.x >= (uint32_t)kHizMinRecs;
     constexpr int kRecWords = sizeof(SetupRec) / 4;
     constexpr int kLaneWords = kBatch * kRecWords / 64;
     static_assert(kBatch * kRecWords % 64 == 0 && kBatch < 32, "record staging; 32-bit record masks");
@@ -537,25 +523,6 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
         // of the image's edge) meet its column box -- and every lane takes
         // its own bit of each record's mask (read from lane r's registers).
         uint64_t hitMask = 0;
-        // Depth rejection.  zTop: the greatest depth the wave's pixels hold at
-        // the batch's start (float depth only: an R16F write rounds, which can
-        // land above a clear value that is not a half).  Depth tests LESS and
-        // LESS_EQUAL only lower a pixel's depth, so zTop bounds it for every
-        // record of the batch before the first one that can raise it (depth
-        // writes with the test off, GREATER(_EQUAL) or NOT_EQUAL).  A filled
-        // triangle with a LESS(_EQUAL) test whose computed depth provably
-        // exceeds zTop at every pixel of the wave it can reach fails each of
-        // its depth tests: it leaves every lane's walk (rejMask), and lane r
-        // counts record r's tests over the wave instead.
-        float zTop = -INFINITY;
-        if (HIZ && hiz)
-        {
-#pragma unroll
-            for (int k = 0; k < SW / 4; ++k) zTop = fmaxf(zTop, sDepth[row][seg * SW + phase + 4 * k]);
-            zTop = wave_max_f32(zTop);
-        }
-        bool rej = false, raise = false;
-        uint32_t rejTested = 0;   // depth tests of this lane's record in the wave, if it is rejected
         if (wl < nb)
         {
             const SetupRec& R = sRec[wl];
@@ -576,75 +543,10 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
 #pragma unroll
             for (int sg = 0; sg < SEGS; ++sg) colBits |= ((g >> (sg * SW)) & 0xFull) << (sg * 4);
             hitMask = colBits * rowsel;   // colBits < 2^LPR: the row copies do not overlap
-            const uint32_t rst = R.state;
-            const int rdt = (int)(rst & 7u);
-            raise = HIZ && ((rst >> 3) & 1u) != 0u &&
-                    (rdt == SL_DEPTH_TEST_OFF || rdt == SL_DEPTH_TEST_GREATER_THAN ||
-                     rdt == SL_DEPTH_TEST_GREATER_EQUAL || rdt == SL_DEPTH_TEST_NOT_EQUAL);
-            if (HIZ && hiz && hitMask != 0ull && (rst & (kStateWire | kStateLine | kStatePoint)) == 0u &&
-                (rdt == SL_DEPTH_TEST_LESS_THAN || rdt == SL_DEPTH_TEST_LESS_EQUAL))
-            {
-                // The lane computes s_i = fl(x bx_i + fma(by_i, y, bz_i)), then
-                // s_i += 4 bx_i per group up to its pixel (at most X / 4 + 1
-                // steps from the span's start, x >= 0), and z = sum z_i s_i.
-                // With A_i = X |bx_i| + Y |by_i| + |bz_i| (>= |S_i| and each
-                // product term over 0 <= x <= X, 0 <= y <= Y) every rounding
-                // of that chain and of the corner values below is at most
-                // 2^-24 A_i, so the computed depth of any pixel in the
-                // rectangle lies within sum |z_i| A_i 2^-24 (X / 4 + 13) of
-                // the plane's exact value, whose minimum is at a corner.
-                const float xa = (float)(x0 + jlo), xb = (float)(x0 + jhi);
-                const float ya = (float)(wy0 + r0), yb = (float)(wy0 + r1);
-                float zlo = INFINITY, mag = 0.f;
-                float zc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-                {
-                    const float bxi = R.bx[i], byi = R.by[i], bzi = R.bz[i], zi = R.z[i];
-                    const float v = fmaf(byi, ya, bzi), w = fmaf(byi, yb, bzi);
-                    zc[0] = fmaf(zi, fmaf(bxi, xa, v), zc[0]);
-                    zc[1] = fmaf(zi, fmaf(bxi, xb, v), zc[1]);
-                    zc[2] = fmaf(zi, fmaf(bxi, xa, w), zc[2]);
-                    zc[3] = fmaf(zi, fmaf(bxi, xb, w), zc[3]);
-                    mag = fmaf(fabsf(zi), fmaf(xb, fabsf(bxi), fmaf(yb, fabsf(byi), fabsf(bzi))), mag);
-                }
-                zlo = fminf(fminf(zc[0], zc[1]), fminf(zc[2], zc[3]));
-                // twice the bound above, and NaN / infinite terms never reject
-                const float margin = mag * (5.9604645e-8f * (2.f * (0.25f * xb + 13.f))) * 1.0625f;
-                rej = (zlo - margin) > zTop;
-                if (rej && MODE != 1)
-                {
-                    // its depth tests in the wave: per row, the span's pixels
-                    // in the tile and the image (every lane's share of the
-                    // row's columns, as the walk would count them)
-                    const int xr = min(x0 + TW, P.W);
-                    for (int r = r0; r <= r1; ++r)
-                    {
-                        int32_t xMin, xMax;
-                        scanline_step(R, (float)(wy0 + r), xMin, xMax);
-                        if ((uint32_t)xMin < (uint32_t)xMax)
-                        {
-                            const int a = max((int)xMin, x0), b = min((int)xMax, xr);
-                            if (a < b) rejTested += (uint32_t)(b - a);
-                        }
-                    }
-                }
-            }
         }
-        uint32_t rejMask = 0;
-        if constexpr (HIZ)
-        {
-            // records before the batch's first depth-raising record
-            const uint64_t rb = __ballot(raise);
-            const uint64_t before = (rb != 0ull) ? ((1ull << (__ffsll((unsigned long long)rb) - 1)) - 1ull) : ~0ull;
-            rejMask = (uint32_t)(__ballot(rej) & before);
-            if (wl < kBatch && ((rejMask >> wl) & 1u)) tested += rejTested;
-        }
-        // only the records that reach some lane of the wave (and, with
-        // rejection, are left after it: rejected ones are counted above)
+        // only the records that reach some lane of the wave
         uint32_t cand = 0;
         uint32_t todo = (uint32_t)__ballot(hitMask != 0ull);   // lanes nb.. hold no mask
-        if constexpr (HIZ) todo &= ~rejMask;
         for (; todo != 0u; todo &= todo - 1u)
         {
             const int bi = __ffs(todo) - 1;
@@ -668,9 +570,8 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
             const bool dmask = ((st >> 3) & 1u) != 0;
             const int blendMode = (int)((st >> 4) & 7u);
             const bool hasOut = ((st >> 7) & 1u) != 0;
-            // deferred: unblended fragments with outputs, and any
-            // fragment whose visibility record is wanted
-            const bool defer = (hasOut && blendMode == SL_BLEND_OFF) || (VIS && !hasOut);
+            // deferred: unblended fragments with outputs
+            const bool defer = hasOut && blendMode == SL_BLEND_OFF;
             // depth test and fragment work of this lane's pixel x of row y;
             // s0..s2 are a triangle's barycentrics, a line's position
             // along it (s0)
@@ -702,7 +603,6 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
                                                 (uint64_t)y * P.W + x, blendMode);
                         if (have) blend_into<CF>(&sCol8[CF == 1 ? row : 0][CF == 1 ? c : 0],
                                                  &sColF[CF == 2 ? row : 0][CF == 2 ? c : 0], blendMode, out, P.colorComps, P.colorPacked);
-                        if (VIS) sVis[row][c] = make_float4(__uint_as_float(R.seq), wv.x, wv.y, wv.z);
                     }
                     if (dmask) sDepth[row][c] = P.depthHalf ? __half2float(__float2half_rn(z)) : z;
                     if (DBG)
@@ -713,7 +613,7 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
                     ++shaded;
                 }
             };
-            if (EXTRA && (st & (kStateLine | kStatePoint)) != 0u)
+            if ((st & (kStateLine | kStatePoint)) != 0u)
             {
                 // This lane's texels of a point or line: columns x, x + 4,
                 // ... up to xe of row y, and for a line the walk's texel
@@ -792,7 +692,7 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
                 // This lane's pixels: x, x + 4, ... below xe, then those of
                 // a second run [xn, xen) (wireframe).  One loop serves both
                 // kinds so the fragment work is inlined once.
-                const bool wire = EXTRA && (st & kStateWire) != 0u;
+                const bool wire = (st & kStateWire) != 0u;
                 int x, xe, xn = 0, xen = 0;
                 float s0, s1, s2, d0, d1, d2;
                 if (wire)
@@ -1005,7 +905,6 @@ __global__ __launch_bounds__(TH * 4 * SEGS) void k_raster(RasterParams P)
                 P.dbgLast[gi] = sLast[r][c];
                 P.dbgCount[gi] = sCount[r][c];
             }
-            if (VIS) P.vis[gi] = sVis[r][c];
         }
     }
 
@@ -1097,9 +996,9 @@ static void launch_raster_mode(const RasterParams& p, int grid, int cfg, hipStre
         case 9: launch_raster_shape<CF, AUX, 32, 8, 8, MODE>(p, grid, s); break;
         case 10: launch_raster_shape<CF, AUX, 8, 8, 2, MODE>(p, grid, s); break;
         case 11:
-            // the runtime maps configuration 11 to kLargeTileFallback for the
-            // variants whose 64x64 tile does not fit in LDS (effective_tile_config)
-            if constexpr (CF != 2 && (AUX & 2) == 0) launch_raster_shape<CF, AUX, 64, 64, 1, MODE>(p, grid, s);
+            // the runtime maps configuration 11 to kLargeTileFallback for float
+            // colour, whose 64x64 tile does not fit in LDS (effective_tile_config)
+            if constexpr (CF != 2) launch_raster_shape<CF, AUX, 64, 64, 1, MODE>(p, grid, s);
             else launch_raster_shape<CF, AUX, 32, 32, 2, MODE>(p, grid, s);
             break;
         default: launch_raster_shape<CF, AUX, 32, 16, 1, MODE>(p, grid, s); break;
@@ -1112,12 +1011,11 @@ void launch_raster_cfg(const RasterParams& p, int grid, int cfg, hipStream_t s)
     launch_raster_mode<CF, AUX, 0>(p, grid, cfg, s);
 }
 
-// The first pass over split tiles' parts (MODE 1); EXTRA: the batch holds
-// wireframe, line or point records.
-template <int EXTRA>
+// The first pass over split tiles' parts (MODE 1).
+template <int CF>
 void launch_raster_depth_cfg(const RasterParams& p, int grid, int cfg, hipStream_t s)
 {
-    launch_raster_mode<0, EXTRA ? 4 : 0, 1>(p, grid, cfg, s);
+    launch_raster_mode<CF, 0, 1>(p, grid, cfg, s);
 }
 static_assert(kTileConfigs[0].tileW == 32 && kTileConfigs[0].tileH == 16 && kTileConfigs[0].segs == 1 &&
               kTileConfigs[1].tileW == 32 && kTileConfigs[1].tileH == 8 && kTileConfigs[1].segs == 2 &&

@@ -3,8 +3,8 @@
 
 namespace slg {
 
-template void launch_raster_cfg<0, 5>(const RasterParams&, int, int, hipStream_t);
-template void launch_raster_cfg<1, 5>(const RasterParams&, int, int, hipStream_t);
-template void launch_raster_cfg<2, 5>(const RasterParams&, int, int, hipStream_t);
+template void launch_raster_cfg<0, 1>(const RasterParams&, int, int, hipStream_t);
+template void launch_raster_cfg<1, 1>(const RasterParams&, int, int, hipStream_t);
+template void launch_raster_cfg<2, 1>(const RasterParams&, int, int, hipStream_t);
 
 }  // namespace slg

@@ -263,7 +263,6 @@ struct sl_context
     uint32_t splitRecs = kDefaultSplitRecords;   // heavy-tile split: records per part (0: off)
     bool splitAll = false;                       // split triangle-only batches too (sl_set_raster_split)
     uint32_t wgPerCU = 0;                        // raster occupancy cap (sl_set_raster_occupancy; 0: none)
-    bool depthReject = false;                    // sl_set_raster_depth_reject
     uint32_t triSeq = 0;
     sl_frame_stats stats{};
     std::string err;
@@ -471,10 +470,16 @@ uint32_t split_class(const Batch& B, const Plan& p, bool all)
 {
     if (B.draws.empty() || p.dt->type != SL_COLOR_R_FLOAT) return kSplitNone;
     // by default only batches with point or line draws, whose records pile
-    // onto few tiles (a distant mesh's vertices); triangle batches when asked
-    bool prims = false;
-    for (const DrawDesc& d : B.draws) prims = prims || d.prim == kPrimPoint || d.prim == kPrimLine;
-    if (!all && !prims) return kSplitNone;
+    // onto few tiles (a distant mesh's vertices); wireframe batches when
+    // asked.  Batches of filled triangles never split: k_raster_wave's waves
+    // are 8x8 blocks and it drops hidden records 64 at a time
+    bool prims = false, wire = false;
+    for (const DrawDesc& d : B.draws)
+    {
+        prims = prims || d.prim == kPrimPoint || d.prim == kPrimLine;
+        wire = wire || d.prim == kPrimWire;
+    }
+    if (!prims && !(all && wire)) return kSplitNone;
     const DrawDesc& d0 = B.draws[0];
     for (const DrawDesc& d : B.draws)
         if (d.blend != SL_BLEND_OFF || d.dtest != d0.dtest || d.dmask != d0.dmask) return kSplitNone;
@@ -600,10 +605,12 @@ RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool have
     rp.clearDepthValue = rp.depthHalf ? host_half_to_float(host_float_to_half((float)B.depth)) : (float)B.depth;
     rp.extra = 0;
     rp.mrt = 0;
+    rp.blend = 0;
     for (const DrawDesc& d : B.draws)
     {
         rp.extra |= (d.prim != kPrimFill) ? 1 : 0;
         rp.mrt |= (d.nout > 1) ? 1 : 0;
+        rp.blend |= (d.nout > 0 && d.blend != SL_BLEND_OFF) ? 1 : 0;
     }
     rp.ctrl = reinterpret_cast<FrameCtrl*>(R.ctrl.p);
     rp.items = nullptr;
@@ -700,9 +707,9 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
         // the device)
         if (rp.splitClass != kSplitConst && (rc = check(c, launch_raster_depth(rp, (int)R.maxParts, p.cfg, s), "k_raster depth pass")) != SL_OK)
             return rc;
-        return check(c, launch_raster(rp, p.numTiles + (int)R.maxParts, p.cfg, p.debug, s, c->depthReject), "k_raster");
+        return check(c, launch_raster(rp, p.numTiles + (int)R.maxParts, p.cfg, p.debug, s), "k_raster");
     }
-    return check(c, launch_raster(rp, p.numTiles, p.cfg, p.debug, s, c->depthReject), "k_raster");
+    return check(c, launch_raster(rp, p.numTiles, p.cfg, p.debug, s), "k_raster");
 }
 
 int upload_batch(sl_context* c, FrameRes& R, const Batch& B, hipStream_t s)
@@ -1495,10 +1502,8 @@ int sl_set_raster_occupancy(sl_context* c, uint32_t workgroupsPerCU)
 int sl_set_raster_depth_reject(sl_context* c, int enable)
 {
     if (!c) return SL_ERR_INVALID_ARG;
-    const int rc = flush(c);
-    if (rc != SL_OK) return rc;
-    c->depthReject = enable != 0;
-    return SL_OK;
+    (void)enable;   // every batch of filled triangles rejects (k_raster_wave)
+    return flush(c);
 }
 
 int sl_get_raster_config(const sl_context* c, int config, int* tileW, int* tileH, int* segments)

@@ -484,9 +484,18 @@ __device__ __forceinline__ void setup_record(float4 p0, float4 p1, float4 p2, ui
     r.p10xy = (bxx - ax) * rcpf(byy - ay);
 }
 
+// A record's scanline constants, apart from the rest of it.
+struct ScanEdges { float v0y, v1y, v0x, v1x, p20y, p20x, p21xy, p10xy; };
+
+__device__ __forceinline__ ScanEdges scan_edges(const SetupRec& r)
+{
+    return ScanEdges{r.v0y, r.v1y, r.v0x, r.v1x, r.p20y, r.p20x, r.p21xy, r.p10xy};
+}
+
 // SL_ScanlineBounds::step, generic branch (:310-322); only the selected edge
 // is converted (the other may be +-inf or NaN).
-__device__ __forceinline__ void scanline_step(const SetupRec& r, float yf, int32_t& xMin, int32_t& xMax)
+template <class Edges>   // SetupRec or ScanEdges
+__device__ __forceinline__ void scanline_step(const Edges& r, float yf, int32_t& xMin, int32_t& xMax)
 {
     const float d0 = yf - r.v0y;
     const float d1 = yf - r.v1y;

@@ -1,0 +1,71 @@
+"""The raster of filled-triangle batches (one wave per 8x8 pixel block) at the
+sizes where it can go wrong, against the CPU oracle bit for bit (depth,
+per-pixel order and counts; colour within 1 LSB):
+
+  targets      smaller than a block, one pixel past it, ragged in both axes,
+               and wide enough (> 1,028 columns) that a fragment's barycentrics
+               are advanced by the exact jump instead of stepping
+  lists        63, 64, 65 and 129 records in a tile (64 are taken at a time)
+  queue        more than 64 waiting fragments of one record and of one pixel
+  depth        the seven functions mixed in one batch, with depth-raising draws
+               between LESS draws, into float and half depth, and with blending
+"""
+import numpy as np
+import pytest
+
+from softlight_amd import api as A
+from softlight_amd import scenes
+from tests.parity import assert_parity, render_both
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("size", [(1, 1), (7, 5), (8, 8), (9, 8), (8, 9), (33, 17), (64, 64), (1500, 20)])
+@pytest.mark.parametrize("blend", [A.SL_BLEND_OFF, A.SL_BLEND_ALPHA])
+def test_target_sizes(gpu_lib, oracle_lib, size, blend):
+    g, o = render_both(gpu_lib, oracle_lib, scenes.build_random_triangles, seed=21, ntri=150, W=size[0], H=size[1],
+                       debug=True, blend=blend)
+    assert_parity(g, o)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 129])
+@pytest.mark.parametrize("config", [0, 3, 10, 11])
+def test_list_lengths(gpu_lib, oracle_lib, n, config):
+    """n triangles that each cover the whole target, nearer and nearer: every
+    one is in every tile's list, covers whole blocks and passes."""
+    def build(ctx):
+        ctx.set_raster_config(config)
+        rec = np.zeros((3 * n, 16), dtype=np.uint8)
+        xyz = np.empty((n, 3, 3), dtype=np.float32)
+        xyz[:] = [[-1.0, -1.0, 0.0], [1.0, -1.0, 0.0], [-1.0, 1.0, 0.0]]
+        xyz[1::2, :, :2] *= -1.0                       # both halves of the target
+        xyz[:, :, 2] = np.linspace(0.9, -0.9, n, dtype=np.float32)[:, None]
+        xyz[:, 1, 2] += 0.05                           # slanted in depth
+        rec[:, 0:12] = xyz.reshape(-1, 3).view(np.uint8).reshape(3 * n, 12)
+        rec[:, 12:16] = scenes.uniform_u8(5, 12 * n, stream=3).reshape(3 * n, 4)
+        return scenes.build_from_vertex_records(ctx, rec, 70, 45, True)
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
+
+
+@pytest.mark.parametrize("depth_type", [A.SL_COLOR_R_FLOAT, A.SL_COLOR_R_HALF])
+@pytest.mark.parametrize("blend", [A.SL_BLEND_OFF, A.SL_BLEND_ADDITIVE])
+def test_depth_functions_in_one_batch(gpu_lib, oracle_lib, depth_type, blend):
+    """Twelve draws of 60 triangles, each of another depth function and mask:
+    LESS draws after GREATER, NOT_EQUAL and test-off draws see raised depths."""
+    def build(ctx):
+        s = scenes.build_from_vertex_records(ctx, scenes.random_triangle_vertices(31, 720), 93, 61, True,
+                                             depth_type=depth_type)
+        vao = s.draws[0][1].vaoId
+        s.draws = []
+        tests = [A.SL_DEPTH_TEST_LESS_THAN, A.SL_DEPTH_TEST_GREATER_THAN, A.SL_DEPTH_TEST_LESS_EQUAL,
+                 A.SL_DEPTH_TEST_OFF, A.SL_DEPTH_TEST_LESS_THAN, A.SL_DEPTH_TEST_NOT_EQUAL,
+                 A.SL_DEPTH_TEST_LESS_THAN, A.SL_DEPTH_TEST_GREATER_EQUAL, A.SL_DEPTH_TEST_EQUAL,
+                 A.SL_DEPTH_TEST_LESS_THAN, A.SL_DEPTH_TEST_OFF, A.SL_DEPTH_TEST_LESS_EQUAL]
+        for k, t in enumerate(tests):
+            sh = scenes.gouraud_shader(ctx, depth_test=t, blend=blend if k % 3 == 1 else A.SL_BLEND_OFF,
+                                       depth_mask=A.SL_DEPTH_MASK_OFF if k == 4 else A.SL_DEPTH_MASK_ON)
+            s.draws.append(("draw_shader", A.sl_mesh(vao, 180 * k, 180 * (k + 1), A.RENDER_MODE_TRIANGLES, 0), sh))
+        return s
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
