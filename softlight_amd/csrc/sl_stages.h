@@ -72,8 +72,11 @@ __device__ __forceinline__ float4 read_attr(const DrawDesc& d, int bind, uint64_
         {
             if ((off & 3) == 0)
             {
+                // unrolled, so that the components' loads are in flight together
                 const auto p = gptr(reinterpret_cast<const float*>(d.vbo + off));
-                for (int i = 0; i < n; ++i) o[i] = p[i];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i < n) o[i] = p[i];
             }
             else
             {
@@ -92,7 +95,9 @@ __device__ __forceinline__ float4 read_attr(const DrawDesc& d, int bind, uint64_
         if (off >= 0 && (uint64_t)off + (uint64_t)n <= d.vboBytes)
         {
             const auto p = gptr(d.vbo + off);
-            for (int i = 0; i < n; ++i) o[i] = (float)p[i] * 0.00392156862745f;   // color_cast<float,uint8_t>, SL_Color.hpp:666-669
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (i < n) o[i] = (float)p[i] * 0.00392156862745f;   // color_cast<float,uint8_t>, SL_Color.hpp:666-669
         }
     }
     return f4(o[0], o[1], o[2], o[3]);
