@@ -211,20 +211,23 @@ struct DrawDesc
 // Screen-space triangle after setup: SL_FragmentBin (SL_ShaderUtil.hpp:627-647)
 // without the varyings, plus the per-triangle scanline constants of
 // SL_ScanlineBounds::init (SL_ScanlineBounds.hpp:137-166).
-struct SetupRec
+struct alignas(16) SetupRec
 {
-    float x[3], y[3];          // snapped screen coordinates
-    float z[3];                // NDC depth
-    float hw[3];               // 1/w
-    float bx[3], by[3], bz[3]; // barycentric planes (ddx, ddy, ddz) * denom
-    float bc3;                 // 4th barycentric component times 0 (+-0, or NaN when denom is not finite)
-    float v0y, v1y, v0x, v1x;  // scanline constants
-    float p20y, p20x, p21xy, p10xy;
+    // what the raster's 8x8 blocks filter by, in one 16-byte load
     int32_t minY, maxY;
-    uint32_t draw;
-    uint32_t seq;
     uint32_t state;            // the draw's raster state, see pack_raster_state
     uint32_t xbox;             // columns its spans can reach: min x - 1 | (max x - 1) << 16, clamped to 0..65535
+    float v0y, v1y, v0x, v1x;  // scanline constants
+    float p20y, p20x, p21xy, p10xy;
+    float bx[3];               // barycentric planes (ddx, ddy, ddz) * denom
+    float bc3;                 // 4th barycentric component times 0 (+-0, or NaN when denom is not finite)
+    float by[3];
+    uint32_t draw;
+    float bz[3];
+    uint32_t seq;
+    float z[3];                // NDC depth
+    float hw[3];               // 1/w
+    float x[3], y[3];          // snapped screen coordinates
 };
 static_assert(sizeof(SetupRec) == 144, "SetupRec layout");
 
@@ -411,19 +414,19 @@ constexpr uint32_t kMaxTileParts = 1024;        // parts of one split tile at mo
 // One raster workgroup's work: a whole tile (parts == 1) or part `part` of
 // a split tile, records [begin, end) of its list; part results live in slot
 // `slot` (the tile's parts in slots slot - part .. slot - part + parts - 1);
-// `done` counts the split tile's finished parts.
+// `split` numbers the split tiles.
 struct RasterItem
 {
     uint32_t tile;
     uint32_t begin, end;
     uint32_t slot;
     uint32_t part, parts;
-    uint32_t done;
+    uint32_t split;
     uint32_t pad;
 };
 
 // A part's result for one pixel: its last passing fragment (record or
-// kNoPart, barycentric values) and, with the parity attachments, its pass
+// kNoPending, barycentric values) and, with the parity attachments, its pass
 // count and the last passing fragment's sequence number.
 struct PartPixel
 {
@@ -432,7 +435,6 @@ struct PartPixel
     uint32_t count;
     uint32_t seq;
 };
-constexpr uint32_t kNoPart = 0xFFFFFFFFu;
 
 struct RasterParams
 {
@@ -471,7 +473,7 @@ struct RasterParams
     const uint32_t* itemCount;    // [0] items, [1] parts of split tiles (items [0, [1]))
     float* partDepth;             // per part slot, per tile pixel: the part's own depth result m
     PartPixel* partRes;           // per part slot, per tile pixel
-    uint32_t* partDone;           // per split tile: parts finished
+    uint32_t* partWin;            // per split tile, per tile pixel: 1 + the last part with a pending fragment
     uint32_t splitClass;          // kSplit*
     int32_t splitDtest;           // the batch's depth function
     uint32_t wgPerCU;             // launch: cap on resident raster workgroups per CU (0: none)

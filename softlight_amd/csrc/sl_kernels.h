@@ -28,24 +28,16 @@ BinPlan bin_plan(uint32_t entries);
 hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const FrameCtrl* ctrl, uint32_t cap,
                           BinPlan plan, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items = nullptr,
-                          uint32_t* itemCount = nullptr, uint32_t* partDone = nullptr, uint32_t partRecs = 1,
+                          uint32_t* itemCount = nullptr, uint32_t partRecs = 1,
                           uint32_t splitAbove = 0, uint32_t maxParts = 0);
-hipError_t launch_raster(const RasterParams& p, int numTiles, int cfg, bool debug, hipStream_t s);
-// k_raster (batches with wireframe, line or point records) of one colour
-// format (CF: 0 none, 1 8-bit/packed, 2 float) and variant (AUX bits, see
-// k_raster) on tile configuration `cfg`; defined in sl_raster_impl.h and
-// instantiated in the sl_raster_m*.hip units.
+// The raster of a batch: units workgroup shares, one per tile or (with
+// p.items) the most work items there can be, maxParts of them parts.
+hipError_t launch_raster(const RasterParams& p, int units, int maxParts, int cfg, bool debug, hipStream_t s);
+// k_raster_wave of one colour format (CF: 0 none, 1 8-bit/packed, 2 float)
+// and variant (AUX bits, see there) on tiles of 2^shx x 2^shy pixels; defined
+// in sl_raster_wave.h and instantiated in the sl_raster_*.hip units.
 template <int CF, int AUX>
-void launch_raster_cfg(const RasterParams& p, int grid, int cfg, hipStream_t s);
-// k_raster_wave (batches of filled triangles, no split) of one colour format
-// and variant, on tiles of 2^shx x 2^shy pixels; defined in sl_raster_wave.h.
-template <int CF, int AUX>
-void launch_raster_wave_cfg(const RasterParams& p, int numTiles, int shx, int shy, hipStream_t s);
-// The heavy-tile split's first pass (k_raster MODE 1) on tile configuration
-// `cfg`, over the parts of split tiles (CF 0: it touches no colour).
-template <int CF>
-void launch_raster_depth_cfg(const RasterParams& p, int grid, int cfg, hipStream_t s);
-hipError_t launch_raster_depth(const RasterParams& p, int grid, int cfg, hipStream_t s);
+void launch_raster_wave_cfg(const RasterParams& p, int units, int maxParts, int shx, int shy, hipStream_t s);
 
 hipError_t launch_blit(const BlitParams& p, int srcType, int dstType, hipStream_t s);
 

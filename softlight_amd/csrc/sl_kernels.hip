@@ -1647,7 +1647,6 @@ struct SplitPlan
 {
     RasterItem* items;         // null: no work items
     uint32_t* itemCount;
-    uint32_t* partDone;
     uint32_t partRecs, splitAbove, maxParts;
 };
 
@@ -1734,7 +1733,6 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
             if (j < per && t0 + j < numTiles && ((splitMask >> j) & 1u))
             {
                 const uint32_t n = tot[j], p = wanted(n);
-                SP.partDone[rc] = 0u;
                 for (uint32_t k = 0; k < p; ++k)
                 {
                     RasterItem it;
@@ -1744,7 +1742,7 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
                     it.slot = ra + k;
                     it.part = k;
                     it.parts = p;
-                    it.done = rc;
+                    it.split = rc;
                     it.pad = 0u;
                     SP.items[ra + k] = it;
                 }
@@ -1795,7 +1793,7 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
                 it.slot = 0u;
                 it.part = 0u;
                 it.parts = ((splitMask >> j) & 1u) ? 0u : 1u;   // a split tile's parts come first
-                it.done = 0u;
+                it.split = 0u;
                 it.pad = 0u;
                 SP.items[nParts + pos] = it;
             }
@@ -2068,9 +2066,9 @@ BinPlan bin_plan(uint32_t entries)
 hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const FrameCtrl* ctrl, uint32_t cap,
                           BinPlan plan, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items, uint32_t* itemCount,
-                          uint32_t* partDone, uint32_t partRecs, uint32_t splitAbove, uint32_t maxParts)
+                          uint32_t partRecs, uint32_t splitAbove, uint32_t maxParts)
 {
-    SplitPlan sp{items, itemCount, partDone, partRecs, splitAbove, maxParts};
+    SplitPlan sp{items, itemCount, partRecs, splitAbove, maxParts};
     (void)hipGetLastError();   // drop a stale error from an earlier call
     const size_t lds = sizeof(uint32_t) * (size_t)numTiles;
     hipLaunchKernelGGL(k_bin_count, dim3(plan.blocks), dim3(256), lds, s, keys, ctrl, cap, plan.per, counts, numTiles);
@@ -2083,84 +2081,31 @@ hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const Fram
     return hipGetLastError();
 }
 
-hipError_t launch_raster_depth(const RasterParams& p, int grid, int cfg, hipStream_t s)
-{
-    (void)hipGetLastError();   // drop a stale error from an earlier call
-    launch_raster_depth_cfg<0>(p, grid, cfg, s);
-    return hipGetLastError();
-}
-
-// Batches of filled triangles: k_raster_wave.
-static hipError_t launch_raster_wave(const RasterParams& p, int cf, int numTiles, int cfg, bool debug, hipStream_t s)
-{
-    const int shx = ilog2i(kTileConfigs[cfg].tileW), shy = ilog2i(kTileConfigs[cfg].tileH);
-    const bool bl = p.blend != 0;
-    if (p.vis != nullptr)
-    {
-        // the visibility attachment is only built for RGBA32F colour targets
-        // and single-output programs
-        if (cf != 2 || p.mrt) return hipErrorInvalidValue;
-        if (debug) launch_raster_wave_cfg<2, 35>(p, numTiles, shx, shy, s);
-        else if (bl) launch_raster_wave_cfg<2, 34>(p, numTiles, shx, shy, s);
-        else launch_raster_wave_cfg<2, 2>(p, numTiles, shx, shy, s);
-    }
-    else if (p.mrt)
-    {
-        if (cf == 0) return hipErrorInvalidValue;   // outputs need colour attachment 0
-        if (debug && cf == 1) launch_raster_wave_cfg<1, 41>(p, numTiles, shx, shy, s);
-        else if (debug) launch_raster_wave_cfg<2, 41>(p, numTiles, shx, shy, s);
-        else if (cf == 1 && bl) launch_raster_wave_cfg<1, 40>(p, numTiles, shx, shy, s);
-        else if (cf == 1) launch_raster_wave_cfg<1, 8>(p, numTiles, shx, shy, s);
-        else if (bl) launch_raster_wave_cfg<2, 40>(p, numTiles, shx, shy, s);
-        else launch_raster_wave_cfg<2, 8>(p, numTiles, shx, shy, s);
-    }
-    else if (cf == 0)
-    {
-        if (debug) launch_raster_wave_cfg<0, 1>(p, numTiles, shx, shy, s);
-        else launch_raster_wave_cfg<0, 0>(p, numTiles, shx, shy, s);
-    }
-    else if (cf == 1)
-    {
-        if (debug) launch_raster_wave_cfg<1, 33>(p, numTiles, shx, shy, s);
-        else if (bl) launch_raster_wave_cfg<1, 32>(p, numTiles, shx, shy, s);
-        else launch_raster_wave_cfg<1, 0>(p, numTiles, shx, shy, s);
-    }
-    else
-    {
-        if (debug) launch_raster_wave_cfg<2, 33>(p, numTiles, shx, shy, s);
-        else if (bl) launch_raster_wave_cfg<2, 32>(p, numTiles, shx, shy, s);
-        else launch_raster_wave_cfg<2, 0>(p, numTiles, shx, shy, s);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_raster(const RasterParams& p, int numTiles, int cfg, bool debug, hipStream_t s)
+hipError_t launch_raster(const RasterParams& p, int units, int maxParts, int cfg, bool debug, hipStream_t s)
 {
     (void)hipGetLastError();   // drop a stale error from an earlier call
     const bool floatColor = p.colorType == SL_COLOR_R_FLOAT || p.colorType == SL_COLOR_RG_FLOAT ||
                             p.colorType == SL_COLOR_RGB_FLOAT || p.colorType == SL_COLOR_RGBA_FLOAT;
     const int cf = (p.color == nullptr) ? 0 : (floatColor ? 2 : 1);
-    if (!p.extra) return launch_raster_wave(p, cf, numTiles, cfg, debug, s);
-    if (p.vis != nullptr) return hipErrorInvalidValue;   // built for filled triangles only
-    if (p.mrt)
+    const int shx = ilog2i(kTileConfigs[cfg].tileW), shy = ilog2i(kTileConfigs[cfg].tileH);
+    // k_raster_wave's variant; the debug instances and those of several
+    // outputs with lines or points have blending compiled in
+    int aux = (debug ? 1 : 0) | (p.vis != nullptr ? 2 : 0) | (p.extra ? 4 : 0) | (p.mrt ? 8 : 0);
+    if (cf != 0 && (p.blend || debug || (p.mrt && p.extra))) aux |= 32;
+    // visibility is built for RGBA32F colour, filled triangles and single
+    // outputs; several outputs need colour attachment 0
+    switch (cf << 8 | aux)
     {
-        if (cf == 0) return hipErrorInvalidValue;   // outputs need colour attachment 0
-        if (debug && cf == 1) launch_raster_cfg<1, 9>(p, numTiles, cfg, s);
-        else if (debug) launch_raster_cfg<2, 9>(p, numTiles, cfg, s);
-        else if (cf == 1) launch_raster_cfg<1, 8>(p, numTiles, cfg, s);
-        else launch_raster_cfg<2, 8>(p, numTiles, cfg, s);
-    }
-    else if (debug)
-    {
-        if (cf == 0) launch_raster_cfg<0, 1>(p, numTiles, cfg, s);
-        else if (cf == 1) launch_raster_cfg<1, 1>(p, numTiles, cfg, s);
-        else launch_raster_cfg<2, 1>(p, numTiles, cfg, s);
-    }
-    else
-    {
-        if (cf == 0) launch_raster_cfg<0, 0>(p, numTiles, cfg, s);
-        else if (cf == 1) launch_raster_cfg<1, 0>(p, numTiles, cfg, s);
-        else launch_raster_cfg<2, 0>(p, numTiles, cfg, s);
+#define SL_RASTER(CF, AUX) case CF << 8 | AUX: launch_raster_wave_cfg<CF, AUX>(p, units, maxParts, shx, shy, s); break
+        SL_RASTER(0, 0); SL_RASTER(1, 0); SL_RASTER(2, 0); SL_RASTER(1, 32); SL_RASTER(2, 32);
+        SL_RASTER(0, 1); SL_RASTER(1, 33); SL_RASTER(2, 33);
+        SL_RASTER(2, 2); SL_RASTER(2, 34); SL_RASTER(2, 35);
+        SL_RASTER(0, 4); SL_RASTER(1, 4); SL_RASTER(2, 4); SL_RASTER(1, 36); SL_RASTER(2, 36);
+        SL_RASTER(0, 5); SL_RASTER(1, 37); SL_RASTER(2, 37);
+        SL_RASTER(1, 8); SL_RASTER(2, 8); SL_RASTER(1, 40); SL_RASTER(2, 40); SL_RASTER(1, 41); SL_RASTER(2, 41);
+        SL_RASTER(1, 44); SL_RASTER(2, 44); SL_RASTER(1, 45); SL_RASTER(2, 45);
+#undef SL_RASTER
+        default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }

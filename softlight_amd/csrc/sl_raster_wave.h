@@ -32,6 +32,55 @@ __device__ __forceinline__ void wave_lds_fence()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Depth and position along the line of its texel (vx, vy)
+// (SL_LineRasterizer::render_line, SL_LineRasterizer.cpp:27-80).
+__device__ __forceinline__ float line_depth(const SetupRec& R, int vx, int vy, float& interp)
+{
+    const float fx = (float)vx - R.x[0], fy = (float)vy - R.y[0];
+    interp = sqrtf((fx * fx) + (fy * fy)) * R.bx[0];   // length(p - p0) * dist
+    return R.z[0] + interp * (R.z[1] - R.z[0]);        // mix(z0, z1, interp)
+}
+
+// Row y's steps of a line's Bresenham walk, in closed form, into block row r
+// of `mask`; with `wraps` (the block holds column 0) also the walk's texel
+// (W, y - 1), which is texel 0 of row y, before or after them in walk order.
+template <class Run>
+__device__ __forceinline__ void line_row(const LineWalk& w, int W, int y, bool wraps, int r, const Run& run, uint64_t& mask,
+                                         uint64_t& before, uint64_t& after)
+{
+    const int dyAbs = w.dErr >> 1;
+    int xa = 1, xb = 0;
+    if (!w.steep)
+    {
+        const int n = (y - w.Y1) * w.yErr;
+        if (n >= 0 && n <= dyAbs)
+        {
+            xa = w.X1 + ((n == 0) ? 0 : (w.dx * (2 * n - 1)) / w.dErr + 1);
+            xb = w.X1 + ((n == dyAbs) ? w.dx : (w.dx * (2 * n + 1)) / w.dErr);
+        }
+    }
+    else
+    {
+        const int k = y - w.X1;
+        if (k >= 0 && k <= w.dx) xa = xb = w.Y1 + w.yErr * line_minor_steps(w, k);
+    }
+    mask |= run(xa, xb + 1, r);
+    if (wraps && y >= 1)
+    {
+        const int ka = w.steep ? (y - 1) - w.X1 : W - w.X1;
+        if (ka >= 0 && ka <= w.dx)
+        {
+            const int m = w.Y1 + w.yErr * line_minor_steps(w, ka);
+            if (w.steep ? (m == W) : (m == y - 1))
+            {
+                const int k0 = w.steep ? y - w.X1 : -w.X1;
+                const bool first = !(xa <= 0 && 0 <= xb && k0 < ka);
+                (first ? before : after) |= 1ull << (8 * r);
+            }
+        }
+    }
+}
+
 // k_raster_wave: a wave owns an 8x8 block of its tile and walks the tile's
 // record list; a pixel's depth, colour and pending fragment live in its
 // lane's registers for the whole batch.
@@ -72,13 +121,35 @@ __device__ __forceinline__ void wave_lds_fence()
 // combined coefficients within 11 of the same units (block corners included);
 // 2.125 (X / 4 + 13) units are allowed, and non-finite terms decide nothing.
 //
-// AUX: bit 0 debug buffers, bit 1 visibility, bit 3 several fragment outputs
-// (as k_raster), bit 5 some draw of the batch blends.
-template <int CF, int AUX>
-__global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShiftX, int tileShiftY, int wavesShift)
+// Wireframe triangles, lines and points go through the same three stages with
+// masks and depths of their own: a wireframe row's second run can visit a
+// pixel again and a line's texel (W, y - 1) is texel 0 of row y, before or
+// after the row's own, so such a record has up to three masks, queued in the
+// order the walk visits them.
+//
+// Heavy tiles (RasterParams::items, batches with such records only): a
+// workgroup takes a work item, a whole tile or one part of a split tile's
+// record list.  MODE 1 walks a part from +inf (-inf) and leaves the depth it
+// ends with, the part's own result m; a MODE 0 part starts from
+// fold(initial depth, m of the earlier parts) -- exactly the depth the
+// sequential walk has there -- so it counts the fragments that pass exactly
+// and ends with its last passing fragment pending; it leaves those per pixel
+// and raises the pixel's entry in partWin to itself.  A last launch (merge)
+// takes for every pixel the depth after all parts and the pending fragment of
+// the last part that left one.  (The merge used to be done by the part that
+// finished last, which searched up to 1,024 parts' results per pixel: the
+// lines of a frame of 16 spheres, 1280x720, took 1,228 us in the two passes,
+// now 290; the frame 1,363 -> 603.)
+//
+// AUX: bit 0 debug buffers, bit 1 visibility, bit 2 wireframe, line or point
+// records in the batch, bit 3 several fragment outputs, bit 5 some draw of
+// the batch blends.
+template <int CF, int AUX, int MODE>
+__global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShiftX, int tileShiftY, int wavesShift, int merge)
 {
     constexpr bool DBG = (AUX & 1) != 0;
     constexpr bool VIS = (AUX & 2) != 0;
+    constexpr bool EXTRA = (AUX & 4) != 0;
     constexpr bool MRT = (AUX & 8) != 0;
     constexpr bool BLEND = (AUX & 32) != 0;
     __shared__ uint32_t sIdW[4][64];
@@ -94,16 +165,28 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     uint32_t* sMeta = sMetaW[wave];
     float4* sRes = sResW[wave];
 
-    // wave -> block of a tile; tiles in launch order (heaviest first)
+    // wave -> block of a tile; tiles in launch order (heaviest first), or work items
     const int groupShift = tileShiftX + tileShiftY - 6 - wavesShift;    // log2 workgroups per tile
     const int slot = (int)(blockIdx.x >> groupShift);
+    RasterItem item{};
+    bool part = false;
+    if (EXTRA && P.items != nullptr)
+    {
+        if ((uint32_t)slot >= P.itemCount[(MODE == 1 || merge) ? 1 : 0]) return;
+        item = P.items[slot];
+        if (item.parts == 0u || (merge && item.part != 0u)) return;    // a split tile's entry in launch order: its parts do the work
+        part = item.parts > 1u && !merge;
+    }
+    else if (MODE == 1) return;
     const int blk = (int)(((blockIdx.x & ((1u << groupShift) - 1u)) << wavesShift) + (uint32_t)wave);
-    const int tile = (P.tileOrder != nullptr) ? (int)P.tileOrder[slot] : slot;
+    const int tile = (EXTRA && P.items != nullptr) ? (int)item.tile : (P.tileOrder != nullptr) ? (int)P.tileOrder[slot] : slot;
     const int tx = tile % P.tilesX, ty = tile / P.tilesX;
     const int bx0 = (tx << tileShiftX) + ((blk & ((1 << (tileShiftX - 3)) - 1)) << 3);
     const int by0 = (ty << tileShiftY) + ((blk >> (tileShiftX - 3)) << 3);
     if (bx0 >= P.W || by0 >= P.H) return;
-    const uint2 range = P.tileRange[tile];
+    uint2 range;
+    if (EXTRA && P.items != nullptr) range = merge ? make_uint2(0u, 0u) : make_uint2(item.begin, item.end);
+    else range = P.tileRange[tile];
     const int x = bx0 + (lane & 7), y = by0 + (lane >> 3);
     const bool inb = x < P.W && y < P.H;
     const uint64_t gi = (uint64_t)y * P.W + x;
@@ -136,6 +219,39 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     }
     uint32_t pend = kNoPending;                 // pending fragment: its record and barycentric values
     float ps0 = 0.f, ps1 = 0.f, ps2 = 0.f;
+    // a split tile's pixel in the part slots: slot s's entry at s * tilePix + tp
+    const uint64_t tilePix = 1ull << (tileShiftX + tileShiftY);
+    const uint64_t tp = (uint64_t)((y & ((1 << tileShiftY) - 1)) << tileShiftX) + (uint64_t)(x & ((1 << tileShiftX) - 1));
+    if (MODE == 1) depth = (P.splitClass == kSplitMax) ? -INFINITY : INFINITY;
+    if (EXTRA && MODE == 0 && (part || merge) && inb)
+    {
+        // the fold pass left fold(initial, m_0 .. m_j) in part j's slot
+        const uint32_t upTo = merge ? item.parts : item.part;
+        if (P.splitClass != kSplitConst && upTo > 0u) depth = P.partDepth[(uint64_t)(item.slot - item.part + upTo - 1u) * tilePix + tp];
+        if (part && DBG) dbgLast = dbgCount = 0u;       // the merge adds the parts' counts
+        if (merge)
+        {
+            const uint32_t win = P.partWin[(uint64_t)item.split * tilePix + tp];
+            if (win != 0u)
+            {
+                const PartPixel q = P.partRes[(uint64_t)(item.slot + win - 1u) * tilePix + tp];
+                pend = q.rid;
+                ps0 = q.s0;
+                ps1 = q.s1;
+                ps2 = q.s2;
+            }
+            if (DBG)
+            {
+                for (uint32_t j = 0; j < item.parts; ++j)
+                {
+                    const PartPixel q = P.partRes[(uint64_t)(item.slot + j) * tilePix + tp];
+                    if (q.count == 0u) continue;
+                    dbgCount += q.count;
+                    dbgLast = q.seq;
+                }
+            }
+        }
+    }
 
     // shades a fragment of this lane's pixel into its colour
     auto shade_into = [&](uint32_t rid, float s0, float s1, float s2, int blendMode) {
@@ -154,10 +270,11 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     uint32_t tested = 0, shaded = 0;
 
     // this lane's record of the current 64
-    uint64_t mask = 0;
+    uint64_t mask = 0, maskBefore = 0, maskAfter = 0;
     uint32_t id = 0, state = 0;
     float zx = 0.f, zy = 0.f, zlo = 0.f, zwid = 0.f;
     uint64_t todo = 0;
+    uint32_t masks = 0;                         // masks left of the record at hand (EXTRA)
     uint32_t base = range.x;
     bool more = true;
     while (more)
@@ -173,61 +290,132 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                 }
                 const int nb = (int)min(64u, range.y - base);
                 const float top = wave_max_f32(bound);
-                mask = 0;
+                mask = maskBefore = maskAfter = 0;
                 bool rej = false, raise = false;
                 if (lane < nb)
                 {
                     id = P.tileRecs[base + lane];
                     const SetupRec& R = P.recs[id];
-                    const ScanEdges E = scan_edges(R);
                     state = R.state;
+                    const ScanEdges E = scan_edges(R);
                     const int r0 = max(R.minY - by0, 0), r1 = min(min(R.maxY, P.H) - by0, 8);
                     const int xr = min(P.W - bx0, 8);
-                    for (int r = r0; r < r1; ++r)
+                    // columns [from, to) of block row r
+                    auto run = [&](int from, int to, int r) -> uint64_t {
+                        const int a = max(from, bx0) - bx0, b = max(min(to, bx0 + xr), bx0) - bx0;
+                        return a < b ? (uint64_t)((1u << b) - (1u << a)) << (8 * r) : 0ull;
+                    };
+                    const bool line = EXTRA && (state & kStateLine) != 0u, point = EXTRA && (state & kStatePoint) != 0u;
+                    const bool wire = EXTRA && (state & kStateWire) != 0u;
+                    if (!line && !point)
                     {
-                        int32_t xMin, xMax;
-                        scanline_step(E, (float)(by0 + r), xMin, xMax);
-                        const int a = max(xMin, bx0) - bx0, b = max(min(xMax, bx0 + xr), bx0) - bx0;
-                        if ((uint32_t)xMin < (uint32_t)xMax && a < b)
-                            mask |= (uint64_t)((1u << b) - (1u << a)) << (8 * r);
+                        for (int r = r0; r < r1; ++r)
+                        {
+                            int32_t xMin, xMax;
+                            scanline_step(E, (float)(by0 + r), xMin, xMax);
+                            if ((uint32_t)xMin >= (uint32_t)xMax) continue;
+                            if (!wire)
+                            {
+                                mask |= run(xMin, xMax, r);
+                                continue;
+                            }
+                            // the run from the left end over the distance the left
+                            // end moved since the row above, then the run up to the
+                            // right end over the distance it moved; the second can
+                            // start inside the first
+                            int32_t xMin1, xMax1;
+                            scanline_step(E, (float)(by0 + r) - 1.f, xMin1, xMax1);
+                            const int32_t g0 = wire_gap(xMin, xMin1), g1 = wire_gap(xMax, xMax1);
+                            const int64_t firstEnd = (int64_t)xMin + g0;
+                            mask |= run(xMin, (firstEnd < (int64_t)xMax) ? (int)firstEnd : xMax, r);
+                            if (firstEnd < (int64_t)xMax)
+                            {
+                                const int32_t t = (int32_t)((uint32_t)xMax - (uint32_t)g1 - 1u);
+                                maskAfter |= run(max(xMin, t) + 1, xMax, r);
+                            }
+                        }
                     }
-                    if (mask != 0)
+                    else if (point)
                     {
-                        tested += (uint32_t)__popcll(mask);
+                        const int px = (int)R.x[0], py = (int)R.y[0];
+                        if (py >= by0 + r0 && py < by0 + r1) mask = run(px, px + 1, py - by0);
+                    }
+                    else
+                    {
+                        const LineWalk w = line_walk_of(R);
+                        const bool wraps = bx0 == 0 && (R.xbox & 0xFFFFu) == 0u;
+                        for (int r = r0; r < r1; ++r) line_row(w, P.W, by0 + r, wraps, r, run, mask, maskBefore, maskAfter);
+                    }
+                    const uint32_t covers = (uint32_t)(__popcll(mask) + __popcll(maskBefore) + __popcll(maskAfter));
+                    if (covers != 0u)
+                    {
+                        tested += covers;
                         const int dt = (int)(state & 7u);
                         const bool less = dt == SL_DEPTH_TEST_LESS_THAN || dt == SL_DEPTH_TEST_LESS_EQUAL;
                         raise = ((state >> 3) & 1u) != 0u && !less && dt != SL_DEPTH_TEST_EQUAL;
                         const float X = (float)(bx0 + 7), Y = (float)(by0 + 7);
-                        float zc = R.bc3, mag = 0.f;
                         zx = 0.f;
                         zy = 0.f;
-#pragma unroll
-                        for (int i = 0; i < 3; ++i)
+                        if (!line && !point)
                         {
-                            const float zi = R.z[i], bx = R.bx[i], by = R.by[i], bz = R.bz[i];
-                            zx = fmaf(zi, bx, zx);
-                            zy = fmaf(zi, by, zy);
-                            zc = fmaf(zi, bz, zc);
-                            mag = fmaf(fabsf(zi), fmaf(X, fabsf(bx), fmaf(Y, fabsf(by), fabsf(bz))), mag);
+                            float zc = R.bc3, mag = 0.f;
+#pragma unroll
+                            for (int i = 0; i < 3; ++i)
+                            {
+                                const float zi = R.z[i], bx = R.bx[i], by = R.by[i], bz = R.bz[i];
+                                zx = fmaf(zi, bx, zx);
+                                zy = fmaf(zi, by, zy);
+                                zc = fmaf(zi, bz, zc);
+                                mag = fmaf(fabsf(zi), fmaf(X, fabsf(bx), fmaf(Y, fabsf(by), fabsf(bz))), mag);
+                            }
+                            const float margin = fmaf(mag * (5.9604645e-8f * 2.125f), fmaf(0.25f, X, 13.f), 1e-37f);
+                            zlo = zc - margin;
+                            zwid = 2.125f * margin;
                         }
-                        const float margin = fmaf(mag * (5.9604645e-8f * 2.125f), fmaf(0.25f, X, 13.f), 1e-37f);
-                        zlo = zc - margin;
-                        zwid = 2.125f * margin;
+                        else if (covers == 1u)
+                        {
+                            // one texel (a point, a distant line): its depth itself
+                            const uint64_t m = mask | maskBefore | maskAfter;
+                            const int px = __ffsll((unsigned long long)m) - 1;
+                            float interp;
+                            zlo = point ? R.z[0] : line_depth(R, mask != 0 ? bx0 + (px & 7) : P.W, by0 + (px >> 3) - (mask != 0 ? 0 : 1), interp);
+                            zwid = 0.f;
+                            // a line of no length: NaN passes no ordered test
+                            rej = zlo != zlo && dt != SL_DEPTH_TEST_OFF && dt != SL_DEPTH_TEST_NOT_EQUAL;
+                        }
+                        else
+                        {
+                            // depths between the first end's and the one at the
+                            // greatest position a texel of the block can have
+                            const float z0 = R.z[0], dz = R.z[1] - z0;
+                            const float fx = fmaxf(fmaxf(fabsf((float)bx0 - R.x[0]), fabsf(X - R.x[0])), bx0 == 0 ? fabsf((float)P.W - R.x[0]) : 0.f);
+                            const float fy = fmaxf(fabsf((float)(by0 - 1) - R.y[0]), fabsf(Y - R.y[0]));
+                            const float far = sqrtf((fx * fx) + (fy * fy)) * fabsf(R.bx[0]) * 1.000001f;
+                            const float margin = fmaf(1e-6f, fabsf(z0) + far * fabsf(dz), 1e-37f);
+                            zlo = fminf(z0, z0 + far * dz) - margin;
+                            zwid = far * fabsf(dz) + 2.125f * margin;
+                            if (zlo != zlo || z0 + far * dz != z0 + far * dz) zlo = -INFINITY, zwid = INFINITY;
+                        }
                         const float lo = (zlo + fminf(zx * (float)bx0, zx * X)) + fminf(zy * (float)by0, zy * Y);
-                        rej = less && lo > top;
+                        rej = rej || (less && lo > top);
+                        if (MODE == 1) tested = 0;
                     }
                 }
                 base += 64u;
                 // records from the first one that can raise a depth on stay
                 const uint64_t rb = __ballot(raise);
                 const uint64_t before = (rb != 0) ? ((rb & (0ull - rb)) - 1ull) : ~0ull;
-                todo = __ballot(mask != 0) & ~(__ballot(rej) & before);
+                todo = __ballot((mask | maskBefore | maskAfter) != 0) & ~(__ballot(rej) & before);
                 continue;
             }
             const int bi = __ffsll((unsigned long long)todo) - 1;
+            // the record's masks in walk order
+            if (EXTRA && masks == 0u)
+                masks = (uint32_t)__builtin_amdgcn_readlane((maskBefore != 0 ? 1 : 0) | (mask != 0 ? 2 : 0) | (maskAfter != 0 ? 4 : 0), bi);
+            const uint64_t mcur = !EXTRA || (masks & 3u) == 2u ? mask : ((masks & 1u) != 0u ? maskBefore : maskAfter);
             const uint32_t st = (uint32_t)__builtin_amdgcn_readlane((int)state, bi);
-            const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mask >> 32), bi) << 32) |
-                               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mask, bi);
+            const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mcur >> 32), bi) << 32) |
+                               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mcur, bi);
             const int dt = (int)(st & 7u);
             const bool less = dt == SL_DEPTH_TEST_LESS_THAN || dt == SL_DEPTH_TEST_LESS_EQUAL;
             const float zp = fmaf(readlane_f32(zx, bi), (float)x, fmaf(readlane_f32(zy, bi), (float)y, readlane_f32(zlo, bi)));
@@ -241,7 +429,8 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                 {
                     const uint32_t e = (uint32_t)queued + lanes_below(cm);
                     sId[e] = (uint32_t)__builtin_amdgcn_readlane((int)id, bi);
-                    sMeta[e] = (uint32_t)lane | (st << 8);
+                    // (a line's other masks hold its wrapped texels)
+                    sMeta[e] = (uint32_t)lane | (EXTRA && (masks & 3u) != 2u ? 64u : 0u) | (st << 8);
                     mine |= 1ull << e;
                     if (((st >> 3) & 1u) != 0u)
                     {
@@ -253,6 +442,7 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                 }
                 queued += n;
             }
+            if (EXTRA && (masks &= masks - 1u) != 0u) continue;
             todo &= todo - 1ull;
         }
         if (queued == 0) continue;
@@ -265,44 +455,66 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
             const uint32_t px = sMeta[lane] & 63u;
             const int ex = bx0 + (int)(px & 7u);
             const float yf = (float)(by0 + (int)(px >> 3));
-            int32_t xMin, xMax;
-            scanline_step(scan_edges(R), yf, xMin, xMax);
-            // bc(x) = fl(fl(x*dx) + fma(dy, y, c)) at the span's first pixel of
-            // this one's class mod 4, then += 4*dx per group of 4 pixels
-            const int g = (ex - xMin) >> 2;
-            const float fx = (float)(ex - 4 * g);
-            float s0 = (fx * R.bx[0]) + fmaf(R.by[0], yf, R.bz[0]);
-            float s1 = (fx * R.bx[1]) + fmaf(R.by[1], yf, R.bz[1]);
-            float s2 = (fx * R.bx[2]) + fmaf(R.by[2], yf, R.bz[2]);
-            const float d0 = R.bx[0] * 4.f, d1 = R.bx[1] * 4.f, d2 = R.bx[2] * 4.f;
-            if (g <= kStepLimit)
+            const uint32_t kind = EXTRA ? (sMeta[lane] >> 8) & (kStateWire | kStateLine | kStatePoint) : 0u;
+            float z, s0 = 0.f, s1 = 0.f, s2 = 0.f;
+            if (EXTRA && kind == kStatePoint)
             {
-                int k = 0;
-                for (; k + 4 <= g; k += 4)
+                z = R.z[0];
+            }
+            else if (EXTRA && kind == kStateLine)
+            {
+                const bool wrapped = (sMeta[lane] & 64u) != 0u;
+                z = line_depth(R, wrapped ? P.W : ex, by0 + (int)(px >> 3) - (wrapped ? 1 : 0), s0);
+            }
+            else if (EXTRA && kind == kStateWire)
+            {
+                const float fx = (float)ex;
+                s0 = fmaf(R.bx[0], fx, fmaf(R.by[0], yf, R.bz[0]));
+                s1 = fmaf(R.bx[1], fx, fmaf(R.by[1], yf, R.bz[1]));
+                s2 = fmaf(R.bx[2], fx, fmaf(R.by[2], yf, R.bz[2]));
+                z = (((R.z[0] * s0) + (R.z[1] * s1)) + (R.z[2] * s2)) + R.bc3;
+            }
+            else
+            {
+                int32_t xMin, xMax;
+                scanline_step(scan_edges(R), yf, xMin, xMax);
+                // bc(x) = fl(fl(x*dx) + fma(dy, y, c)) at the span's first pixel of
+                // this one's class mod 4, then += 4*dx per group of 4 pixels
+                const int g = (ex - xMin) >> 2;
+                const float fx = (float)(ex - 4 * g);
+                s0 = (fx * R.bx[0]) + fmaf(R.by[0], yf, R.bz[0]);
+                s1 = (fx * R.bx[1]) + fmaf(R.by[1], yf, R.bz[1]);
+                s2 = (fx * R.bx[2]) + fmaf(R.by[2], yf, R.bz[2]);
+                const float d0 = R.bx[0] * 4.f, d1 = R.bx[1] * 4.f, d2 = R.bx[2] * 4.f;
+                if (g <= kStepLimit)
                 {
+                    int k = 0;
+                    for (; k + 4 <= g; k += 4)
+                    {
 #pragma unroll
-                    for (int u = 0; u < 4; ++u)
+                        for (int u = 0; u < 4; ++u)
+                        {
+                            s0 = s0 + d0;
+                            s1 = s1 + d1;
+                            s2 = s2 + d2;
+                        }
+                    }
+                    for (; k < g; ++k)
                     {
                         s0 = s0 + d0;
                         s1 = s1 + d1;
                         s2 = s2 + d2;
                     }
                 }
-                for (; k < g; ++k)
+                else
                 {
-                    s0 = s0 + d0;
-                    s1 = s1 + d1;
-                    s2 = s2 + d2;
+                    const float3 a = recur_advance3(make_float3(s0, s1, s2), make_float3(d0, d1, d2), g);
+                    s0 = a.x;
+                    s1 = a.y;
+                    s2 = a.z;
                 }
+                z = (((R.z[0] * s0) + (R.z[1] * s1)) + (R.z[2] * s2)) + R.bc3;
             }
-            else
-            {
-                const float3 a = recur_advance3(make_float3(s0, s1, s2), make_float3(d0, d1, d2), g);
-                s0 = a.x;
-                s1 = a.y;
-                s2 = a.z;
-            }
-            const float z = (((R.z[0] * s0) + (R.z[1] * s1)) + (R.z[2] * s2)) + R.bc3;
             sRes[lane] = make_float4(z, s0, s1, s2);
         }
         wave_lds_fence();
@@ -314,6 +526,11 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
             const float4 f = sRes[e];
             const uint32_t rid = sId[e], st = sMeta[e] >> 8;
             if (!depth_test((int)(st & 7u), f.x, depth)) continue;
+            if (MODE == 1)
+            {
+                depth = f.x;
+                continue;
+            }
             const int blendMode = (int)((st >> 4) & 7u);
             const bool hasOut = ((st >> 7) & 1u) != 0u;
             // an unblended fragment with outputs, and any whose visibility
@@ -352,18 +569,35 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
         wave_lds_fence();
     }
 
-    if (pend != kNoPending) shade_into(pend, ps0, ps1, ps2, SL_BLEND_OFF);
-    if (inb)
+    if (MODE == 1)
     {
-        store_depth(P, gi, depth);
-        if (CF == 1) store_color8(P, gi, col8);
-        if (CF == 2) store_colorF(P, gi, colF);
-        if (DBG)
+        if (inb) P.partDepth[(uint64_t)item.slot * tilePix + tp] = depth;
+        return;
+    }
+    if (EXTRA && part)
+    {
+        if (inb)
         {
-            P.dbgLast[gi] = dbgLast;
-            P.dbgCount[gi] = dbgCount;
+            // the part's last passing fragment (and, with the debug buffers, its counts)
+            if (pend != kNoPending || DBG) P.partRes[(uint64_t)item.slot * tilePix + tp] = PartPixel{pend, ps0, ps1, ps2, dbgCount, dbgLast};
+            if (pend != kNoPending) atomicMax(&P.partWin[(uint64_t)item.split * tilePix + tp], item.part + 1u);
         }
-        if (VIS) P.vis[gi] = vis;
+    }
+    else
+    {
+        if (pend != kNoPending) shade_into(pend, ps0, ps1, ps2, SL_BLEND_OFF);
+        if (inb)
+        {
+            store_depth(P, gi, depth);
+            if (CF == 1) store_color8(P, gi, col8);
+            if (CF == 2) store_colorF(P, gi, colF);
+            if (DBG)
+            {
+                P.dbgLast[gi] = dbgLast;
+                P.dbgCount[gi] = dbgCount;
+            }
+            if (VIS) P.vis[gi] = vis;
+        }
     }
 
     // the block's counts (a lane's stay below 64 per record of its 64th of the list)
@@ -384,13 +618,61 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
 
 }  // namespace
 
-template <int CF, int AUX>
-void launch_raster_wave_cfg(const RasterParams& p, int numTiles, int shx, int shy, hipStream_t s)
+// Between the passes over split tiles' parts: for every pixel of a split tile
+// part j's slot gets fold(initial depth, m_0 .. m_j), the depth the sequential
+// walk has after part j, and the pixel's entry in partWin is cleared.  One
+// workgroup per split tile (the work item of its part 0).
+static __global__ __launch_bounds__(256) void k_split_fold(RasterParams P, int tileShiftX, int tileShiftY)
+{
+    if (P.ctrl != nullptr && P.ctrl->overflow != 0u) return;
+    if (blockIdx.x >= P.itemCount[1]) return;
+    const RasterItem item = P.items[blockIdx.x];
+    if (item.part != 0u) return;
+    const int tilePix = 1 << (tileShiftX + tileShiftY);
+    const int tx = (int)item.tile % P.tilesX, ty = (int)item.tile / P.tilesX;
+    for (int k = threadIdx.x; k < tilePix; k += 256)
+    {
+        P.partWin[(uint64_t)item.split * tilePix + k] = 0u;
+        if (P.splitClass == kSplitConst) continue;
+        const int gx = (tx << tileShiftX) + (k & ((1 << tileShiftX) - 1)), gy = (ty << tileShiftY) + (k >> tileShiftX);
+        if (gx >= P.W || gy >= P.H) continue;
+        float d = P.clearDepth ? P.clearDepthValue : load_depth(P, (uint64_t)gy * P.W + gx);
+        float* m = P.partDepth + (uint64_t)item.slot * tilePix + k;
+        for (uint32_t j = 0; j < item.parts; ++j)
+        {
+            const float mj = m[(uint64_t)j * tilePix];
+            if (depth_test(P.splitDtest, mj, d)) d = mj;
+            m[(uint64_t)j * tilePix] = d;
+        }
+    }
+}
+
+template <int CF, int AUX, int MODE>
+static void launch_wave(const RasterParams& p, int units, int shx, int shy, int merge, hipStream_t s)
 {
     const int blocksShift = shx + shy - 6, wavesShift = blocksShift < 2 ? blocksShift : 2;
-    const auto kernel = k_raster_wave<CF, AUX>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)numTiles << (blocksShift - wavesShift)), dim3(64u << wavesShift),
-                       occupancy_lds(kernel, p.wgPerCU), s, p, shx, shy, wavesShift);
+    const auto kernel = k_raster_wave<CF, AUX, MODE>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)units << (blocksShift - wavesShift)), dim3(64u << wavesShift),
+                       occupancy_lds(kernel, p.wgPerCU), s, p, shx, shy, wavesShift, merge);
+}
+
+// units: tiles, or (items) the most work items there can be; maxParts: the
+// most parts of split tiles among them.
+template <int CF, int AUX>
+void launch_raster_wave_cfg(const RasterParams& p, int units, int maxParts, int shx, int shy, hipStream_t s)
+{
+    if constexpr ((AUX & 4) != 0)
+    {
+        if (p.items != nullptr)
+        {
+            if (p.splitClass != kSplitConst) launch_wave<0, 4, 1>(p, maxParts, shx, shy, 0, s);
+            hipLaunchKernelGGL(k_split_fold, dim3((unsigned)maxParts), dim3(256), 0, s, p, shx, shy);
+            launch_wave<CF, AUX, 0>(p, units, shx, shy, 0, s);
+            launch_wave<CF, AUX, 0>(p, maxParts, shx, shy, 1, s);
+            return;
+        }
+    }
+    launch_wave<CF, AUX, 0>(p, units, shx, shy, 0, s);
 }
 
 }  // namespace slg

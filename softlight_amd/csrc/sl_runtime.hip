@@ -92,9 +92,9 @@ struct FrameRes
     DevBuf draws, uni, recs, vars, keys, vals, sorted, clip, status, ranges, ctrl, binCounts, binTotals, order;
     uint32_t recCap = 0, pairCap = 0, clipCap = 0;
     // heavy-tile split: work items, their counts, per part slot the first
-    // pass's depths and the part results, per split tile a finished-parts
-    // counter (absent: no split)
-    DevBuf items, itemCount, partDepth, partRes, partDone;
+    // pass's depths and the part results, per split tile and pixel the last
+    // part with a pending fragment (absent: no split)
+    DevBuf items, itemCount, partDepth, partRes, partWin;
     uint32_t maxParts = 0;
     DevBuf positions, vtxDraws;   // the vertex pass's output and work table
 };
@@ -522,7 +522,8 @@ int ensure_frame(sl_context* c, FrameRes& R, const Plan& p, const Batch& B)
         if ((rc = ensure(c, R.itemCount, 2 * sizeof(uint32_t))) != SL_OK) return rc;
         if ((rc = ensure(c, R.partDepth, sizeof(float) * pix * parts)) != SL_OK) return rc;
         if ((rc = ensure(c, R.partRes, sizeof(PartPixel) * pix * parts)) != SL_OK) return rc;
-        if ((rc = ensure(c, R.partDone, sizeof(uint32_t) * parts)) != SL_OK) return rc;
+        // a split tile has more than kSplitAboveParts parts
+        if ((rc = ensure(c, R.partWin, sizeof(uint32_t) * pix * (parts / (kSplitAboveParts + 1) + 1))) != SL_OK) return rc;
         R.maxParts = parts;
     }
     return SL_OK;
@@ -617,7 +618,7 @@ RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool have
     rp.itemCount = nullptr;
     rp.partDepth = nullptr;
     rp.partRes = nullptr;
-    rp.partDone = nullptr;
+    rp.partWin = nullptr;
     rp.splitClass = kSplitNone;
     rp.splitDtest = 0;
     if (haveEntries && R.items.p != nullptr && R.maxParts > 0)
@@ -629,7 +630,7 @@ RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool have
             rp.itemCount = reinterpret_cast<const uint32_t*>(R.itemCount.p);
             rp.partDepth = reinterpret_cast<float*>(R.partDepth.p);
             rp.partRes = reinterpret_cast<PartPixel*>(R.partRes.p);
-            rp.partDone = reinterpret_cast<uint32_t*>(R.partDone.p);
+            rp.partWin = reinterpret_cast<uint32_t*>(R.partWin.p);
             rp.splitClass = cls;
             rp.splitDtest = B.draws[0].dtest;
         }
@@ -695,21 +696,21 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
                                               reinterpret_cast<uint32_t*>(R.binCounts.p), reinterpret_cast<uint32_t*>(R.binTotals.p),
                                               reinterpret_cast<uint2*>(R.ranges.p), reinterpret_cast<uint32_t*>(R.sorted.p),
                                               reinterpret_cast<uint32_t*>(R.order.p), p.numTiles, s,
-                                              const_cast<RasterItem*>(rp.items), const_cast<uint32_t*>(rp.itemCount), rp.partDone,
+                                              const_cast<RasterItem*>(rp.items), const_cast<uint32_t*>(rp.itemCount),
                                               partRecs, kSplitAboveParts * partRecs, R.maxParts), "binning")) != SL_OK) return rc;
         }
     }
     if (evBin1) (void)hipEventRecord(evBin1, s);
     if (rp.items != nullptr)
     {
-        // heavy tiles: the first pass over split tiles' parts, then one
-        // workgroup per work item (capacity-sized grids: the counts stay on
-        // the device)
-        if (rp.splitClass != kSplitConst && (rc = check(c, launch_raster_depth(rp, (int)R.maxParts, p.cfg, s), "k_raster depth pass")) != SL_OK)
-            return rc;
-        return check(c, launch_raster(rp, p.numTiles + (int)R.maxParts, p.cfg, p.debug, s), "k_raster");
+        // heavy tiles: the grids cover the most work items the entries can
+        // make (a split tile of n records, n > kSplitAboveParts * partRecs, has
+        // at most n / partRecs + 1 parts); the counts stay on the device
+        const uint64_t partRecs = std::max<uint32_t>(c->splitRecs, 1u);
+        const int parts = (int)std::min<uint64_t>(R.maxParts, (uint64_t)entries * (kSplitAboveParts + 1) / (kSplitAboveParts * partRecs) + 1);
+        return check(c, launch_raster(rp, p.numTiles + parts, parts, p.cfg, p.debug, s), "raster");
     }
-    return check(c, launch_raster(rp, p.numTiles, p.cfg, p.debug, s), "k_raster");
+    return check(c, launch_raster(rp, p.numTiles, 0, p.cfg, p.debug, s), "raster");
 }
 
 int upload_batch(sl_context* c, FrameRes& R, const Batch& B, hipStream_t s)
@@ -1016,7 +1017,7 @@ void graph_release(sl_context* c)
     G.graph = nullptr;
     for (DevBuf* b : {&G.res.draws, &G.res.uni, &G.res.recs, &G.res.vars, &G.res.keys, &G.res.vals, &G.res.sorted,
                       &G.res.clip, &G.res.status, &G.res.ranges, &G.res.ctrl, &G.res.binCounts, &G.res.binTotals, &G.res.order,
-                      &G.res.items, &G.res.itemCount, &G.res.partDepth, &G.res.partRes, &G.res.partDone,
+                      &G.res.items, &G.res.itemCount, &G.res.partDepth, &G.res.partRes, &G.res.partWin,
                       &G.res.positions, &G.res.vtxDraws}) release(*b);
     G.res = FrameRes{};
     if (G.hCtrl) (void)hipHostFree(G.hCtrl);
@@ -1440,7 +1441,7 @@ void sl_context_destroy(sl_context* c)
     graph_release(c);
     for (DevBuf* b : {&c->res.draws, &c->res.uni, &c->res.recs, &c->res.vars, &c->res.keys, &c->res.vals, &c->res.sorted,
                       &c->res.clip, &c->res.status, &c->res.ranges, &c->res.ctrl, &c->res.binCounts, &c->res.binTotals, &c->res.order,
-                      &c->res.items, &c->res.itemCount, &c->res.partDepth, &c->res.partRes, &c->res.partDone,
+                      &c->res.items, &c->res.itemCount, &c->res.partDepth, &c->res.partRes, &c->res.partWin,
                       &c->res.positions, &c->res.vtxDraws}) release(*b);
     for (auto& e : c->ev) if (e) (void)hipEventDestroy(e);
     for (auto& f : c->fbos)

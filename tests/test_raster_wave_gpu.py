@@ -69,3 +69,21 @@ def test_depth_functions_in_one_batch(gpu_lib, oracle_lib, depth_type, blend):
         return s
     g, o = render_both(gpu_lib, oracle_lib, build)
     assert_parity(g, o)
+
+
+@pytest.mark.parametrize("mode", [A.RENDER_MODE_TRI_WIRE, A.RENDER_MODE_LINES, A.RENDER_MODE_POINTS])
+@pytest.mark.parametrize("size", [(1, 1), (7, 9), (8, 8), (33, 17), (70, 45)])
+@pytest.mark.parametrize("blend,depth_type", [(A.SL_BLEND_OFF, A.SL_COLOR_R_FLOAT), (A.SL_BLEND_ALPHA, A.SL_COLOR_R_HALF)])
+def test_render_modes_target_sizes(gpu_lib, oracle_lib, mode, size, blend, depth_type):
+    """Wireframe, lines (some of no length) and points on targets around a
+    block's size; the opaque batches with heavy tiles split into parts of 3."""
+    def build(ctx):
+        ctx.set_raster_split(3)
+        rec = scenes.random_triangle_vertices(41, 80).copy()
+        rec[6:12] = rec[0:6]                                # repeated primitives: equal depths
+        rec[13] = rec[12]                                   # a line of no length
+        rec[60:90, 0:8] = rec[60, 0:8]                      # a pile on one texel
+        return scenes.build_from_vertex_records(ctx, rec, size[0], size[1], True, mode=mode, depth_type=depth_type,
+                                                shader_kw=dict(blend=blend))
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
