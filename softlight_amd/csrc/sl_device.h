@@ -296,6 +296,15 @@ struct ClipJob
     uint32_t npair;            // pairs reserved by k_setup
 };
 
+// The bin entries of a record that covers many tiles, written by a whole wave.
+struct PairJob
+{
+    uint32_t rec;
+    uint32_t pairOff;          // its first entry
+    uint16_t tx0, ty0, w, h;   // its tiles
+};
+static_assert(sizeof(PairJob) == 16, "PairJob layout");
+
 // Setup runs as a counting pass, a chunk scan and an emitting pass.  Per
 // chunk of kSetupBlock triangles the counting pass leaves this summary (and
 // one staging word per surviving triangle); the chunk scan fills in the
@@ -331,6 +340,8 @@ struct FrameCtrl
     // clears them, so a replayed graph frame that overflowed is still
     // reported after later replays succeed
     uint32_t sticky;
+    uint32_t pairJobs;         // records whose bin entries the clip kernel's waves write (PairJob)
+    uint32_t pad;
     // Fragment counters, spread over kCounterSlots cache lines (a workgroup
     // adds to slot blockIdx % kCounterSlots): tens of thousands of atomics on
     // one address serialise, on 64 lines they do not.  Readers sum the slots.
@@ -379,6 +390,7 @@ struct SetupParams
     uint32_t pairCap;
     ClipJob* clipJobs;
     uint32_t clipCap;
+    PairJob* pairJobs;            // in the sorted list's storage (idle until the scatter): a job has more than kLanePairs entries
     ChunkInfo* chunkInfo;         // per chunk
     unsigned long long* stage;    // per chunk, kSetupBlock staging words
     unsigned long long* blockAgg; // packed counts per kScanBlock chunks (summed by atomics)

@@ -243,70 +243,58 @@ __device__ __forceinline__ void write_record(const SetupParams& P, uint32_t recI
 
 // The (tile, record) entries of a wave's records, entry j of a record at
 // pairOff + j in row-major order over its tile rectangle (as write_record
-// writes them).  When some record of the wave covers more than kLanePairs
-// tiles and more than kShareRatio times the wave's mean, the wave writes all
-// of its records' entries together, 64 a step:
-// entry k of the wave's concatenated lists goes to the lane k % 64, which
-// finds its record by a binary search over the lanes' inclusive counts.
+// writes them).  A lane writes its own record's entries up to kLanePairs;
+// a larger record becomes a job, whose entries a whole wave of the clip
+// kernel's launch writes (write_pair_jobs).  A lane's own loop holds its wave
+// for as long as its largest record, and a batch of few large triangles has
+// few waves: 4,096 overlapping triangles at 640x480 (708k entries, 16
+// workgroups) took 66 us in the emitting pass, now 13 and 3 more here; 1,200
+// at 801x603 89, now 12.  Sharing a wave's records 64 entries a step with a
+// search per entry had only paid where one record dwarfed its wave.
 // Called by every lane of the wave; `has` marks the lanes with a record.
-constexpr uint32_t kLanePairs = 8, kShareRatio = 6;
+constexpr uint32_t kLanePairs = 16;
+static_assert(sizeof(PairJob) <= kLanePairs * sizeof(uint32_t), "the jobs fit the sorted list's storage");
 
 __device__ __forceinline__ void write_pairs_wave(const SetupParams& P, bool has, uint32_t recId, uint32_t pairOff,
                                                  const TileRect& tr)
 {
-    const int lane = threadIdx.x & 63;
     const int wi = tr.tx1 - tr.tx0 + 1, hi = tr.ty1 - tr.ty0 + 1;
     const bool any = has && wi > 0 && hi > 0;
-    const uint32_t w = any ? (uint32_t)wi : 1u;
-    const uint32_t n = any ? (uint32_t)wi * (uint32_t)hi : 0u;
-    uint32_t mx = n, inc = n;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1)
+    const bool job = any && (uint32_t)(wi * hi) > kLanePairs;
+    const unsigned long long jobs = __ballot(job);
+    if (jobs != 0ull)
     {
-        const uint32_t v = (uint32_t)__shfl_up((int)inc, o, 64);
-        if (lane >= o) inc += v;
-    }
-    const uint32_t total = (uint32_t)__shfl((int)inc, 63, 64);
-    // a lane's own loop costs its count; the shared loop costs the wave's
-    // total / 64 steps of several times the work (the search and the
-    // shuffles): share only when one lane's list dominates the wave
-    if (mx <= kLanePairs || (uint64_t)mx * 64u <= (uint64_t)kShareRatio * total)
-    {
-        if (!any) return;
-        uint32_t o = pairOff;
-        for (int ty = tr.ty0; ty <= tr.ty1; ++ty)
-            for (int tx = tr.tx0; tx <= tr.tx1; ++tx, ++o)
-            {
-                P.pairKeys[o] = (uint32_t)(ty * P.tilesX + tx);
-                P.pairVals[o] = recId;
-            }
-        return;
-    }
-    const int tx0 = any ? tr.tx0 : 0, ty0 = any ? tr.ty0 : 0;
-    for (uint32_t base = 0; base < total; base += 64)
-    {
-        const uint32_t k = base + (uint32_t)lane;
-        // the first lane whose inclusive count exceeds k
-        int L = 0;
-#pragma unroll
-        for (int step = 32; step > 0; step >>= 1)
+        uint32_t at = 0;
+        if ((threadIdx.x & 63) == 0) at = atomicAdd(&P.ctrl->pairJobs, (uint32_t)__popcll(jobs));
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+        if (job)
         {
-            const uint32_t v = (uint32_t)__shfl((int)inc, L + step - 1, 64);
-            if (v <= k) L += step;
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(jobs >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)jobs, 0u));
+            P.pairJobs[at + below] = PairJob{recId, pairOff, (uint16_t)tr.tx0, (uint16_t)tr.ty0, (uint16_t)wi, (uint16_t)hi};
         }
-        const uint32_t incL = (uint32_t)__shfl((int)inc, L, 64);
-        const uint32_t nL = (uint32_t)__shfl((int)n, L, 64);
-        const uint32_t wL = (uint32_t)__shfl((int)w, L, 64);
-        const int tx0L = __shfl(tx0, L, 64), ty0L = __shfl(ty0, L, 64);
-        const uint32_t offL = (uint32_t)__shfl((int)pairOff, L, 64);
-        const uint32_t recL = (uint32_t)__shfl((int)recId, L, 64);
-        if (k < total)
+    }
+    if (!any || job) return;
+    uint32_t o = pairOff;
+    for (int ty = tr.ty0; ty <= tr.ty1; ++ty)
+        for (int tx = tr.tx0; tx <= tr.tx1; ++tx, ++o)
         {
-            const uint32_t j = k - (incL - nL);
-            P.pairKeys[offL + j] = (uint32_t)((ty0L + (int)(j / wL)) * P.tilesX + tx0L + (int)(j % wL));
-            P.pairVals[offL + j] = recL;
+            P.pairKeys[o] = (uint32_t)(ty * P.tilesX + tx);
+            P.pairVals[o] = recId;
+        }
+}
+
+// The jobs' entries, one job per wave at a time.
+__device__ __forceinline__ void write_pair_jobs(const SetupParams& P, uint32_t wave, uint32_t waves)
+{
+    const uint32_t n = P.ctrl->pairJobs;
+    for (uint32_t j = wave; j < n; j += waves)
+    {
+        const PairJob J = P.pairJobs[j];
+        const uint32_t w = J.w, total = w * J.h;
+        for (uint32_t k = threadIdx.x & 63; k < total; k += 64)
+        {
+            P.pairKeys[J.pairOff + k] = (uint32_t)((J.ty0 + k / w) * (uint32_t)P.tilesX + J.tx0 + k % w);
+            P.pairVals[J.pairOff + k] = J.rec;
         }
     }
 }
@@ -1444,6 +1432,7 @@ __global__ __launch_bounds__(kClipBlock) void k_clip(SetupParams P)
     const unsigned long long gmask = 0xFFFFull << (gi * kClipGroup);
     const unsigned long long below = gmask & ((1ull << lane) - 1ull);
     const unsigned long long above = gmask & ~below & ~(1ull << lane);
+    write_pair_jobs(P, blockIdx.x, gridDim.x);
     const uint32_t njobs = min(P.ctrl->clipJobs, P.clipCap);
     // the loop bound is uniform over the workgroup: every lane reaches the barriers
     for (uint32_t base = blockIdx.x * kClipGroups; base < njobs; base += gridDim.x * kClipGroups)
@@ -2025,11 +2014,11 @@ hipError_t launch_emit(const SetupParams& p, bool tris, bool prims, hipStream_t 
     return hipGetLastError();
 }
 
-hipError_t launch_clip(const SetupParams& p, uint32_t jobs, hipStream_t s)
+hipError_t launch_clip(const SetupParams& p, hipStream_t s)
 {
     (void)hipGetLastError();   // drop a stale error from an earlier call
-    if (jobs == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_clip, dim3(grid_for(jobs, kClipGroups, 1024)), dim3(kClipBlock), 0, s, p);
+    // (the counts of clip jobs and of large records' entries stay on the device)
+    hipLaunchKernelGGL(k_clip, dim3(1024), dim3(kClipBlock), 0, s, p);
     return hipGetLastError();
 }
 

@@ -548,6 +548,7 @@ SetupParams setup_params(const Plan& p, const Batch& B, FrameRes& R)
     sp.pairCap = R.pairCap;
     sp.clipJobs = reinterpret_cast<ClipJob*>(R.clip.p);
     sp.clipCap = R.clipCap;
+    sp.pairJobs = reinterpret_cast<PairJob*>(R.sorted.p);
     sp.chunkInfo = reinterpret_cast<ChunkInfo*>(R.status.p);
     sp.stage = reinterpret_cast<unsigned long long*>(sp.chunkInfo + p.chunks);
     sp.blockAgg = sp.stage + (size_t)kSetupBlock * p.chunks;
@@ -664,12 +665,12 @@ int enqueue_front(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, hip
         tris = tris || !pl;
     }
     if ((rc = check(c, launch_emit(sp, tris, prims, s), "k_emit")) != SL_OK) return rc;
-    // the straddling triangles, whose jobs the counting pass reserved (a
-    // grid for the job capacity: the count stays on the device)
+    // the straddling triangles, whose jobs the counting pass reserved, and the
+    // bin entries of large records (the counts stay on the device)
     if (tris)
     {
         if (evClip0 && (rc = check(c, hipEventRecord(evClip0, s), "event")) != SL_OK) return rc;
-        if ((rc = check(c, launch_clip(sp, R.clipCap, s), "k_clip")) != SL_OK) return rc;
+        if ((rc = check(c, launch_clip(sp, s), "k_clip")) != SL_OK) return rc;
         if (evClip1 && (rc = check(c, hipEventRecord(evClip1, s), "event")) != SL_OK) return rc;
     }
     return SL_OK;

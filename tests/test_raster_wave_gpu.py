@@ -87,3 +87,22 @@ def test_render_modes_target_sizes(gpu_lib, oracle_lib, mode, size, blend, depth
                                                 shader_kw=dict(blend=blend))
     g, o = render_both(gpu_lib, oracle_lib, build)
     assert_parity(g, o)
+
+
+@pytest.mark.parametrize("tiles", [(4, 4), (17, 1), (1, 17), (20, 7)])
+def test_bin_entries_of_large_records(gpu_lib, oracle_lib, tiles):
+    """Triangles of up to 16 tiles (whose entries the emitting lane writes),
+    just above (written by a wave) and of many tiles, among small ones, with
+    parts of them clipped; 32x16 tiles."""
+    def build(ctx):
+        W, H = 32 * 24, 16 * 20
+        rec = scenes.random_triangle_vertices(51, 700).copy()
+        xyz = rec[:, 0:12].copy().view(np.float32).reshape(-1, 3, 3)
+        k = np.arange(xyz.shape[0])
+        sx, sy = 2.0 * 32 * tiles[0] / W, 2.0 * 16 * tiles[1] / H
+        size = np.where((k % 3 == 0)[:, None, None], np.float32([sx, sy, 1.0]), np.float32([0.02, 0.03, 1.0]))
+        xyz[:, 1:] = xyz[:, :1] + (xyz[:, 1:] * size).astype(np.float32)
+        rec[:, 0:12] = xyz.astype(np.float32).reshape(-1, 3).view(np.uint8).reshape(-1, 12)
+        return scenes.build_from_vertex_records(ctx, rec, W, H, True)
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
