@@ -6,11 +6,11 @@
 namespace slg {
 
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
-hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, uint64_t n, hipStream_t s);
-// Clears the control block before a frame, keeping (and adding the last
-// frame's overflow / error flags to) FrameCtrl::sticky.
 hipError_t launch_vertex(const SetupParams& p, hipStream_t s);
-hipError_t launch_ctrl_reset(FrameCtrl* ctrl, hipStream_t s);
+// Clears the control block before a frame, keeping (and adding the last
+// frame's overflow / error flags to) FrameCtrl::sticky, and na words of a and
+// nb of b.
+hipError_t launch_frame_reset(FrameCtrl* ctrl, uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb, hipStream_t s);
 hipError_t launch_setup(const SetupParams& p, uint64_t chunks, hipStream_t s);
 hipError_t launch_chunk_scan(const SetupParams& p, hipStream_t s);
 // tris / prims: the batch holds triangle draws / point or line draws.
@@ -20,7 +20,7 @@ hipError_t launch_clip(const SetupParams& p, hipStream_t s);
 // Binning splits the entries into at most kMaxBinBlocks blocks of `per`
 // entries (a multiple of 64, at least kMinBinBlock).
 constexpr uint32_t kMaxBinBlocks = 512;
-constexpr uint32_t kMinBinBlock = 1024;
+constexpr uint32_t kMinBinBlock = 256;   // (1,024: a frame of 1,000 .. 3,000 entries spent 13 us in a few waves of the scatter, now 5)
 struct BinPlan { uint32_t blocks; uint32_t per; };
 BinPlan bin_plan(uint32_t entries);
 // With items non-null the tile scan also writes the raster's work items of

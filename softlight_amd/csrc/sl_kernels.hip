@@ -45,15 +45,33 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, uint64_t n)
     for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = v;
 }
 
-__global__ void k_fill_u64(unsigned long long* __restrict__ p, unsigned long long v, uint64_t n)
+__device__ __forceinline__ bool lane_is_first()
 {
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = v;
+    const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    return lane == __builtin_amdgcn_readfirstlane(lane);
 }
 
-// Per-frame reset of the control block: every word is cleared except
-// `sticky`, which gathers the previous frame's overflow and error flags.
-__global__ void __launch_bounds__(256) k_ctrl_reset(FrameCtrl* __restrict__ ctrl)
+// Sets a flag of the control block, one store a wave: an exchange per lane
+// serialised a million records that had outgrown their buffer into 7 ms.
+__device__ __forceinline__ void raise_flag(uint32_t* flag)
 {
+    if (lane_is_first()) __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Per-frame reset, one launch: the control block by workgroup 0 -- every word
+// is cleared except `sticky`, which gathers the previous frame's overflow and
+// error flags -- and na words of a and nb of b (the tile ranges, setup's block
+// sums) by the others.
+__global__ void __launch_bounds__(256) k_frame_reset(FrameCtrl* __restrict__ ctrl, uint32_t* __restrict__ a, uint32_t na,
+                                                     uint32_t* __restrict__ b, uint32_t nb)
+{
+    if (blockIdx.x > 0)
+    {
+        const uint32_t step = (gridDim.x - 1) * blockDim.x;
+        for (uint32_t i = (blockIdx.x - 1) * blockDim.x + threadIdx.x; i < na; i += step) a[i] = 0u;
+        for (uint32_t i = (blockIdx.x - 1) * blockDim.x + threadIdx.x; i < nb; i += step) b[i] = 0u;
+        return;
+    }
     __shared__ uint32_t prev;
     if (threadIdx.x == 0) prev = ctrl->overflow | (ctrl->error << 1);
     __syncthreads();
@@ -1156,7 +1174,7 @@ __global__ __launch_bounds__(kSetupBlock, 7) void k_setup(SetupParams P)
                 }
                 else
                 {
-                    atomicExch(&P.ctrl->overflow, 1u);
+                    raise_flag(&P.ctrl->overflow);
                 }
             }
         }
@@ -1193,11 +1211,17 @@ __device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long v
     return s;
 }
 
+// Batches of at most this many chunks have their survivor map written by the
+// scan (in one workgroup of 16 waves; at 14 .. 32 workgroups' worth of chunks
+// that cost 12 .. 28 us against the map kernel's 5).
+constexpr uint32_t kScanMapChunks = 64;
+
 __global__ __launch_bounds__(kScanBlock) void k_chunk_scan(SetupParams P)
 {
     __shared__ unsigned long long sRed[kScanBlock / 64];
     __shared__ unsigned long long sA[kScanBlock / 64];
     __shared__ uint32_t sS[kScanBlock / 64];
+    __shared__ uint32_t sMapPre[kScanMapChunks], sMapNum[kScanMapChunks];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const uint32_t b = blockIdx.x;
     const uint32_t c = b * kScanBlock + t;
@@ -1244,6 +1268,19 @@ __global__ __launch_bounds__(kScanBlock) void k_chunk_scan(SetupParams P)
         ChunkInfo& I = P.chunkInfo[c];
         I.pre = ea;
         I.survPre = es;
+    }
+    if (gridDim.x == 1 && P.numChunks <= kScanMapChunks)
+    {
+        // few chunks: the survivors' chunks here, without a launch of k_surv_map
+        // (a wave per chunk; 3 us of a small frame)
+        if (c < P.numChunks)
+        {
+            sMapPre[c] = es;
+            sMapNum[c] = sv;
+        }
+        __syncthreads();
+        for (uint32_t k = (uint32_t)wave; k < P.numChunks; k += kScanBlock / 64)
+            for (uint32_t i = (uint32_t)lane; i < sMapNum[k]; i += 64) P.survChunk[sMapPre[k] + i] = k;
     }
     if (t == 0)
     {
@@ -1305,7 +1342,7 @@ __global__ __launch_bounds__(kEmitBlock, 4) void k_emit(SetupParams P)
         bool bad = false;
         if (chunk >= P.numChunks)
         {
-            atomicExch(&P.ctrl->error, 1u);
+            raise_flag(&P.ctrl->error);
             bad = true;        // the lane goes on without a triangle, with the rest of its wave
         }
         TriIn T;
@@ -1326,7 +1363,7 @@ __global__ __launch_bounds__(kEmitBlock, 4) void k_emit(SetupParams P)
             const ChunkInfo& I = P.chunkInfo[chunk];
             const uint32_t r = s - I.survPre;
             act2 = r < I.surv;
-            if (!act2) atomicExch(&P.ctrl->error, 1u);
+            if (!act2) raise_flag(&P.ctrl->error);
         }
         if (act2)
         {
@@ -1372,14 +1409,14 @@ __global__ __launch_bounds__(kEmitBlock, 4) void k_emit(SetupParams P)
         bool ok = act2 && !C.needClip;
         if (ok && C.nrec == 0)
         {
-            atomicExch(&P.ctrl->error, 1u);
+            raise_flag(&P.ctrl->error);
             ok = false;
         }
         const uint32_t recOff = (uint32_t)(off & ((1ull << kRecBits) - 1));
         const uint64_t pairOff = off >> kRecBits;
         if (ok && ((uint64_t)recOff + C.nrec > P.recCap || pairOff + C.npair > P.pairCap))
         {
-            atomicExch(&P.ctrl->overflow, 1u);
+            raise_flag(&P.ctrl->overflow);
             ok = false;
         }
         if (ok)
@@ -1452,7 +1489,7 @@ __global__ __launch_bounds__(kClipBlock) void k_clip(SetupParams P)
             pairOff = off >> kRecBits;
             if (recOff + J.nrec > P.recCap || pairOff + J.npair > P.pairCap)
             {
-                if (li == 0) atomicExch(&P.ctrl->overflow, 1u);   // the host grows the buffers and runs setup again
+                if (li == 0) raise_flag(&P.ctrl->overflow);   // the host grows the buffers and runs setup again
                 live = false;
             }
         }
@@ -1966,10 +2003,11 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_ctrl_reset(FrameCtrl* ctrl, hipStream_t s)
+hipError_t launch_frame_reset(FrameCtrl* ctrl, uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb, hipStream_t s)
 {
     (void)hipGetLastError();   // drop a stale error from an earlier call
-    hipLaunchKernelGGL(k_ctrl_reset, dim3(1), dim3(256), 0, s, ctrl);
+    const uint32_t fill = (std::max(na, nb) + 255u) / 256u;
+    hipLaunchKernelGGL(k_frame_reset, dim3(1 + std::min(fill, 128u)), dim3(256), 0, s, ctrl, a, na, b, nb);
     return hipGetLastError();
 }
 
@@ -1978,14 +2016,6 @@ hipError_t launch_vertex(const SetupParams& p, hipStream_t s)
     (void)hipGetLastError();   // drop a stale error from an earlier call
     if (p.vtxBlocks == 0) return hipSuccess;
     hipLaunchKernelGGL(k_vertex, dim3(p.vtxBlocks), dim3(kVertexBlock), 0, s, p);
-    return hipGetLastError();
-}
-
-hipError_t launch_fill_u64(unsigned long long* p, unsigned long long v, uint64_t n, hipStream_t s)
-{
-    (void)hipGetLastError();   // drop a stale error from an earlier call
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(n, 256)), dim3(256), 0, s, p, v, n);
     return hipGetLastError();
 }
 
@@ -2001,7 +2031,7 @@ hipError_t launch_chunk_scan(const SetupParams& p, hipStream_t s)
     (void)hipGetLastError();   // drop a stale error from an earlier call
     const uint32_t blocks = (p.numChunks + kScanBlock - 1) / kScanBlock;
     hipLaunchKernelGGL(k_chunk_scan, dim3(blocks), dim3(kScanBlock), 0, s, p);
-    hipLaunchKernelGGL(k_surv_map, dim3((p.numChunks + kSurvMapChunks - 1) / kSurvMapChunks), dim3(64 * kSurvMapChunks), 0, s, p);
+    if (p.numChunks > kScanMapChunks) hipLaunchKernelGGL(k_surv_map, dim3((p.numChunks + kSurvMapChunks - 1) / kSurvMapChunks), dim3(64 * kSurvMapChunks), 0, s, p);
     return hipGetLastError();
 }
 
