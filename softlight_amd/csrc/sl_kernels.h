@@ -21,13 +21,18 @@ hipError_t launch_clip(const SetupParams& p, hipStream_t s);
 // entries (a multiple of 64, at least kMinBinBlock).
 constexpr uint32_t kMaxBinBlocks = 512;
 constexpr uint32_t kMinBinBlock = 256;   // (1,024: a frame of 1,000 .. 3,000 entries spent 13 us in a few waves of the scatter, now 5)
-struct BinPlan { uint32_t blocks; uint32_t per; };
-BinPlan bin_plan(uint32_t entries);
+// The kernels work out `per` from the device's entry count, so a launch needs
+// only an upper bound of the entries (blocks past the count end at once).
+__host__ __device__ inline uint32_t bin_per(uint32_t entries)
+{
+    const uint32_t per = (entries / kMaxBinBlocks + (entries % kMaxBinBlocks ? 1u : 0u) + 63u) / 64u * 64u;
+    return per > kMinBinBlock ? per : kMinBinBlock;
+}
 // With items non-null the tile scan also writes the raster's work items of
 // the heavy-tile split (see RasterItem): tiles of more than splitAbove
 // records cut into parts of about partRecs records, at most maxParts parts.
 hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const FrameCtrl* ctrl, uint32_t cap,
-                          BinPlan plan, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
+                          uint32_t entries, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items = nullptr,
                           uint32_t* itemCount = nullptr, uint32_t partRecs = 1,
                           uint32_t splitAbove = 0, uint32_t maxParts = 0);

@@ -1573,10 +1573,10 @@ __device__ __forceinline__ uint32_t bin_entries(const FrameCtrl* ctrl, uint32_t 
 
 // Block b of the binning kernels owns entries [b*per, (b+1)*per).
 __global__ __launch_bounds__(256) void k_bin_count(const uint32_t* __restrict__ keys, const FrameCtrl* __restrict__ ctrl,
-                                                   uint32_t cap, uint32_t per, uint32_t* __restrict__ counts, int numTiles)
+                                                   uint32_t cap, uint32_t* __restrict__ counts, int numTiles)
 {
     extern __shared__ uint32_t sCnt[];
-    const uint32_t n = bin_entries(ctrl, cap);
+    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n);
     const uint32_t start = blockIdx.x * per;
     if (start >= n) return;
     const uint32_t end = min(start + per, n);
@@ -1596,14 +1596,14 @@ __global__ __launch_bounds__(256) void k_bin_count(const uint32_t* __restrict__ 
 // column split into 8 parts summed independently, then scanned in order.
 constexpr int kColTiles = 32, kColParts = 8;
 
-__global__ __launch_bounds__(kColTiles * kColParts) void k_bin_colscan(const FrameCtrl* __restrict__ ctrl, uint32_t cap, uint32_t per,
+__global__ __launch_bounds__(kColTiles * kColParts) void k_bin_colscan(const FrameCtrl* __restrict__ ctrl, uint32_t cap,
                                                                       uint32_t* __restrict__ counts, uint32_t* __restrict__ totals,
                                                                       int numTiles)
 {
     __shared__ uint32_t sPart[kColParts][kColTiles];
     const int tl = threadIdx.x % kColTiles, part = threadIdx.x / kColTiles;
     const int t = blockIdx.x * kColTiles + tl;
-    const uint32_t n = bin_entries(ctrl, cap);
+    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n);
     const uint32_t blocks = (n + per - 1) / per;
     const uint32_t rpp = (blocks + kColParts - 1) / kColParts;
     const uint32_t r0 = min(blocks, part * rpp), r1 = min(blocks, r0 + rpp);
@@ -1829,12 +1829,12 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
 }
 
 __global__ __launch_bounds__(64) void k_bin_scatter(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                    const FrameCtrl* __restrict__ ctrl, uint32_t cap, uint32_t per,
+                                                    const FrameCtrl* __restrict__ ctrl, uint32_t cap,
                                                     const uint32_t* __restrict__ counts, const uint2* __restrict__ range,
                                                     uint32_t* __restrict__ out, int numTiles)
 {
     extern __shared__ uint32_t sBase[];
-    const uint32_t n = bin_entries(ctrl, cap);
+    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n);
     const uint32_t start = blockIdx.x * per;
     if (start >= n) return;
     const uint32_t end = min(start + per, n);
@@ -2070,32 +2070,21 @@ hipError_t launch_blit(const BlitParams& p, int srcType, int dstType, hipStream_
     return hipGetLastError();
 }
 
-BinPlan bin_plan(uint32_t entries)
-{
-    BinPlan b;
-    uint64_t per = ((uint64_t)entries + kMaxBinBlocks - 1) / kMaxBinBlocks;
-    per = (per + 63) / 64 * 64;
-    if (per < kMinBinBlock) per = kMinBinBlock;
-    b.per = (uint32_t)per;
-    b.blocks = (uint32_t)(((uint64_t)entries + per - 1) / per);
-    if (b.blocks == 0) b.blocks = 1;
-    return b;
-}
-
 hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const FrameCtrl* ctrl, uint32_t cap,
-                          BinPlan plan, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
+                          uint32_t entries, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items, uint32_t* itemCount,
                           uint32_t partRecs, uint32_t splitAbove, uint32_t maxParts)
 {
     SplitPlan sp{items, itemCount, partRecs, splitAbove, maxParts};
     (void)hipGetLastError();   // drop a stale error from an earlier call
     const size_t lds = sizeof(uint32_t) * (size_t)numTiles;
-    hipLaunchKernelGGL(k_bin_count, dim3(plan.blocks), dim3(256), lds, s, keys, ctrl, cap, plan.per, counts, numTiles);
+    const uint32_t blocks = std::min(kMaxBinBlocks, std::max(1u, (entries + kMinBinBlock - 1) / kMinBinBlock));
+    hipLaunchKernelGGL(k_bin_count, dim3(blocks), dim3(256), lds, s, keys, ctrl, cap, counts, numTiles);
     hipLaunchKernelGGL(k_bin_colscan, dim3((numTiles + kColTiles - 1) / kColTiles), dim3(kColTiles * kColParts), 0, s,
-                       ctrl, cap, plan.per, counts, totals, numTiles);
+                       ctrl, cap, counts, totals, numTiles);
     if (numTiles > 1024 * kTilesPerThread) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_bin_tilescan, dim3(1), dim3(1024), 0, s, totals, range, order, numTiles, sp);
-    hipLaunchKernelGGL(k_bin_scatter, dim3(plan.blocks), dim3(64), lds, s, keys, vals, ctrl, cap, plan.per, counts, range, out,
+    hipLaunchKernelGGL(k_bin_scatter, dim3(blocks), dim3(64), lds, s, keys, vals, ctrl, cap, counts, range, out,
                        numTiles);
     return hipGetLastError();
 }

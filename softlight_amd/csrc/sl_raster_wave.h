@@ -156,8 +156,9 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     __shared__ uint32_t sMetaW[4][64];
     __shared__ float4 sResW[4][64];
 
-    // a frame whose setup outgrew the bin capacities leaves its targets untouched
-    if (P.ctrl != nullptr && P.ctrl->overflow != 0u) return;
+    // a frame whose setup outgrew the bin capacities (or went wrong) leaves its
+    // targets untouched: the host reads the flags after the whole frame
+    if (P.ctrl != nullptr && (P.ctrl->overflow | P.ctrl->error) != 0u) return;
 
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = (int)(threadIdx.x & 63);
@@ -624,7 +625,7 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
 // workgroup per split tile (the work item of its part 0).
 static __global__ __launch_bounds__(256) void k_split_fold(RasterParams P, int tileShiftX, int tileShiftY)
 {
-    if (P.ctrl != nullptr && P.ctrl->overflow != 0u) return;
+    if (P.ctrl != nullptr && (P.ctrl->overflow | P.ctrl->error) != 0u) return;
     if (blockIdx.x >= P.itemCount[1]) return;
     const RasterItem item = P.items[blockIdx.x];
     if (item.part != 0u) return;

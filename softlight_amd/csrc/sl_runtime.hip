@@ -89,14 +89,16 @@ struct Shader { uint8_t cull, dtest, dmask, blend, nvary, nout; uint32_t vsProg,
 // Device buffers of one frame.
 struct FrameRes
 {
-    DevBuf draws, uni, recs, vars, keys, vals, sorted, clip, status, ranges, ctrl, binCounts, binTotals, order;
+    // draws: the batch's tables (table_layout): draw descriptors, uniform
+    // snapshots, the vertex pass's work table
+    DevBuf draws, recs, vars, keys, vals, sorted, clip, status, ranges, ctrl, binCounts, binTotals, order;
     uint32_t recCap = 0, pairCap = 0, clipCap = 0;
     // heavy-tile split: work items, their counts, per part slot the first
     // pass's depths and the part results, per split tile and pixel the last
     // part with a pending fragment (absent: no split)
     DevBuf items, itemCount, partDepth, partRes, partWin;
     uint32_t maxParts = 0;
-    DevBuf positions, vtxDraws;   // the vertex pass's output and work table
+    DevBuf positions;             // the vertex pass's output
 };
 
 struct FrameGraph
@@ -246,6 +248,11 @@ uint32_t bytes_per_index(int type)
 
 }  // namespace
 
+// The pinned allocation of a context: the control block's readback, then the
+// first staging of queued uploads (a batch of some 180 draws).
+constexpr size_t kCtrlBytes = (sizeof(FrameCtrl) + 255) / 256 * 256;
+constexpr size_t kFirstStage = 256u << 10;
+
 struct sl_context
 {
     hipStream_t stream = nullptr;
@@ -273,6 +280,9 @@ struct sl_context
     FrameGraph graph;                              // captured frame
     uint64_t lastTotals[3] = {0, 0, 0};            // records, bin entries, clip jobs of the last eager frame
     FrameCtrl* hCtrl = nullptr;                    // pinned readback of the control block
+    uint8_t* stage = nullptr;                      // pinned staging of queued uploads (stage_space): behind hCtrl, or
+    void* stageOwn = nullptr;                      // an allocation of its own
+    size_t stageBytes = 0, stageUsed = 0;
     hipEvent_t ev[11] = {};                        // eager frames: 0-5 stages, 6-7 graph replays, 8-9 counting pass, 10 binning
     hipEvent_t bwdEv[2] = {};                      // first / last backward since the last collection
     hipEvent_t gEv[4] = {};                        // graph replays: setup start/end, raster start/end
@@ -384,6 +394,20 @@ int flush(sl_context* c, bool staticScratch = false);
 // ---------------------------------------------------------------------------
 // batch execution
 // ---------------------------------------------------------------------------
+// A batch's tables lie in one device buffer, uploaded by one copy: the draw
+// descriptors, then the uniform snapshots, then the vertex pass's work table.
+struct TableLayout { size_t uni, vtx, bytes; };
+
+TableLayout table_layout(const Batch& B)
+{
+    auto up = [](size_t n) { return (n + 255) & ~size_t(255); };
+    TableLayout t;
+    t.uni = up(sizeof(DrawDesc) * B.draws.size());
+    t.vtx = t.uni + up(std::max<size_t>(B.uni.size(), 16));
+    t.bytes = t.vtx + sizeof(VtxDraw) * B.vtxDraws.size();
+    return t;
+}
+
 // Everything derived from a batch and its target framebuffer.
 struct Plan
 {
@@ -498,8 +522,7 @@ int ensure_frame(sl_context* c, FrameRes& R, const Plan& p, const Batch& B)
     if ((rc = ensure(c, R.order, sizeof(uint32_t) * (size_t)p.numTiles)) != SL_OK) return rc;
     if (B.totalTris == 0) return SL_OK;
     if (R.recCap == 0) { R.recCap = 1u << 18; R.pairCap = 1u << 20; R.clipCap = 1u << 16; }
-    if ((rc = ensure(c, R.draws, sizeof(DrawDesc) * B.draws.size())) != SL_OK) return rc;
-    if ((rc = ensure(c, R.uni, std::max<size_t>(B.uni.size(), 16))) != SL_OK) return rc;
+    if ((rc = ensure(c, R.draws, table_layout(B).bytes)) != SL_OK) return rc;
     if ((rc = ensure(c, R.status, chunk_buffer_bytes(p.chunks))) != SL_OK) return rc;
     if ((rc = ensure(c, R.recs, sizeof(SetupRec) * (size_t)R.recCap)) != SL_OK) return rc;
     if ((rc = ensure(c, R.vars, sizeof(float4) * (size_t)p.varStride * R.recCap)) != SL_OK) return rc;
@@ -512,7 +535,6 @@ int ensure_frame(sl_context* c, FrameRes& R, const Plan& p, const Batch& B)
     if (B.posEntries > 0)
     {
         if ((rc = ensure(c, R.positions, sizeof(float4) * (size_t)B.posEntries)) != SL_OK) return rc;
-        if ((rc = ensure(c, R.vtxDraws, sizeof(VtxDraw) * B.vtxDraws.size())) != SL_OK) return rc;
     }
     if (c->splitRecs > 0)
     {
@@ -535,7 +557,8 @@ SetupParams setup_params(const Plan& p, const Batch& B, FrameRes& R)
     sp.draws = reinterpret_cast<const DrawDesc*>(R.draws.p);
     sp.numDraws = (uint32_t)B.draws.size();
     sp.totalTris = B.totalTris;
-    sp.uniforms = reinterpret_cast<const uint8_t*>(R.uni.p);
+    const TableLayout tables = table_layout(B);
+    sp.uniforms = reinterpret_cast<const uint8_t*>(R.draws.p) + tables.uni;
     sp.W = p.W; sp.H = p.H; sp.tilesX = p.tilesX; sp.tilesY = p.tilesY;
     sp.tileShiftX = ilog2i(p.tc.tileW);
     sp.tileShiftY = ilog2i(p.tc.tileH);
@@ -559,7 +582,7 @@ SetupParams setup_params(const Plan& p, const Batch& B, FrameRes& R)
     if (B.posEntries > 0)
     {
         sp.positions = reinterpret_cast<float4*>(R.positions.p);
-        sp.vtxDraws = reinterpret_cast<const VtxDraw*>(R.vtxDraws.p);
+        sp.vtxDraws = reinterpret_cast<const VtxDraw*>(reinterpret_cast<const uint8_t*>(R.draws.p) + tables.vtx);
         sp.numVtxDraws = (uint32_t)B.vtxDraws.size();
         sp.vtxBlocks = (uint32_t)(B.posEntries / kVertexItem);
     }
@@ -570,7 +593,7 @@ RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool have
 {
     RasterParams rp{};
     rp.draws = reinterpret_cast<const DrawDesc*>(R.draws.p);
-    rp.uniforms = reinterpret_cast<const uint8_t*>(R.uni.p);
+    rp.uniforms = reinterpret_cast<const uint8_t*>(R.draws.p) + table_layout(B).uni;
     rp.recs = reinterpret_cast<const SetupRec*>(R.recs.p);
     rp.vars = reinterpret_cast<const float4*>(R.vars.p);
     rp.varStride = p.varStride;
@@ -676,8 +699,9 @@ int enqueue_front(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, hip
     return SL_OK;
 }
 
-// Binning and raster.  entries sizes the grids (a graph uses the capacity;
-// the kernels read the actual counts from the control block).
+// Binning and raster.  entries bounds the bin entries and sizes the grids (the
+// capacity, where the count has not been read back; the kernels read the
+// actual counts from the control block).
 int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint32_t entries, hipStream_t s,
                  hipEvent_t evBin0, hipEvent_t evBin1)
 {
@@ -693,7 +717,7 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
             // with the heavy-tile split on, the tile scan also writes the
             // raster's work items
             const uint32_t partRecs = std::max<uint32_t>(c->splitRecs, 1u);
-            if ((rc = check(c, launch_binning(sp.pairKeys, sp.pairVals, sp.ctrl, R.pairCap, bin_plan(entries),
+            if ((rc = check(c, launch_binning(sp.pairKeys, sp.pairVals, sp.ctrl, R.pairCap, entries,
                                               reinterpret_cast<uint32_t*>(R.binCounts.p), reinterpret_cast<uint32_t*>(R.binTotals.p),
                                               reinterpret_cast<uint2*>(R.ranges.p), reinterpret_cast<uint32_t*>(R.sorted.p),
                                               reinterpret_cast<uint32_t*>(R.order.p), p.numTiles, s,
@@ -714,17 +738,68 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
     return check(c, launch_raster(rp, p.numTiles, 0, p.cfg, p.debug, s), "raster");
 }
 
-int upload_batch(sl_context* c, FrameRes& R, const Batch& B, hipStream_t s)
+// Page-locked staging for uploads that are queued on the stream instead of
+// waited for.  Space is taken in order; when it runs out the stream is waited
+// for and the space is free again (as after every eager frame, which ends in
+// a wait).  It grows with the largest request, and belongs to the context.
+void* stage_space(sl_context* c, size_t bytes, int& rc)
+{
+    const size_t n = (bytes + 255) & ~size_t(255);
+    rc = SL_OK;
+    if (c->stageUsed + n > c->stageBytes)
+    {
+        if ((rc = check(c, hipStreamSynchronize(c->stream), "sync")) != SL_OK) return nullptr;
+        c->stageUsed = 0;
+        if (n > c->stageBytes)
+        {
+            if (c->stageOwn) (void)hipHostFree(c->stageOwn);
+            c->stageOwn = nullptr;
+            c->stageBytes = 0;
+            const size_t want = std::max<size_t>(n + n / 2, 1u << 20);
+            void* h = nullptr;
+            if (hipHostMalloc(&h, want, hipHostMallocDefault) != hipSuccess)
+            {
+                rc = fail(c, SL_ERR_OUT_OF_MEMORY, "upload staging");
+                return nullptr;
+            }
+            c->stageOwn = h;
+            c->stage = reinterpret_cast<uint8_t*>(h);
+            c->stageBytes = want;
+        }
+    }
+    void* at = c->stage + c->stageUsed;
+    c->stageUsed += n;
+    return at;
+}
+
+// Queues an upload of n bytes from host memory that may change right away.
+int upload_queued(sl_context* c, void* dst, const void* src, size_t n, const char* what)
 {
     int rc;
+    void* h = stage_space(c, n, rc);
+    if (rc != SL_OK) return rc;
+    std::memcpy(h, src, n);
+    return check(c, hipMemcpyAsync(dst, h, n, hipMemcpyHostToDevice, c->stream), what);
+}
+
+// staged: through the context's staging; else straight from the batch, without
+// allocating (sl_draw_static, whose batch has no vertex pass).
+int upload_batch(sl_context* c, FrameRes& R, const Batch& B, bool staged)
+{
     if (B.draws.empty()) return SL_OK;
-    if ((rc = check(c, hipMemcpyAsync(R.draws.p, B.draws.data(), sizeof(DrawDesc) * B.draws.size(), hipMemcpyHostToDevice, s), "upload draws")) != SL_OK) return rc;
-    if (!B.uni.empty() && (rc = check(c, hipMemcpyAsync(R.uni.p, B.uni.data(), B.uni.size(), hipMemcpyHostToDevice, s), "upload uniforms")) != SL_OK) return rc;
-    if (!B.vtxDraws.empty() &&
-        (rc = check(c, hipMemcpyAsync(R.vtxDraws.p, B.vtxDraws.data(), sizeof(VtxDraw) * B.vtxDraws.size(), hipMemcpyHostToDevice, s),
-                    "upload vertex-pass table")) != SL_OK)
-        return rc;
-    return SL_OK;
+    const TableLayout t = table_layout(B);
+    int rc;
+    if (!staged)
+    {
+        if ((rc = check(c, hipMemcpyAsync(R.draws.p, B.draws.data(), sizeof(DrawDesc) * B.draws.size(), hipMemcpyHostToDevice, c->stream), "upload draws")) != SL_OK) return rc;
+        return B.uni.empty() ? SL_OK : check(c, hipMemcpyAsync(reinterpret_cast<uint8_t*>(R.draws.p) + t.uni, B.uni.data(), B.uni.size(), hipMemcpyHostToDevice, c->stream), "upload uniforms");
+    }
+    uint8_t* h = reinterpret_cast<uint8_t*>(stage_space(c, t.bytes, rc));
+    if (rc != SL_OK) return rc;
+    std::memcpy(h, B.draws.data(), sizeof(DrawDesc) * B.draws.size());
+    if (!B.uni.empty()) std::memcpy(h + t.uni, B.uni.data(), B.uni.size());
+    if (!B.vtxDraws.empty()) std::memcpy(h + t.vtx, B.vtxDraws.data(), sizeof(VtxDraw) * B.vtxDraws.size());
+    return check(c, hipMemcpyAsync(R.draws.p, h, t.bytes, hipMemcpyHostToDevice, c->stream), "upload batch tables");
 }
 
 // Draw i's uniform block as the batch snapshotted it (empty without one).
@@ -827,7 +902,7 @@ size_t static_fixed_bytes(const Plan& p, const Batch& B)
 {
     size_t n = align256(sizeof(FrameCtrl)) + align256(sizeof(uint2) * (size_t)p.numTiles) + align256(sizeof(uint32_t) * (size_t)p.numTiles);
     if (B.totalTris == 0) return n;
-    n += align256(sizeof(DrawDesc) * B.draws.size()) + align256(std::max<size_t>(B.uni.size(), 16)) + align256(chunk_buffer_bytes(p.chunks)) +
+    n += align256(table_layout(B).bytes) + align256(chunk_buffer_bytes(p.chunks)) +
          align256(sizeof(uint32_t) * (size_t)p.numTiles);
     return n;
 }
@@ -852,8 +927,7 @@ int bind_static(sl_context* c, uint8_t* base, FrameRes& R, const Plan& p, const 
     take(R.ranges, sizeof(uint2) * (size_t)p.numTiles);
     take(R.order, sizeof(uint32_t) * (size_t)p.numTiles);
     if (B.totalTris == 0) return SL_OK;
-    take(R.draws, sizeof(DrawDesc) * B.draws.size());
-    take(R.uni, std::max<size_t>(B.uni.size(), 16));
+    take(R.draws, table_layout(B).bytes);
     take(R.status, chunk_buffer_bytes(p.chunks));
     take(R.binTotals, sizeof(uint32_t) * (size_t)p.numTiles);
     take(R.recs, sizeof(SetupRec) * recs);
@@ -914,6 +988,12 @@ int execute_batch(sl_context* c, bool staticScratch = false)
     float msVertex = 0.f, msBin = 0.f, msRaster = 0.f;
     uint32_t totalRecs = 0, totalPairs = 0, jobs = 0;
 
+    // The whole frame is queued at once and its flags are read after it: a
+    // frame that outgrew its buffers touches no pixel (the raster reads the
+    // flags first), and is run again with larger ones.  A batch whose heavy
+    // tiles may split, or without triangles, reads the entry count first: its
+    // raster's grids are sized by it.
+    const bool whole = B.totalTris > 0 && (staticScratch || c->splitRecs == 0 || split_class(B, p, c->splitAll) == kSplitNone);
     for (int attempt = 0; attempt < 4; ++attempt)
     {
         if (staticScratch)
@@ -929,7 +1009,7 @@ int execute_batch(sl_context* c, bool staticScratch = false)
             return rc;
         }
         ctrl = reinterpret_cast<FrameCtrl*>(R.ctrl.p);
-        if (attempt == 0 && (rc = upload_batch(c, R, B, s)) != SL_OK) return rc;
+        if (attempt == 0 && (rc = upload_batch(c, R, B, !staticScratch)) != SL_OK) return rc;
         if (B.totalTris == 0)
         {
             if ((rc = enqueue_front(c, R, p, B, s)) != SL_OK) return rc;
@@ -939,8 +1019,14 @@ int execute_batch(sl_context* c, bool staticScratch = false)
         if ((rc = enqueue_front(c, R, p, B, s, c->ev[8], c->ev[9], c->ev[2], c->ev[3])) != SL_OK) return rc;
         (void)hipEventRecord(c->ev[1], s);
         c->stats.setup_launches += 1;
+        if (whole)
+        {
+            if ((rc = enqueue_back(c, R, p, B, R.pairCap, s, c->ev[10], c->ev[4])) != SL_OK) return rc;
+            (void)hipEventRecord(c->ev[5], s);
+        }
         if ((rc = check(c, hipMemcpyAsync(c->hCtrl, ctrl, sizeof(FrameCtrl), hipMemcpyDeviceToHost, s), "read ctrl")) != SL_OK) return rc;
-        if ((rc = check(c, hipStreamSynchronize(s), "k_setup sync")) != SL_OK) return rc;
+        if ((rc = check(c, hipStreamSynchronize(s), "frame sync")) != SL_OK) return rc;
+        c->stageUsed = 0;
         if (c->hCtrl->error) return fail(c, SL_ERR_DEVICE, "setup emitting pass disagrees with the counting pass");
         if (!c->hCtrl->overflow) break;
         if (staticScratch)
@@ -972,10 +1058,14 @@ int execute_batch(sl_context* c, bool staticScratch = false)
         totalPairs = c->hCtrl->totalPairs;
         jobs = c->hCtrl->clipJobs;
     }
-    if ((rc = enqueue_back(c, R, p, B, totalPairs, s, c->ev[10], c->ev[4])) != SL_OK) return rc;
-    (void)hipEventRecord(c->ev[5], s);
-    if ((rc = check(c, hipMemcpyAsync(c->hCtrl, ctrl, sizeof(FrameCtrl), hipMemcpyDeviceToHost, s), "read ctrl")) != SL_OK) return rc;
-    if ((rc = check(c, hipStreamSynchronize(s), "frame sync")) != SL_OK) return rc;
+    if (!whole)
+    {
+        if ((rc = enqueue_back(c, R, p, B, totalPairs, s, c->ev[10], c->ev[4])) != SL_OK) return rc;
+        (void)hipEventRecord(c->ev[5], s);
+        if ((rc = check(c, hipMemcpyAsync(c->hCtrl, ctrl, sizeof(FrameCtrl), hipMemcpyDeviceToHost, s), "read ctrl")) != SL_OK) return rc;
+        if ((rc = check(c, hipStreamSynchronize(s), "frame sync")) != SL_OK) return rc;
+        c->stageUsed = 0;
+    }
 
     float t = 0.f;
     if (B.totalTris > 0)
@@ -1016,10 +1106,10 @@ void graph_release(sl_context* c)
     if (G.graph) (void)hipGraphDestroy(G.graph);
     G.exec = nullptr;
     G.graph = nullptr;
-    for (DevBuf* b : {&G.res.draws, &G.res.uni, &G.res.recs, &G.res.vars, &G.res.keys, &G.res.vals, &G.res.sorted,
+    for (DevBuf* b : {&G.res.draws, &G.res.recs, &G.res.vars, &G.res.keys, &G.res.vals, &G.res.sorted,
                       &G.res.clip, &G.res.status, &G.res.ranges, &G.res.ctrl, &G.res.binCounts, &G.res.binTotals, &G.res.order,
                       &G.res.items, &G.res.itemCount, &G.res.partDepth, &G.res.partRes, &G.res.partWin,
-                      &G.res.positions, &G.res.vtxDraws}) release(*b);
+                      &G.res.positions}) release(*b);
     G.res = FrameRes{};
     if (G.hCtrl) (void)hipHostFree(G.hCtrl);
     G.hCtrl = nullptr;
@@ -1045,7 +1135,7 @@ int graph_capture(sl_context* c)
     G.res.pairCap = grow(c->lastTotals[1]);
     G.res.clipCap = grow(c->lastTotals[2]);
     if ((rc = ensure_frame(c, G.res, p, B)) != SL_OK) { graph_release(c); return rc; }
-    if ((rc = upload_batch(c, G.res, B, s)) != SL_OK) { graph_release(c); return rc; }
+    if ((rc = upload_batch(c, G.res, B, true)) != SL_OK) { graph_release(c); return rc; }
     // the replays' reset keeps FrameCtrl::sticky: start it (and the rest) at zero
     if ((rc = check(c, launch_fill_u32(reinterpret_cast<uint32_t*>(G.res.ctrl.p), 0u, sizeof(FrameCtrl) / 4, s), "fill ctrl")) != SL_OK)
     {
@@ -1425,8 +1515,11 @@ int sl_context_create(sl_context** out)
         if (hipEventCreate(&e) != hipSuccess) { delete c; return SL_ERR_DEVICE; }
     for (auto& e : c->gEv)
         if (hipEventCreate(&e) != hipSuccess) { delete c; return SL_ERR_DEVICE; }
-    if (hipHostMalloc(reinterpret_cast<void**>(&c->hCtrl), sizeof(FrameCtrl), hipHostMallocDefault) != hipSuccess) { delete c; return SL_ERR_DEVICE; }
+    // the control block's readback and the first staging in one allocation
+    if (hipHostMalloc(reinterpret_cast<void**>(&c->hCtrl), kCtrlBytes + kFirstStage, hipHostMallocDefault) != hipSuccess) { delete c; return SL_ERR_DEVICE; }
     std::memset(c->hCtrl, 0, sizeof(FrameCtrl));
+    c->stage = reinterpret_cast<uint8_t*>(c->hCtrl) + kCtrlBytes;
+    c->stageBytes = kFirstStage;
     *out = c;
     return SL_OK;
 }
@@ -1440,16 +1533,17 @@ void sl_context_destroy(sl_context* c)
     for (auto& v : c->ibos) release(v.buf);
     for (auto& t : c->texs) release(t.buf);
     graph_release(c);
-    for (DevBuf* b : {&c->res.draws, &c->res.uni, &c->res.recs, &c->res.vars, &c->res.keys, &c->res.vals, &c->res.sorted,
+    for (DevBuf* b : {&c->res.draws, &c->res.recs, &c->res.vars, &c->res.keys, &c->res.vals, &c->res.sorted,
                       &c->res.clip, &c->res.status, &c->res.ranges, &c->res.ctrl, &c->res.binCounts, &c->res.binTotals, &c->res.order,
                       &c->res.items, &c->res.itemCount, &c->res.partDepth, &c->res.partRes, &c->res.partWin,
-                      &c->res.positions, &c->res.vtxDraws}) release(*b);
+                      &c->res.positions}) release(*b);
     for (auto& e : c->ev) if (e) (void)hipEventDestroy(e);
     for (auto& f : c->fbos)
         for (DevBuf* b : {&f.gradDev, &f.smoothDev, &f.smoothUniDev}) release(*b);
     release(c->smoothBounds);
     for (auto& e : c->bwdEv) if (e) (void)hipEventDestroy(e);
     for (auto& e : c->gEv) if (e) (void)hipEventDestroy(e);
+    if (c->stageOwn) (void)hipHostFree(c->stageOwn);
     if (c->hCtrl) (void)hipHostFree(c->hCtrl);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -2119,8 +2213,8 @@ int smooth_setup(sl_context* c, size_t fbo, size_t srcTex, size_t dstTex, float 
     {
         if ((rc = ensure(c, F.smoothDev, sizeof(GradDesc) * nd)) != SL_OK) return rc;
         if ((rc = ensure(c, F.smoothUniDev, U.size())) != SL_OK) return rc;
-        if ((rc = upload(c, F.smoothDev.p, G.data(), sizeof(GradDesc) * nd, "upload smoothing draws")) != SL_OK) return rc;
-        if ((rc = upload(c, F.smoothUniDev.p, U.data(), U.size(), "upload smoothing uniforms")) != SL_OK) return rc;
+        if ((rc = upload_queued(c, F.smoothDev.p, G.data(), sizeof(GradDesc) * nd, "upload smoothing draws")) != SL_OK) return rc;
+        if ((rc = upload_queued(c, F.smoothUniDev.p, U.data(), U.size(), "upload smoothing uniforms")) != SL_OK) return rc;
         F.smoothHost = G;
         F.smoothUniHost = U;
     }
@@ -2283,15 +2377,14 @@ int sl_framebuffer_backward(sl_context* c, size_t fbo, size_t gradImageTex)
         }
     }
     // the table only changes with the draws or the gradient attachments;
-    // re-upload (synchronously, after all queued work) only then
+    // re-upload (queued behind the work that reads it) only then
     hipStream_t s = c->stream;
     const bool same = F.gradHost.size() == G.size() && F.gradDev.p &&
                       std::memcmp(F.gradHost.data(), G.data(), sizeof(GradDesc) * G.size()) == 0;
     if (!same)
     {
         if ((rc = ensure(c, F.gradDev, sizeof(GradDesc) * G.size())) != SL_OK) return rc;
-        if ((rc = check(c, hipStreamSynchronize(s), "sync")) != SL_OK) return rc;
-        if ((rc = upload(c, F.gradDev.p, G.data(), sizeof(GradDesc) * G.size(), "upload backward draws")) != SL_OK) return rc;
+        if ((rc = upload_queued(c, F.gradDev.p, G.data(), sizeof(GradDesc) * G.size(), "upload backward draws")) != SL_OK) return rc;
         F.gradHost = G;
     }
     BackwardParams bp{};
