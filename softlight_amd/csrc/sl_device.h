@@ -536,6 +536,7 @@ struct SmoothParams
     // between rows y and y + 1 with its sign bit set when row y receives; NaN
     // where there is no boundary
     float2* bounds;
+    uint32_t* clippedTiles;    // per block of the boundary pass: it holds a clipped winner
 };
 
 struct BackwardParams

@@ -45,19 +45,26 @@
 // screen positions of the edge's two vertices.  Every pixel recomputes the
 // boundaries it needs from the visibility attachment (the winner's triangle
 // is re-fetched and re-transformed), so nothing but the attachment is stored.
+#include <algorithm>
+
 #include "sl_device.h"
 #include "sl_stages.h"
 #include "sl_smooth.h"
 
 namespace slg {
 
-__device__ __forceinline__ uint32_t find_saved_draw(const GradDesc* D, uint32_t n, uint32_t seq)
+// Last draw whose first sequence number is below seq (draws ordered by seqBase).
+__device__ __forceinline__ uint32_t saved_base(const GradDesc* D, uint32_t i) { return D[i].d.seqBase; }
+__device__ __forceinline__ uint32_t saved_base(const uint32_t* D, uint32_t i) { return D[i]; }
+
+template <class Bases>
+__device__ __forceinline__ uint32_t find_saved_draw(Bases D, uint32_t n, uint32_t seq)
 {
     uint32_t lo = 0, hi = n;
     while (hi - lo > 1)
     {
         const uint32_t mid = (lo + hi) >> 1;
-        if (D[mid].d.seqBase < seq) lo = mid;
+        if (saved_base(D, mid) < seq) lo = mid;
         else hi = mid;
     }
     return lo;
@@ -423,16 +430,224 @@ __device__ __forceinline__ float4 add_scaled_diff(float4 o, float w, float4 a, f
     return make_float4(o.x + w * (a.x - b.x), o.y + w * (a.y - b.y), o.z + w * (a.z - b.z), o.w + w * (a.w - b.w));
 }
 
+// ---------------------------------------------------------------------------
+// The winners of a block of pixels, in LDS.  A workgroup of kShapeThreads
+// covers kShapeW x kShapeH pixels and, beside them, the column to their left
+// and the row after them: the pixels whose winners bound them.  Each winner is
+// fetched and transformed once; a boundary used to fetch its two by itself,
+// which made up to four a pixel, each a chain of a search over the draws,
+// indices, attributes and matrices (a wave takes its draws one after the
+// other, so that these come through scalar registers).  Blocks with a clipped
+// winner are marked and left to launches of their own (k_smooth_bounds_clipped,
+// k_smooth_scatter_clipped), whose pixels fetch their winners themselves: the
+// polygons' registers and scratch would cost these kernels their occupancy.
+// Measured per 2048x1024 framebuffer (eight views of eight spheres, triangles
+// of a pixel or two, so nearly every pixel is a boundary): boundary pass 142 ->
+// 107 us and 5 for the clipped launch, adjoint 267 -> 185 and 4 (half its gain
+// from add_position's pairing; the rest of it is position atomics and the
+// latency of the winners' fetches).
+// ---------------------------------------------------------------------------
+constexpr int kShapeW = 32, kShapeH = 8;
+constexpr int kShapeCols = kShapeW + 1, kShapeEntries = kShapeCols * (kShapeH + 1);
+constexpr int kShapeThreads = 320;
+constexpr int kShapeDraws = 64;       // draws whose sequence bases are searched in LDS
+static_assert(kShapeEntries <= kShapeThreads, "one entry per thread");
+enum : uint32_t { kShapeNone = 0, kShapeTri = 1, kShapeClipped = 2 };
+
+struct ShapeTile
+{
+    uint32_t seq[kShapeEntries];
+    uint32_t kind[kShapeEntries];
+    uint32_t draw[kShapeEntries];
+    uint32_t vid[3][kShapeEntries];
+    float rx[3][kShapeEntries], ry[3][kShapeEntries];
+    uint32_t base[kShapeDraws];
+};
+
+__device__ __forceinline__ SVert tile_vert(const SmoothParams& P, const ShapeTile& T, int i, int j)
+{
+    SVert v;
+    v.rx = T.rx[j][i];
+    v.ry = T.ry[j][i];
+    v.vid = T.vid[j][i];
+    v.orig = true;
+    float2 o = make_float2(0.f, 0.f);
+    if (P.posOffset != nullptr && v.vid < P.numVerts) o = P.posOffset[(uint64_t)T.draw[i] * P.numVerts + v.vid];
+    v.sx = v.rx + o.x;
+    v.sy = v.ry + o.y;
+    return v;
+}
+
+// Fills T for the block at (x0, y0); every thread of the workgroup calls it.
+// What it holds (the same for all of them): kShapeNone where no two
+// neighbours' winners differ, kShapeClipped where one that bounds another is
+// clipped.
+__device__ __forceinline__ uint32_t load_shapes(const SmoothParams& P, ShapeTile& T, int x0, int y0)
+{
+    const int i = (int)threadIdx.x;
+    const int ex = i % kShapeCols, ey = i / kShapeCols;
+    const int x = x0 - 1 + ex, y = y0 + ey;
+    const bool entry = i < kShapeEntries;
+    const bool inb = entry && x >= 0 && x < P.W && y < P.H;
+    const bool ldsDraws = P.numDraws <= (uint32_t)kShapeDraws;
+    if (ldsDraws && i < (int)P.numDraws) T.base[i] = P.draws[i].d.seqBase;
+    const uint32_t seq = inb ? __float_as_uint(P.vis[(uint64_t)y * P.W + x].x) : 0u;
+    if (entry)
+    {
+        T.seq[i] = seq;
+        T.kind[i] = kShapeNone;
+    }
+    __syncthreads();
+    // does the entry bound a neighbour of the tile that shows something else
+    bool need = false;
+    if (entry)
+    {
+        need = (ex > 0 && T.seq[i - 1] != seq) || (ex + 1 < kShapeCols && T.seq[i + 1] != seq) ||
+               (ey > 0 && T.seq[i - kShapeCols] != seq) || (ey < kShapeH && T.seq[i + kShapeCols] != seq);
+        need = need && inb;
+    }
+    if (!__syncthreads_or(need)) return kShapeNone;
+    bool clipped = false;
+    need = need && seq != 0u;
+    uint32_t k = 0;
+    if (need) k = ldsDraws ? find_saved_draw(T.base, P.numDraws, seq) : find_saved_draw(P.draws, P.numDraws, seq);
+    for (uint64_t left = __ballot(need); left != 0;)
+    {
+        const uint32_t cur = (uint32_t)__builtin_amdgcn_readlane((int)k, __ffsll((unsigned long long)left) - 1);
+        const DrawDesc& D = P.draws[cur].d;
+        const bool mine = need && k == cur;
+        left &= ~__ballot(mine);
+        if (!mine || seq <= D.seqBase) continue;
+        const uint64_t t = (uint64_t)(seq - 1u - D.seqBase);
+        if (t >= D.numTris) continue;
+        const uint64_t inst = (D.numTris == D.trisPerInstance) ? 0 : t / D.trisPerInstance;
+        const uint64_t ti = t - inst * D.trisPerInstance;
+        const uint64_t e = D.elementBegin + 3u * ti;
+        uint32_t vid[3] = {(uint32_t)e, (uint32_t)(e + 1), (uint32_t)(e + 2)};
+        if (D.indexed)
+        {
+#pragma unroll
+            for (int j = 0; j < 3; ++j) vid[j] = (uint32_t)fetch_index(D, e + j);
+        }
+        const bool all3[3] = {true, true, true};
+        float4 pos[3];
+        vertex_positions3(D, P.uniforms, vid, inst, all3, pos);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) pos[j] = mat_mul(D.scissor, pos[j]);
+        const int status = clip_status(pos[0], pos[1], pos[2]);
+        clipped = status == 1;
+        if (status != 3) continue;
+        T.kind[i] = kShapeTri;
+        T.draw[i] = cur;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+        {
+            const float4 sp = divide_and_snap(pos[j], D.vp);
+            T.vid[j][i] = vid[j];
+            T.rx[j][i] = sp.x;
+            T.ry[j][i] = sp.y;
+        }
+    }
+    return __syncthreads_or(clipped) ? kShapeClipped : kShapeTri;
+}
+
+// boundary_x / boundary_y of the pixel of tile entry i, its winners from the tile.
+__device__ __forceinline__ Bnd tile_boundary_x(const SmoothParams& P, const ShapeTile& T, int i, int x, int y)
+{
+    if (x <= 0 || T.seq[i - 1] == T.seq[i]) return no_bnd();
+    const float lo = (float)x, hi = (float)(x + 1), yf = (float)y;
+    Bnd B = no_bnd();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+    {
+        if (B.ok) continue;
+        // the right end of the left pixel's winner, else the left end of this one's
+        const int n = i - 1 + q;
+        if (T.kind[n] != kShapeTri) continue;
+        End l, r;
+        tri_row_ends(tile_vert(P, T, n, 0), tile_vert(P, T, n, 1), tile_vert(P, T, n, 2), yf, l, r);
+        const End e = q == 0 ? r : l;
+        if (e.e >= lo && e.e < hi) B = make_bnd(T.draw[n], e, true, hi, yf, 1.f);
+    }
+    return B;
+}
+
+__device__ __forceinline__ Bnd tile_boundary_y(const SmoothParams& P, const ShapeTile& T, int i, int x, int y)
+{
+    if (y + 1 >= P.H || T.seq[i] == T.seq[i + kShapeCols]) return no_bnd();
+    const float lo = (float)y, hi = (float)(y + 1), u = (float)(x + 1);
+    Bnd B = no_bnd();
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+    {
+        if (B.ok) continue;
+        // the high end of row y's winner, else the low end of row y + 1's
+        const int n = i + q * kShapeCols;
+        if (T.kind[n] != kShapeTri) continue;
+        const SVert a = tile_vert(P, T, n, 0), b = tile_vert(P, T, n, 1), c = tile_vert(P, T, n, 2);
+        End l, h;
+        bool any = false;
+        col_edge(a, b, u, any, l, h);
+        col_edge(b, c, u, any, l, h);
+        col_edge(c, a, u, any, l, h);
+        const End e = q == 0 ? h : l;
+        if (any && e.e >= lo && e.e <= hi) B = col_bnd(T.draw[n], e, y, x);
+    }
+    return B;
+}
+
+// The workgroup's block and the thread's pixel (entry i of the tile); threads
+// of the halo have none.
+__device__ __forceinline__ bool tile_pixel(const SmoothParams& P, int& x0, int& y0, int& x, int& y, int& i)
+{
+    const int bxN = (P.W + kShapeW - 1) / kShapeW;
+    x0 = (int)(blockIdx.x % (unsigned)bxN) * kShapeW;
+    y0 = (int)(blockIdx.x / (unsigned)bxN) * kShapeH;
+    i = (int)threadIdx.x;
+    const int ex = i % kShapeCols, ey = i / kShapeCols;
+    x = x0 - 1 + ex;
+    y = y0 + ey;
+    return ex > 0 && ey < kShapeH && x < P.W && y < P.H;
+}
+
 // The boundary pass: each pixel's row-pass boundary (x - 1 | x) and
 // column-pass boundary (y | y + 1), as weights (NaN: none; the column
 // weight's sign bit: row y receives).  Every pass below reads them, so each
-// boundary's winners are fetched once instead of by every pixel that uses it.
-__global__ __launch_bounds__(256) void k_smooth_bounds(SmoothParams P)
+// boundary is worked out once instead of by every pixel that uses it.
+__global__ __launch_bounds__(kShapeThreads) void k_smooth_bounds(SmoothParams P)
 {
-    const uint64_t n = (uint64_t)P.W * P.H;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    __shared__ ShapeTile T;
+    int x0, y0, x, y, e;
+    const bool mine = tile_pixel(P, x0, y0, x, y, e);
+    const uint32_t kind = load_shapes(P, T, x0, y0);
+    if (threadIdx.x == 0) P.clippedTiles[blockIdx.x] = kind == kShapeClipped ? 1u : 0u;
+    if (!mine || kind == kShapeClipped) return;
+    const float none = __builtin_nanf("");
+    float wx = none, wy = none;
+    if (kind == kShapeTri)
     {
-        const int x = (int)(i % (uint64_t)P.W), y = (int)(i / (uint64_t)P.W);
+        const Bnd Bx = tile_boundary_x(P, T, e, x, y);
+        if (Bx.ok) wx = bnd_weight(Bx, P.sigma);
+        const Bnd By = tile_boundary_y(P, T, e, x, y);
+        if (By.ok)
+        {
+            const float w = bnd_weight(By, P.sigma);
+            wy = By.recvLow ? -w : w;
+        }
+    }
+    P.bounds[(uint64_t)y * P.W + x] = make_float2(wx, wy);
+}
+
+// The boundaries of the blocks marked as holding clipped winners, one block a
+// workgroup at a time.
+__global__ __launch_bounds__(kShapeW * kShapeH) void k_smooth_bounds_clipped(SmoothParams P)
+{
+    const int bxN = (P.W + kShapeW - 1) / kShapeW, n = bxN * ((P.H + kShapeH - 1) / kShapeH);
+    for (int b = (int)blockIdx.x; b < n; b += (int)gridDim.x)
+    {
+        if (P.clippedTiles[b] == 0u) continue;
+        const int x = (b % bxN) * kShapeW + (int)threadIdx.x % kShapeW, y = (b / bxN) * kShapeH + (int)threadIdx.x / kShapeW;
+        if (x >= P.W || y >= P.H) continue;
         const Bnd Bx = boundary_x(P, x, y);
         const Bnd By = boundary_y(P, x, y);
         const float wx = Bx.ok ? bnd_weight(Bx, P.sigma) : __builtin_nanf("");
@@ -442,7 +657,7 @@ __global__ __launch_bounds__(256) void k_smooth_bounds(SmoothParams P)
             const float w = bnd_weight(By, P.sigma);
             wy = By.recvLow ? -w : w;
         }
-        P.bounds[i] = make_float2(wx, wy);
+        P.bounds[(uint64_t)y * P.W + x] = make_float2(wx, wy);
     }
 }
 
@@ -527,24 +742,36 @@ __device__ __forceinline__ float dot4f(float4 a, float4 b)
     return ((a.x * b.x) + (a.y * b.y)) + ((a.z * b.z) + (a.w * b.w));
 }
 
+// Adds a vertex's two position gradients for every lane with `on` (others pass
+// anything): neighbouring lanes take the x and the y of one vertex, first the
+// even lane's, then the odd lane's, so that an atomic instruction touches 32
+// places and not 64.  Every lane of the wave calls it.
+__device__ __forceinline__ void add_position(const SmoothParams& P, bool on, uint64_t at, float gx, float gy)
+{
+    const bool odd = (threadIdx.x & 1) != 0;
+    const float give = odd ? gx : gy;                              // what the neighbour adds for this lane
+    const float take = __shfl_xor(give, 1, 64);
+    const uint64_t atN = __shfl_xor(on ? at : kNoPositions, 1, 64);
+    const uint64_t atO = on ? at : kNoPositions;
+    float* base = reinterpret_cast<float*>(P.posGrad);
+    // the even lane's vertex: its x here, its y by the odd lane
+    const uint64_t a0 = odd ? atN : atO;
+    if (a0 != kNoPositions) unsafeAtomicAdd(base + 2 * a0 + (odd ? 1 : 0), odd ? take : gx);
+    // the odd lane's vertex
+    const uint64_t a1 = odd ? atO : atN;
+    if (a1 != kNoPositions) unsafeAtomicAdd(base + 2 * a1 + (odd ? 1 : 0), odd ? gy : take);
+}
+
+// Every lane of the wave calls it (B.ok: the lane has a boundary).
 __device__ __forceinline__ void scatter_position(const SmoothParams& P, const Bnd& B, float dLdd, bool rowPass)
 {
-    if (dLdd == 0.f) return;
-    float p[4];
-    bnd_partials(B, p);
-    const int ax = rowPass ? 0 : 1, bx = rowPass ? 1 : 0;
-    if (B.gp && B.vp < P.numVerts)
-    {
-        float* d = reinterpret_cast<float*>(P.posGrad + (uint64_t)B.k * P.numVerts + B.vp);
-        unsafeAtomicAdd(d + ax, dLdd * p[0]);
-        unsafeAtomicAdd(d + bx, dLdd * p[1]);
-    }
-    if (B.gq && B.vq < P.numVerts)
-    {
-        float* d = reinterpret_cast<float*>(P.posGrad + (uint64_t)B.k * P.numVerts + B.vq);
-        unsafeAtomicAdd(d + ax, dLdd * p[2]);
-        unsafeAtomicAdd(d + bx, dLdd * p[3]);
-    }
+    const bool on = B.ok && dLdd != 0.f;
+    float p[4] = {0.f, 0.f, 0.f, 0.f};
+    if (on) bnd_partials(B, p);
+    const uint64_t base = (uint64_t)B.k * P.numVerts;
+    const float pa = dLdd * p[0], pb = dLdd * p[1], qa = dLdd * p[2], qb = dLdd * p[3];
+    add_position(P, on && B.gp && B.vp < P.numVerts, base + B.vp, rowPass ? pa : pb, rowPass ? pb : pa);
+    add_position(P, on && B.gq && B.vq < P.numVerts, base + B.vq, rowPass ? qa : qb, rowPass ? qb : qa);
 }
 
 // dL/dd from dL/dw: w = 1 - d / r gives dw/dd = -sigma^2 / r^3.
@@ -556,20 +783,39 @@ __device__ __forceinline__ float dL_dd(const Bnd& B, float sigma, float dLdw)
     return dLdw * (-(q * q) / r);
 }
 
-__global__ __launch_bounds__(256) void k_smooth_backward(SmoothParams P)
+// dL/d(weight) of the pixel's row-pass boundary (gx: its dL/dX) and
+// column-pass boundary.
+__device__ __forceinline__ float row_dLdw(const SmoothParams& P, uint64_t i, float4 gx)
 {
-    const uint64_t n = (uint64_t)P.W * P.H;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    return dot4f(gx, add_scaled_diff(make_float4(0.f, 0.f, 0.f, 0.f), 1.f, P.color[i - 1], P.color[i]));
+}
+
+__device__ __forceinline__ float col_dLdw(const SmoothParams& P, uint64_t i, int x, int y, bool recvLow)
+{
+    const float4 X0 = row_pass(P, x, y), X1 = row_pass(P, x, y + 1);
+    return recvLow ? dot4f(P.grad[i], add_scaled_diff(make_float4(0.f, 0.f, 0.f, 0.f), 1.f, X1, X0))
+                   : dot4f(P.grad[i + P.W], add_scaled_diff(make_float4(0.f, 0.f, 0.f, 0.f), 1.f, X0, X1));
+}
+
+__global__ __launch_bounds__(kShapeThreads) void k_smooth_backward(SmoothParams P)
+{
+    __shared__ ShapeTile T;
+    int x0, y0, x, y, e;
+    const bool mine = tile_pixel(P, x0, y0, x, y, e);
+    const uint64_t i = mine ? (uint64_t)y * P.W + x : 0;
+    if (!(P.sigma > 0.f))
     {
-        const int x = (int)(i % (uint64_t)P.W), y = (int)(i / (uint64_t)P.W);
-        if (!(P.sigma > 0.f))
-        {
-            P.out[i] = P.grad[i];
-            continue;
-        }
+        if (mine) P.out[i] = P.grad[i];
+        return;
+    }
+    const bool shapes = P.posGrad != nullptr && P.clippedTiles[blockIdx.x] == 0u && load_shapes(P, T, x0, y0) == kShapeTri;
+    float4 gx = make_float4(0.f, 0.f, 0.f, 0.f);
+    StoredBnd Sx{false, false, 0.f};
+    if (mine)
+    {
         // dL/dC = the row pass transposed over dL/dX
-        const float4 gx = grad_x_image(P, x, y);
-        const StoredBnd Sx = stored_x(P, i);
+        gx = grad_x_image(P, x, y);
+        Sx = stored_x(P, i);
         const float wx = Sx.ok ? Sx.w : 0.f;
         float4 gc = make_float4((1.f - wx) * gx.x, (1.f - wx) * gx.y, (1.f - wx) * gx.z, (1.f - wx) * gx.w);
         if (x + 1 < P.W)
@@ -578,24 +824,60 @@ __global__ __launch_bounds__(256) void k_smooth_backward(SmoothParams P)
             if (Sn.ok) gc = add_scaled_diff(gc, Sn.w, grad_x_image(P, x + 1, y), make_float4(0.f, 0.f, 0.f, 0.f));
         }
         P.out[i] = gc;
-        if (P.posGrad == nullptr) continue;
-        // this pixel's row-pass boundary (x - 1 | x) and the column-pass
-        // boundary (y | y + 1), rebuilt for their edges' vertices
-        if (Sx.ok)
-        {
-            const Bnd Bx = boundary_x(P, x, y);
-            const float dLdw = dot4f(gx, add_scaled_diff(make_float4(0.f, 0.f, 0.f, 0.f), 1.f, P.color[i - 1], P.color[i]));
-            scatter_position(P, Bx, dL_dd(Bx, P.sigma, dLdw), true);
-        }
-        if (stored_y(P, i).ok)
-        {
-            const Bnd By = boundary_y(P, x, y);
-            const float4 X0 = row_pass(P, x, y), X1 = row_pass(P, x, y + 1);
-            const float dLdw = By.recvLow ? dot4f(P.grad[i], add_scaled_diff(make_float4(0.f, 0.f, 0.f, 0.f), 1.f, X1, X0))
-                                          : dot4f(P.grad[i + P.W], add_scaled_diff(make_float4(0.f, 0.f, 0.f, 0.f), 1.f, X0, X1));
-            scatter_position(P, By, dL_dd(By, P.sigma, dLdw), false);
-        }
     }
+    if (!shapes) return;
+    // this pixel's row-pass boundary (x - 1 | x) and the column-pass
+    // boundary (y | y + 1), rebuilt for their edges' vertices
+    Bnd B = no_bnd();
+    float d = 0.f;
+    if (mine && Sx.ok)
+    {
+        B = tile_boundary_x(P, T, e, x, y);
+        d = dL_dd(B, P.sigma, row_dLdw(P, i, gx));
+    }
+    scatter_position(P, B, d, true);
+    B = no_bnd();
+    d = 0.f;
+    if (mine && stored_y(P, i).ok)
+    {
+        B = tile_boundary_y(P, T, e, x, y);
+        d = dL_dd(B, P.sigma, col_dLdw(P, i, x, y, B.recvLow));
+    }
+    scatter_position(P, B, d, false);
+}
+
+// The position gradients of the blocks with clipped winners.
+__global__ __launch_bounds__(kShapeW * kShapeH) void k_smooth_scatter_clipped(SmoothParams P)
+{
+    const int bxN = (P.W + kShapeW - 1) / kShapeW, n = bxN * ((P.H + kShapeH - 1) / kShapeH);
+    for (int b = (int)blockIdx.x; b < n; b += (int)gridDim.x)
+    {
+        if (P.clippedTiles[b] == 0u) continue;
+        const int x = (b % bxN) * kShapeW + (int)threadIdx.x % kShapeW, y = (b / bxN) * kShapeH + (int)threadIdx.x / kShapeW;
+        const bool mine = x < P.W && y < P.H;
+        const uint64_t i = mine ? (uint64_t)y * P.W + x : 0;
+        Bnd B = no_bnd();
+        float d = 0.f;
+        if (mine && stored_x(P, i).ok)
+        {
+            B = boundary_x(P, x, y);
+            d = dL_dd(B, P.sigma, row_dLdw(P, i, grad_x_image(P, x, y)));
+        }
+        scatter_position(P, B, d, true);
+        B = no_bnd();
+        d = 0.f;
+        if (mine && stored_y(P, i).ok)
+        {
+            B = boundary_y(P, x, y);
+            d = dL_dd(B, P.sigma, col_dLdw(P, i, x, y, B.recvLow));
+        }
+        scatter_position(P, B, d, false);
+    }
+}
+
+static unsigned tile_grid(const SmoothParams& p)
+{
+    return (unsigned)(((p.W + kShapeW - 1) / kShapeW) * ((p.H + kShapeH - 1) / kShapeH));
 }
 
 static unsigned smooth_grid(const SmoothParams& p)
@@ -605,11 +887,20 @@ static unsigned smooth_grid(const SmoothParams& p)
     return (unsigned)(g > 65536 ? 65536 : (g == 0 ? 1 : g));
 }
 
+// Blocks of the clipped launches: they look through the marks of all blocks.
+static unsigned clipped_grid(const SmoothParams& p) { return std::min(tile_grid(p), 1024u); }
+
+static void launch_bounds(const SmoothParams& p, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_smooth_bounds, dim3(tile_grid(p)), dim3(kShapeThreads), 0, s, p);
+    hipLaunchKernelGGL(k_smooth_bounds_clipped, dim3(clipped_grid(p)), dim3(kShapeW * kShapeH), 0, s, p);
+}
+
 hipError_t launch_smooth(const SmoothParams& p, hipStream_t s)
 {
     (void)hipGetLastError();   // drop a stale error from an earlier call
     if (p.W <= 0 || p.H <= 0) return hipSuccess;
-    if (p.sigma > 0.f) hipLaunchKernelGGL(k_smooth_bounds, dim3(smooth_grid(p)), dim3(256), 0, s, p);
+    if (p.sigma > 0.f) launch_bounds(p, s);
     hipLaunchKernelGGL(k_smooth, dim3(smooth_grid(p)), dim3(256), 0, s, p);
     return hipGetLastError();
 }
@@ -618,9 +909,16 @@ hipError_t launch_smooth_backward(const SmoothParams& p, hipStream_t s)
 {
     (void)hipGetLastError();   // drop a stale error from an earlier call
     if (p.W <= 0 || p.H <= 0) return hipSuccess;
-    if (p.sigma > 0.f) hipLaunchKernelGGL(k_smooth_bounds, dim3(smooth_grid(p)), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(k_smooth_backward, dim3(smooth_grid(p)), dim3(256), 0, s, p);
+    if (p.sigma > 0.f) launch_bounds(p, s);
+    hipLaunchKernelGGL(k_smooth_backward, dim3(tile_grid(p)), dim3(kShapeThreads), 0, s, p);
+    if (p.sigma > 0.f && p.posGrad != nullptr)
+        hipLaunchKernelGGL(k_smooth_scatter_clipped, dim3(clipped_grid(p)), dim3(kShapeW * kShapeH), 0, s, p);
     return hipGetLastError();
+}
+
+size_t smooth_tiles(int W, int H)
+{
+    return (size_t)((W + kShapeW - 1) / kShapeW) * (size_t)((H + kShapeH - 1) / kShapeH);
 }
 
 }  // namespace slg
