@@ -19,7 +19,8 @@ LIB = os.path.join(OUT, "libsoftlight_amd.so")
 SOURCES = ["sl_kernels.hip", "sl_backward.hip", "sl_smooth.hip", "sl_runtime.hip",
            # the raster's instances, split so that they compile in parallel
            "sl_raster_wave.hip", "sl_raster_wave_dbg.hip",
-           "sl_raster_modes.hip", "sl_raster_modes_dbg.hip", "sl_raster_mrt.hip"]
+           "sl_raster_direct.hip", "sl_raster_direct_dbg.hip",
+           "sl_raster_modes.hip", "sl_raster_modes_dbg.hip", "sl_raster_mrt.hip", "sl_raster_mrt_direct.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 

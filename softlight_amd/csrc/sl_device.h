@@ -423,6 +423,13 @@ constexpr uint32_t kDefaultSplitRecords = 256;  // records per part of a split t
 constexpr uint32_t kSplitAboveParts = 4;        // tiles of more than kSplitAboveParts parts' records split
 constexpr uint32_t kMaxTileParts = 1024;        // parts of one split tile at most
 
+// A batch with at least one triangle per this many pixels of the target takes
+// the raster's instances whose small records queue their own fragments: at
+// 5 .. 26 pixels a triangle (sphere and mesh scenes) these take the raster from
+// 65 to 34 us, 120 to 72 and 313 to 246; at 48 .. 400 (overlapping triangles of a
+// tenth of the target) their extra registers cost it 8 - 12% (116 -> 125 us).
+constexpr uint64_t kSmallTrianglePixels = 40;
+
 // One raster workgroup's work: a whole tile (parts == 1) or part `part` of
 // a split tile, records [begin, end) of its list; part results live in slot
 // `slot` (the tile's parts in slots slot - part .. slot - part + parts - 1);
@@ -479,6 +486,7 @@ struct RasterParams
     int32_t extra;                // some draw of the batch draws wireframe triangles, lines or points
     int32_t mrt;                  // some draw of the batch has several fragment outputs
     int32_t blend;                // some draw of the batch with outputs blends them
+    int32_t small;                // the batch's triangles are small on average (kSmallTrianglePixels)
     FrameCtrl* ctrl;
     // heavy-tile split (items == nullptr: one workgroup per tile, tileOrder)
     const RasterItem* items;      // whole tiles and parts of split tiles, parts first

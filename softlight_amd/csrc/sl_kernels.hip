@@ -2100,6 +2100,7 @@ hipError_t launch_raster(const RasterParams& p, int units, int maxParts, int cfg
     // outputs with lines or points have blending compiled in
     int aux = (debug ? 1 : 0) | (p.vis != nullptr ? 2 : 0) | (p.extra ? 4 : 0) | (p.mrt ? 8 : 0);
     if (cf != 0 && (p.blend || debug || (p.mrt && p.extra))) aux |= 32;
+    if (p.small && !p.extra) aux |= 64;
     // visibility is built for RGBA32F colour, filled triangles and single
     // outputs; several outputs need colour attachment 0
     switch (cf << 8 | aux)
@@ -2112,6 +2113,10 @@ hipError_t launch_raster(const RasterParams& p, int units, int maxParts, int cfg
         SL_RASTER(0, 5); SL_RASTER(1, 37); SL_RASTER(2, 37);
         SL_RASTER(1, 8); SL_RASTER(2, 8); SL_RASTER(1, 40); SL_RASTER(2, 40); SL_RASTER(1, 41); SL_RASTER(2, 41);
         SL_RASTER(1, 44); SL_RASTER(2, 44); SL_RASTER(1, 45); SL_RASTER(2, 45);
+        SL_RASTER(0, 64); SL_RASTER(1, 64); SL_RASTER(2, 64); SL_RASTER(1, 96); SL_RASTER(2, 96);
+        SL_RASTER(0, 65); SL_RASTER(1, 97); SL_RASTER(2, 97);
+        SL_RASTER(2, 66); SL_RASTER(2, 98); SL_RASTER(2, 99);
+        SL_RASTER(1, 72); SL_RASTER(2, 72); SL_RASTER(1, 104); SL_RASTER(2, 104); SL_RASTER(1, 105); SL_RASTER(2, 105);
 #undef SL_RASTER
         default: return hipErrorInvalidValue;
     }

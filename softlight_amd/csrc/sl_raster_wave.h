@@ -23,6 +23,24 @@ __device__ __forceinline__ float readlane_f32(float v, int l)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
+// Inclusive prefix sum over the wave's 64 lanes (every lane active): within
+// rows of 16 by shifts, then the last lanes of the rows before.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v)
+{
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v)
+{
+    v = dpp_add<0x111, 0xF>(v);   // row_shr:1
+    v = dpp_add<0x112, 0xF>(v);   // row_shr:2
+    v = dpp_add<0x114, 0xF>(v);   // row_shr:4
+    v = dpp_add<0x118, 0xF>(v);   // row_shr:8
+    v = dpp_add<0x142, 0xA>(v);   // row_bcast:15 into rows 1 and 3
+    return dpp_add<0x143, 0xC>(v);   // row_bcast:31 into rows 2 and 3
+}
+
 // LDS traffic of one wave: its operations execute in order, so ordering them
 // only needs the compiler kept from moving them.
 __device__ __forceinline__ void wave_lds_fence()
@@ -81,6 +99,12 @@ __device__ __forceinline__ void line_row(const LineWalk& w, int W, int y, bool w
     }
 }
 
+// A list's 64 records queue their own fragments when they cover at most
+// kDirectPixels pixels of the block each, on average, and none of those left
+// reaches over more than kDirectColumns columns (whose fragments' exact values
+// take many steps: the filter saves those of hidden ones).
+constexpr uint32_t kDirectPixels = 8, kDirectColumns = 64;
+
 // k_raster_wave: a wave owns an 8x8 block of its tile and walks the tile's
 // record list; a pixel's depth, colour and pending fragment live in its
 // lane's registers for the whole batch.
@@ -96,11 +120,19 @@ __device__ __forceinline__ void line_row(const LineWalk& w, int W, int y, bool w
 //            already decide become queued fragments.  `bound` holds, per
 //            pixel, a value no smaller than the depth after every fragment
 //            queued so far.
+//            Records that cover a few pixels each are not worth a step of
+//            the wave: every lane queues its own record's fragments, at the
+//            place a prefix sum over the 64 records gives it (raster kernel of
+//            64 spheres at 1080p 65 -> 33 us, of 1,000 blended mesh draws 313
+//            -> 251, of 16 views of 512x512 122 -> 71, of a frame of lines
+//            290 -> 173).
 //   flush    when 64 fragments wait: one fragment per lane, the exact
 //            barycentrics (the reference's recurrence, stepped from the
-//            span's first pixel) and depth; then each pixel takes its own
-//            fragments in record order: depth test, counters, pending
-//            fragment or blend.
+//            span's first pixel) and depth, and a blended fragment's colour;
+//            then each pixel takes its own fragments in record order: depth
+//            test, counters, pending fragment or blend.  (Shading a blended
+//            fragment when its turn came ran the programs for a lane or two
+//            at a time: 330 -> 313 us of a 1,000-sphere blended scene's raster.)
 //
 // Why: a record's cost used to be the recurrence's steps (up to W / 4 dependent
 // additions) for every lane it reached, although on overlapping triangles 98%
@@ -143,7 +175,7 @@ __device__ __forceinline__ void line_row(const LineWalk& w, int W, int y, bool w
 //
 // AUX: bit 0 debug buffers, bit 1 visibility, bit 2 wireframe, line or point
 // records in the batch, bit 3 several fragment outputs, bit 5 some draw of
-// the batch blends.
+// the batch blends, bit 6 (and bit 2) small records queue their own fragments.
 template <int CF, int AUX, int MODE>
 __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShiftX, int tileShiftY, int wavesShift, int merge)
 {
@@ -152,9 +184,16 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     constexpr bool EXTRA = (AUX & 4) != 0;
     constexpr bool MRT = (AUX & 8) != 0;
     constexpr bool BLEND = (AUX & 32) != 0;
+    constexpr bool DIRECT = (AUX & (64 | 4)) != 0;
     __shared__ uint32_t sIdW[4][64];
     __shared__ uint32_t sMetaW[4][64];
     __shared__ float4 sResW[4][64];
+    __shared__ unsigned long long sMaskW[DIRECT ? 4 : 1][DIRECT ? 64 : 1];
+    // blended fragments shaded one per lane in the flush; the outputs of a
+    // several-output program go to their attachments, so those wait their turn
+    constexpr bool EARLY = BLEND && !MRT && MODE == 0;
+    __shared__ float4 sColW[EARLY ? 4 : 1][EARLY ? 64 : 1];
+    __shared__ float4 sVisW[EARLY && VIS ? 4 : 1][EARLY && VIS ? 64 : 1];
 
     // a frame whose setup outgrew the bin capacities (or went wrong) leaves its
     // targets untouched: the host reads the flags after the whole frame
@@ -165,6 +204,9 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     uint32_t* sId = sIdW[wave];
     uint32_t* sMeta = sMetaW[wave];
     float4* sRes = sResW[wave];
+    unsigned long long* sMask = sMaskW[DIRECT ? wave : 0];
+    float4* sCol = sColW[EARLY ? wave : 0];
+    float4* sVis = sVisW[EARLY && VIS ? wave : 0];
 
     // wave -> block of a tile; tiles in launch order (heaviest first), or work items
     const int groupShift = tileShiftX + tileShiftY - 6 - wavesShift;    // log2 workgroups per tile
@@ -266,7 +308,7 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     };
 
     float bound = inb ? depth : -INFINITY;      // no smaller than the pixel's depth after the queued fragments
-    uint64_t mine = 0;                          // queued fragments of this lane's pixel
+    uint64_t own = 0;                           // queued fragments of this lane's pixel (those the wave queued)
     int queued = 0;
     uint32_t tested = 0, shaded = 0;
 
@@ -276,6 +318,9 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
     float zx = 0.f, zy = 0.f, zlo = 0.f, zwid = 0.f;
     uint64_t todo = 0;
     uint32_t masks = 0;                         // masks left of the record at hand (EXTRA)
+    bool viaLds = false;                        // some queued fragments were queued by their records
+    bool direct = false;                        // the records at hand queue their own fragments
+    uint32_t num = 0, upTo = 0, taken = 0;      // a record's fragments, theirs up to it, and those taken
     uint32_t base = range.x;
     bool more = true;
     while (more)
@@ -292,7 +337,7 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                 const int nb = (int)min(64u, range.y - base);
                 const float top = wave_max_f32(bound);
                 mask = maskBefore = maskAfter = 0;
-                bool rej = false, raise = false;
+                bool rej = false, raise = false, wide = false;
                 if (lane < nb)
                 {
                     id = P.tileRecs[base + lane];
@@ -354,6 +399,7 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                         const int dt = (int)(state & 7u);
                         const bool less = dt == SL_DEPTH_TEST_LESS_THAN || dt == SL_DEPTH_TEST_LESS_EQUAL;
                         raise = ((state >> 3) & 1u) != 0u && !less && dt != SL_DEPTH_TEST_EQUAL;
+                        wide = (R.xbox >> 16) - (R.xbox & 0xFFFFu) > kDirectColumns;
                         const float X = (float)(bx0 + 7), Y = (float)(by0 + 7);
                         zx = 0.f;
                         zy = 0.f;
@@ -407,6 +453,41 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                 const uint64_t rb = __ballot(raise);
                 const uint64_t before = (rb != 0) ? ((rb & (0ull - rb)) - 1ull) : ~0ull;
                 todo = __ballot((mask | maskBefore | maskAfter) != 0) & ~(__ballot(rej) & before);
+                direct = false;
+                // records of a few pixels each queue their fragments themselves
+                if (DIRECT && todo != 0 && ((rb | __ballot(wide)) & todo) == 0)
+                {
+                    num = (((todo >> lane) & 1ull) != 0ull) ? (uint32_t)(__popcll(mask) + __popcll(maskBefore) + __popcll(maskAfter)) : 0u;
+                    upTo = wave_prefix(num);
+                    taken = 0;
+                    direct = (uint32_t)__builtin_amdgcn_readlane((int)upTo, 63) <= kDirectPixels * (uint32_t)__popcll(todo) &&
+                             (!EXTRA || __ballot(num > 64u) == 0);
+                }
+                continue;
+            }
+            if (DIRECT && direct)
+            {
+                // as many of the records, in order, as the queue has room for
+                const uint64_t fit = __ballot(num != 0u && upTo - taken <= 64u - (uint32_t)queued) & todo;
+                if (fit == 0) break;
+                if (((fit >> lane) & 1ull) != 0ull)
+                {
+                    uint32_t e = (uint32_t)queued + upTo - num - taken;
+                    for (int q = EXTRA ? 0 : 1; q < (EXTRA ? 3 : 2); ++q)
+                    {
+                        for (uint64_t m = q == 0 ? maskBefore : (q == 1 ? mask : maskAfter); m != 0; m &= m - 1ull, ++e)
+                        {
+                            sId[e] = id;
+                            sMeta[e] = (uint32_t)(__ffsll((unsigned long long)m) - 1) | (q != 1 ? 64u : 0u) | (state << 8);
+                        }
+                    }
+                }
+                const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)upTo, 63 - __clzll((long long)fit));
+                queued += (int)(last - taken);
+                taken = last;
+                viaLds = true;
+                todo &= ~fit;
+                if (todo != 0) break;
                 continue;
             }
             const int bi = __ffsll((unsigned long long)todo) - 1;
@@ -431,8 +512,8 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                     const uint32_t e = (uint32_t)queued + lanes_below(cm);
                     sId[e] = (uint32_t)__builtin_amdgcn_readlane((int)id, bi);
                     // (a line's other masks hold its wrapped texels)
+                    own |= 1ull << e;
                     sMeta[e] = (uint32_t)lane | (EXTRA && (masks & 3u) != 2u ? 64u : 0u) | (st << 8);
-                    mine |= 1ull << e;
                     if (((st >> 3) & 1u) != 0u)
                     {
                         // the depth it can leave; a half depth target rounds it
@@ -448,7 +529,9 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
         }
         if (queued == 0) continue;
 
-        // exact barycentrics and depth of the queued fragments, one per lane
+        // exact barycentrics and depth of the queued fragments, one per lane,
+        // and each pixel's fragments as a mask
+        if (DIRECT && viaLds) sMask[lane] = 0ull;
         wave_lds_fence();
         if (lane < queued)
         {
@@ -517,53 +600,84 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                 z = (((R.z[0] * s0) + (R.z[1] * s1)) + (R.z[2] * s2)) + R.bc3;
             }
             sRes[lane] = make_float4(z, s0, s1, s2);
+            if (DIRECT && viaLds) atomicOr(&sMask[px], 1ull << lane);
+            const uint32_t st = sMeta[lane] >> 8;
+            if (EARLY && ((st >> 7) & 1u) != 0u && ((st >> 4) & 7u) != SL_BLEND_OFF)
+            {
+                // a blended fragment's colour (few of those that come this far
+                // fail their depth test)
+                const DrawDesc& D = P.draws[R.draw];
+                const float hw[3] = {R.hw[0], R.hw[1], R.hw[2]};
+                float4 out, wv;
+                (void)shade<false>(P, D, hw, R.bc3, R.state, sId[lane], s0, s1, s2, out, wv, 0, SL_BLEND_OFF);
+                sCol[lane] = out;
+                if (VIS) sVis[lane] = make_float4(__uint_as_float(R.seq), wv.x, wv.y, wv.z);
+            }
         }
         wave_lds_fence();
         // each pixel takes its fragments in record order
-        while (mine != 0)
+        uint64_t mine = own;
+        if (DIRECT && viaLds) mine |= sMask[lane];
+        own = 0;
+        viaLds = false;
+        for (;;)
         {
-            const int e = __ffsll((unsigned long long)mine) - 1;
-            mine &= mine - 1ull;
-            const float4 f = sRes[e];
-            const uint32_t rid = sId[e], st = sMeta[e] >> 8;
-            if (!depth_test((int)(st & 7u), f.x, depth)) continue;
-            if (MODE == 1)
+            bool stall = false;
+            while (mine != 0 && !stall)
             {
-                depth = f.x;
-                continue;
-            }
-            const int blendMode = (int)((st >> 4) & 7u);
-            const bool hasOut = ((st >> 7) & 1u) != 0u;
-            // an unblended fragment with outputs, and any whose visibility
-            // record is wanted, waits until the pixel's colour is needed
-            if ((hasOut && (!BLEND || blendMode == SL_BLEND_OFF)) || (VIS && !hasOut))
-            {
-                pend = rid;
-                ps0 = f.y;
-                ps1 = f.z;
-                ps2 = f.w;
-            }
-            else if (BLEND && hasOut)
-            {
-                // a blended fragment reads the colour: the pending one first
-                uint32_t r = (pend != kNoPending) ? pend : rid;
-                bool own = pend == kNoPending;
-                for (;;)
+                const int e = __ffsll((unsigned long long)mine) - 1;
+                const float4 f = sRes[e];
+                const uint32_t rid = sId[e], st = sMeta[e] >> 8;
+                if (!depth_test((int)(st & 7u), f.x, depth))
                 {
-                    shade_into(r, own ? f.y : ps0, own ? f.z : ps1, own ? f.w : ps2, own ? blendMode : SL_BLEND_OFF);
-                    if (own) break;
-                    r = rid;
-                    own = true;
+                    mine &= mine - 1ull;
+                    continue;
                 }
+                const int blendMode = (int)((st >> 4) & 7u);
+                const bool hasOut = ((st >> 7) & 1u) != 0u;
+                if (MODE == 1)
+                {
+                }
+                else if ((hasOut && (!BLEND || blendMode == SL_BLEND_OFF)) || (VIS && !hasOut))
+                {
+                    // an unblended fragment with outputs, and any whose visibility
+                    // record is wanted, waits until the pixel's colour is needed
+                    pend = rid;
+                    ps0 = f.y;
+                    ps1 = f.z;
+                    ps2 = f.w;
+                }
+                else if (BLEND && hasOut)
+                {
+                    // a blended fragment reads the colour: the pending one first,
+                    // those of all pixels together
+                    stall = pend != kNoPending;
+                    if (stall) continue;
+                    if (EARLY)
+                    {
+                        blend_into<CF>(&col8, &colF, blendMode, sCol[e], P.colorComps, P.colorPacked);
+                        if (VIS) vis = sVis[e];
+                    }
+                    else
+                    {
+                        shade_into(rid, f.y, f.z, f.w, blendMode);
+                    }
+                }
+                mine &= mine - 1ull;
+                if (((st >> 3) & 1u) != 0u) depth = P.depthHalf ? __half2float(__float2half_rn(f.x)) : f.x;
+                if (DBG)
+                {
+                    dbgLast = P.recs[rid].seq;
+                    dbgCount += 1u;
+                }
+                ++shaded;
+            }
+            if (!BLEND || __ballot(stall) == 0) break;
+            if (stall)
+            {
+                shade_into(pend, ps0, ps1, ps2, SL_BLEND_OFF);
                 pend = kNoPending;
             }
-            if (((st >> 3) & 1u) != 0u) depth = P.depthHalf ? __half2float(__float2half_rn(f.x)) : f.x;
-            if (DBG)
-            {
-                dbgLast = P.recs[rid].seq;
-                dbgCount += 1u;
-            }
-            ++shaded;
         }
         queued = 0;
         if (inb) bound = depth;

@@ -631,6 +631,7 @@ RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool have
     rp.extra = 0;
     rp.mrt = 0;
     rp.blend = 0;
+    rp.small = B.totalTris * kSmallTrianglePixels >= (uint64_t)p.W * p.H ? 1 : 0;
     for (const DrawDesc& d : B.draws)
     {
         rp.extra |= (d.prim != kPrimFill) ? 1 : 0;

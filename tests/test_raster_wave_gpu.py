@@ -9,6 +9,8 @@ per-pixel order and counts; colour within 1 LSB):
   queue        more than 64 waiting fragments of one record and of one pixel
   depth        the seven functions mixed in one batch, with depth-raising draws
                between LESS draws, into float and half depth, and with blending
+  small        batches on both sides of a triangle per 40 pixels, whose small
+               records queue their own fragments
 """
 import numpy as np
 import pytest
@@ -104,5 +106,41 @@ def test_bin_entries_of_large_records(gpu_lib, oracle_lib, tiles):
         xyz[:, 1:] = xyz[:, :1] + (xyz[:, 1:] * size).astype(np.float32)
         rec[:, 0:12] = xyz.astype(np.float32).reshape(-1, 3).view(np.uint8).reshape(-1, 12)
         return scenes.build_from_vertex_records(ctx, rec, W, H, True)
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
+
+
+@pytest.mark.parametrize("size,n", [((40, 10), 9), ((40, 10), 10), ((9, 7), 700), ((200, 40), 260), ((130, 70), 3000)])
+@pytest.mark.parametrize("debug", [False, True])
+@pytest.mark.parametrize("depth_type", [A.SL_COLOR_R_FLOAT, A.SL_COLOR_R_HALF])
+def test_small_triangles(gpu_lib, oracle_lib, size, n, debug, depth_type):
+    """Triangles of a pixel or three, every seventh over many columns and a run
+    of them piled on one pixel, opaque and blended draws in turn and one draw
+    that raises depths: batches of at least a triangle per 40 pixels (the
+    first case is just below) take the instances whose small records queue
+    their own fragments, lists with wide or raising records the wave's steps."""
+    def build(ctx):
+        rec = scenes.random_triangle_vertices(61, n).copy()
+        xyz = rec[:, 0:12].copy().view(np.float32).reshape(-1, 3, 3)
+        k = np.arange(n)
+        px = np.float32([2.0 / size[0], 2.0 / size[1], 1.0])
+        ext = np.where((k % 7 == 0)[:, None, None], np.float32([0.9, 0.1, 1.0]), 6.0 * px).astype(np.float32)
+        xyz[:, 1:] = xyz[:, :1] + xyz[:, 1:] * ext
+        xyz[n // 3:n // 2, :, :2] = xyz[n // 3, :, :2]          # a pile
+        if n >= 700:
+            xyz[k % 7 == 0, 1:] = xyz[k % 7 == 0, :1]           # and lists of small ones only
+            xyz[: n // 4: 7] = xyz[n // 4]
+        rec[:, 0:12] = xyz.astype(np.float32).reshape(-1, 3).view(np.uint8).reshape(-1, 12)
+        s = scenes.build_from_vertex_records(ctx, rec, size[0], size[1], debug, depth_type=depth_type)
+        vao = s.draws[0][1].vaoId
+        s.draws = []
+        step = 3 * (n // 6)
+        for d, (blend, test) in enumerate([(A.SL_BLEND_OFF, A.SL_DEPTH_TEST_LESS_THAN), (A.SL_BLEND_ALPHA, A.SL_DEPTH_TEST_LESS_EQUAL),
+                                           (A.SL_BLEND_OFF, A.SL_DEPTH_TEST_LESS_EQUAL), (A.SL_BLEND_ADDITIVE, A.SL_DEPTH_TEST_GREATER_THAN),
+                                           (A.SL_BLEND_ALPHA, A.SL_DEPTH_TEST_LESS_THAN), (A.SL_BLEND_OFF, A.SL_DEPTH_TEST_EQUAL)]):
+            sh = scenes.gouraud_shader(ctx, depth_test=test, blend=blend)
+            end = 3 * n if d == 5 else step * (d + 1)
+            s.draws.append(("draw_shader", A.sl_mesh(vao, step * d, end, A.RENDER_MODE_TRIANGLES, 0), sh))
+        return s
     g, o = render_both(gpu_lib, oracle_lib, build)
     assert_parity(g, o)
