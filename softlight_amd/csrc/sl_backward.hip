@@ -231,15 +231,17 @@ __global__ __launch_bounds__(256) void k_backward(BackwardParams P)
         const uint64_t t = (uint64_t)(seq - 1u - D.seqBase);
         live = seq > D.seqBase && t < D.numTris;
         if (!live) continue;
-        const uint64_t inst = (D.numTris == D.trisPerInstance) ? 0 : t / D.trisPerInstance;
-        const uint64_t ti = t - inst * D.trisPerInstance;
+        uint64_t ti;
+        const uint64_t inst = split_instance(D, t, ti);
         const uint64_t e = D.elementBegin + 3u * ti;
         vid[0] = e; vid[1] = e + 1; vid[2] = e + 2;
         if (D.indexed)
         {
-            vid[0] = fetch_index(D, e);
-            vid[1] = fetch_index(D, e + 1);
-            vid[2] = fetch_index(D, e + 2);
+            uint32_t id[3];
+            fetch_indices3(D, e, id);
+            vid[0] = id[0];
+            vid[1] = id[1];
+            vid[2] = id[2];
         }
         gradCol = G.gradCol;
         gradColCount = G.gradColCount;

@@ -125,8 +125,8 @@ __device__ __forceinline__ void load_varyings(const SetupParams& P, const DrawDe
 __device__ __forceinline__ void load_triangle_ids(uint64_t g, const DrawDesc& D, uint32_t di, TriIn& T)
 {
     const uint64_t t = g - D.triBase;
-    const uint64_t inst = t / D.trisPerInstance;
-    const uint64_t ti = t - inst * D.trisPerInstance;
+    uint64_t ti;
+    const uint64_t inst = split_instance(D, t, ti);
     // a point repeats its vertex in all three slots, a line its second
     const uint64_t per = verts_per_prim(D.prim);
     const uint64_t e = D.elementBegin + per * ti;
@@ -134,9 +134,15 @@ __device__ __forceinline__ void load_triangle_ids(uint64_t g, const DrawDesc& D,
     T.vid[0] = (uint32_t)e; T.vid[1] = (uint32_t)e1; T.vid[2] = (uint32_t)e2;
     if (D.indexed)
     {
-        T.vid[0] = (uint32_t)fetch_index(D, e);
-        T.vid[1] = (uint32_t)fetch_index(D, e1);
-        T.vid[2] = (uint32_t)fetch_index(D, e2);
+        if (per > 2)
+        {
+            fetch_indices3(D, e, T.vid);
+        }
+        else
+        {
+            T.vid[0] = (uint32_t)fetch_index(D, e);
+            T.vid[1] = T.vid[2] = (uint32_t)fetch_index(D, e1);
+        }
     }
     T.inst = (uint32_t)inst;
     T.draw = di;

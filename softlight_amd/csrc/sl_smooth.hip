@@ -125,15 +125,11 @@ __device__ __forceinline__ Shape winner_shape(const SmoothParams& P, uint32_t se
     if (seq <= D.seqBase) return S;
     const uint64_t t = (uint64_t)(seq - 1u - D.seqBase);
     if (t >= D.numTris) return S;
-    const uint64_t inst = t / D.trisPerInstance;
-    const uint64_t ti = t - inst * D.trisPerInstance;
+    uint64_t ti;
+    const uint64_t inst = split_instance(D, t, ti);
     const uint64_t e = D.elementBegin + 3u * ti;
     uint32_t vid[3] = {(uint32_t)e, (uint32_t)(e + 1), (uint32_t)(e + 2)};
-    if (D.indexed)
-    {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) vid[j] = (uint32_t)fetch_index(D, e + j);
-    }
+    if (D.indexed) fetch_indices3(D, e, vid);
     const bool all3[3] = {true, true, true};
     float4 pos[3];
     vertex_positions3(D, P.uniforms, vid, inst, all3, pos);
@@ -520,15 +516,11 @@ __device__ __forceinline__ uint32_t load_shapes(const SmoothParams& P, ShapeTile
         if (!mine || seq <= D.seqBase) continue;
         const uint64_t t = (uint64_t)(seq - 1u - D.seqBase);
         if (t >= D.numTris) continue;
-        const uint64_t inst = (D.numTris == D.trisPerInstance) ? 0 : t / D.trisPerInstance;
-        const uint64_t ti = t - inst * D.trisPerInstance;
+        uint64_t ti;
+        const uint64_t inst = split_instance(D, t, ti);
         const uint64_t e = D.elementBegin + 3u * ti;
         uint32_t vid[3] = {(uint32_t)e, (uint32_t)(e + 1), (uint32_t)(e + 2)};
-        if (D.indexed)
-        {
-#pragma unroll
-            for (int j = 0; j < 3; ++j) vid[j] = (uint32_t)fetch_index(D, e + j);
-        }
+        if (D.indexed) fetch_indices3(D, e, vid);
         const bool all3[3] = {true, true, true};
         float4 pos[3];
         vertex_positions3(D, P.uniforms, vid, inst, all3, pos);
