@@ -393,8 +393,8 @@ struct SetupParams
     PairJob* pairJobs;            // in the sorted list's storage (idle until the scatter): a job has more than kLanePairs entries
     ChunkInfo* chunkInfo;         // per chunk
     unsigned long long* stage;    // per chunk, kSetupBlock staging words
-    unsigned long long* blockAgg; // packed counts per kScanBlock chunks (summed by atomics)
-    uint32_t* blockSurv;          // survivors per kScanBlock chunks (summed by atomics)
+    unsigned long long* blockAgg; // packed counts per kScanBlock chunks
+    uint32_t* blockSurv;          // survivors per kScanBlock chunks
     uint32_t* survChunk;          // per survivor (in submission order): its chunk, written by the chunk scan
     uint32_t numChunks;
     FrameCtrl* ctrl;

@@ -10,7 +10,7 @@ hipError_t launch_vertex(const SetupParams& p, hipStream_t s);
 // Clears the control block before a frame, keeping (and adding the last
 // frame's overflow / error flags to) FrameCtrl::sticky, and na words of a and
 // nb of b.
-hipError_t launch_frame_reset(FrameCtrl* ctrl, uint32_t* a, uint32_t na, uint32_t* b, uint32_t nb, hipStream_t s);
+hipError_t launch_frame_reset(FrameCtrl* ctrl, uint32_t* a, uint32_t na, hipStream_t s);
 hipError_t launch_setup(const SetupParams& p, uint64_t chunks, hipStream_t s);
 hipError_t launch_chunk_scan(const SetupParams& p, hipStream_t s);
 // tris / prims: the batch holds triangle draws / point or line draws.

@@ -672,10 +672,9 @@ int enqueue_front(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, hip
     int rc;
     FrameCtrl* ctrl = reinterpret_cast<FrameCtrl*>(R.ctrl.p);
     uint32_t* ranges = reinterpret_cast<uint32_t*>(R.ranges.p);
-    if (B.totalTris == 0) return check(c, launch_frame_reset(ctrl, ranges, 2u * (uint32_t)p.numTiles, nullptr, 0u, s), "frame reset");
+    if (B.totalTris == 0) return check(c, launch_frame_reset(ctrl, ranges, 2u * (uint32_t)p.numTiles, s), "frame reset");
     const SetupParams sp = setup_params(p, B, R);
-    if ((rc = check(c, launch_frame_reset(ctrl, ranges, 2u * (uint32_t)p.numTiles, reinterpret_cast<uint32_t*>(sp.blockAgg),
-                                          (uint32_t)(3 * chunk_blocks(p.chunks)), s), "frame reset")) != SL_OK) return rc;
+    if ((rc = check(c, launch_frame_reset(ctrl, ranges, 2u * (uint32_t)p.numTiles, s), "frame reset")) != SL_OK) return rc;
     if ((rc = check(c, launch_vertex(sp, s), "k_vertex")) != SL_OK) return rc;
     if (evSetup0 && (rc = check(c, hipEventRecord(evSetup0, s), "event")) != SL_OK) return rc;
     if ((rc = check(c, launch_setup(sp, p.chunks, s), "k_setup")) != SL_OK) return rc;
