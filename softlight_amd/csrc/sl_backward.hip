@@ -1,6 +1,6 @@
 // sl_backward.hip -- fixed-visibility adjoint of the draw path.
 //
-// The forward pass (k_raster with a visibility attachment) leaves, for every
+// The forward pass (k_raster_wave with a visibility attachment) leaves, for every
 // pixel, the submitted-triangle number of the fragment that won the depth test
 // and that fragment's perspective-correct weights b0, b1, b2 of the source
 // triangle's vertices.  For an unclipped triangle the weights are bit-equal to

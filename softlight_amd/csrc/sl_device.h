@@ -43,10 +43,10 @@ constexpr TileConfig kTileConfigs[kNumTileConfigs] = {
 };
 constexpr int kDefaultTileConfig = 0;
 
-// Configuration 11's 64x64 tile keeps 4096 pixels' depth, colour and pending
-// fragments in LDS: 112 KB with an 8-bit colour target, more than the 160 KB a
-// workgroup may hold with an RGBA32F target or the visibility attachment, so
-// a batch with either is rasterised on configuration 7 (32x32) instead.
+// Configuration 11 (64x64) gives each 8x8 block a list four times as long as
+// 32x32 does; a batch with an RGBA32F target or the visibility attachment,
+// whose pixels hold more registers per wave, is rasterised on configuration 7
+// instead.
 constexpr int kLargeTileConfig = 11, kLargeTileFallback = 7;
 SL_HD constexpr int effective_tile_config(int cfg, bool floatColor, bool vis)
 {

@@ -42,9 +42,11 @@
 // (column pass, then row pass); a boundary's weight gets
 // dL/dw = <G(receiver), In(source) - In(receiver)> (In = C for the row pass,
 // X for the column pass), dL/dd = dL/dw * -sigma^2 / r^3, and d flows to the
-// screen positions of the edge's two vertices.  Every pixel recomputes the
-// boundaries it needs from the visibility attachment (the winner's triangle
-// is re-fetched and re-transformed), so nothing but the attachment is stored.
+// screen positions of the edge's two vertices.  The boundaries'
+// weights are worked out from the visibility attachment by a pass of their own
+// (k_smooth_bounds; the winners' triangles are fetched and transformed again,
+// once per 32 x 8 block) and stored, 8 B a pixel; the adjoint rebuilds its own
+// pixel's two for the edges' vertices.
 #include <algorithm>
 
 #include "sl_device.h"

@@ -57,3 +57,21 @@ def test_chunk_blocks(gpu_lib, oracle_lib, ntri):
         return scenes.build_from_vertex_records(ctx, rec, 320, 200, True)
     g, o = render_both(gpu_lib, oracle_lib, build)
     assert_parity(g, o)
+
+
+@pytest.mark.parametrize("tiles,n", [((1, 1), 1), ((1, 1), 65), ((1, 1), 257), ((2, 1), 64), ((3, 1), 63), ((8, 8), 5),
+                                     ((13, 5), 16), ((24, 20), 300)])
+def test_bin_entry_counts(gpu_lib, oracle_lib, tiles, n):
+    """n triangles that each reach every one of the 8x8 tiles: a power of two of
+    them and around it, entries below, at and past 64, a 256-entry block and
+    512 such blocks (144,000 entries, where a block's length grows)."""
+    def build(ctx):
+        ctx.set_raster_config(10)                               # 8x8 tiles
+        rec = scenes.random_triangle_vertices(79, n).copy()
+        xyz = rec[:, 0:12].copy().view(np.float32).reshape(-1, 3, 3)
+        xyz[:, :, :2] = [[-1.0, -1.0], [1.0, -1.0], [-1.0, 1.0]]
+        xyz[1::2, :, :2] *= -1.0
+        rec[:, 0:12] = xyz.reshape(-1, 3).view(np.uint8).reshape(-1, 12)
+        return scenes.build_from_vertex_records(ctx, rec, 8 * tiles[0], 8 * tiles[1], True)
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
