@@ -21,7 +21,6 @@
 #include <hip/hip_fp16.h>
 
 #include "sl_device.h"
-#include "sl_recurrence.h"
 #include "sl_stages.h"
 #include "sl_kernels.h"
 

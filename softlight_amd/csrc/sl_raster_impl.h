@@ -11,22 +11,11 @@
 #include <hip/hip_fp16.h>
 
 #include "sl_device.h"
-#include "sl_recurrence.h"
 #include "sl_stages.h"
 #include "sl_kernels.h"
 
 namespace slg {
 namespace {
-
-// Catch-up distances up to kStepLimit groups are stepped; longer ones use the
-// binade jump (one out-of-line copy for the three barycentric components).
-constexpr int kStepLimit = 256;
-
-__device__ __noinline__ float3 recur_advance3(float3 s, float3 d, int k)
-{
-    sl_recur_advance3(s.x, s.y, s.z, d.x, d.y, d.z, k);
-    return s;
-}
 
 // Greatest value over the wave's 64 lanes (every lane active): pairs and
 // quads with DPP quad permutes, the 16-lane row by rotating it 4 and 8 lanes,

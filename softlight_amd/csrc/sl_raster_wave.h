@@ -563,39 +563,35 @@ __global__ __launch_bounds__(256) void k_raster_wave(RasterParams P, int tileShi
                 int32_t xMin, xMax;
                 scanline_step(scan_edges(R), yf, xMin, xMax);
                 // bc(x) = fl(fl(x*dx) + fma(dy, y, c)) at the span's first pixel of
-                // this one's class mod 4, then += 4*dx per group of 4 pixels
+                // this one's class mod 4, then += 4*dx per group of 4 pixels, all
+                // of them stepped: the exact jump over whole binades
+                // (sl_recurrence.h) costs a fragment as much as thousands of
+                // steps (eight layers of two triangles each, back to front,
+                // 2.1 M pixels a target, raster kernel with jumps above 256
+                // steps and without: 1,920 columns 1,992 -> 308 us, 8,192
+                // 13,016 -> 956, 65,535 106,704 -> 6,697)
                 const int g = (ex - xMin) >> 2;
                 const float fx = (float)(ex - 4 * g);
                 s0 = (fx * R.bx[0]) + fmaf(R.by[0], yf, R.bz[0]);
                 s1 = (fx * R.bx[1]) + fmaf(R.by[1], yf, R.bz[1]);
                 s2 = (fx * R.bx[2]) + fmaf(R.by[2], yf, R.bz[2]);
                 const float d0 = R.bx[0] * 4.f, d1 = R.bx[1] * 4.f, d2 = R.bx[2] * 4.f;
-                if (g <= kStepLimit)
+                int k = 0;
+                for (; k + 4 <= g; k += 4)
                 {
-                    int k = 0;
-                    for (; k + 4 <= g; k += 4)
-                    {
 #pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                        {
-                            s0 = s0 + d0;
-                            s1 = s1 + d1;
-                            s2 = s2 + d2;
-                        }
-                    }
-                    for (; k < g; ++k)
+                    for (int u = 0; u < 4; ++u)
                     {
                         s0 = s0 + d0;
                         s1 = s1 + d1;
                         s2 = s2 + d2;
                     }
                 }
-                else
+                for (; k < g; ++k)
                 {
-                    const float3 a = recur_advance3(make_float3(s0, s1, s2), make_float3(d0, d1, d2), g);
-                    s0 = a.x;
-                    s1 = a.y;
-                    s2 = a.z;
+                    s0 = s0 + d0;
+                    s1 = s1 + d1;
+                    s2 = s2 + d2;
                 }
                 z = (((R.z[0] * s0) + (R.z[1] * s1)) + (R.z[2] * s2)) + R.bc3;
             }

@@ -1,6 +1,7 @@
-// sl_recurrence.h -- exact k-step advance of the barycentric recurrence
-// s <- fl(s + D) used by the scanline raster (SL_TriRasterizer.cpp:857-910:
-// bc += 4*dbc/dx per group of four pixels).
+// sl_recurrence.h -- exact k-step advance of the scanline raster's
+// barycentric recurrence s <- fl(s + D) (SL_TriRasterizer.cpp:857-910:
+// bc += 4*dbc/dx per group of four pixels).  The raster's kernels step
+// instead: one fragment's jump costs as much as thousands of steps there.
 //
 // Stepping k times costs k dependent adds.  Inside one binade of |s| (the
 // interval [2^e, 2^(e+1)) where float spacing is u = 2^(e-23)) every step adds

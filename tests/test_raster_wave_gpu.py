@@ -3,8 +3,9 @@ sizes where it can go wrong, against the CPU oracle bit for bit (depth,
 per-pixel order and counts; colour within 1 LSB):
 
   targets      smaller than a block, one pixel past it, ragged in both axes,
-               and wide enough (> 1,028 columns) that a fragment's barycentrics
-               are advanced by the exact jump instead of stepping
+               and wide: a fragment's barycentrics are stepped from its span's
+               first pixel, thousands of columns away at most, at the cost of
+               the steps and no more
   lists        63, 64, 65 and 129 records in a tile (64 are taken at a time)
   queue        more than 64 waiting fragments of one record and of one pixel
   depth        the seven functions mixed in one batch, with depth-raising draws
@@ -28,6 +29,48 @@ def test_target_sizes(gpu_lib, oracle_lib, size, blend):
     g, o = render_both(gpu_lib, oracle_lib, scenes.build_random_triangles, seed=21, ntri=150, W=size[0], H=size[1],
                        debug=True, blend=blend)
     assert_parity(g, o)
+
+
+def _layers(ctx, W, H, n=8, debug=False, blend=A.SL_BLEND_OFF):
+    """n pairs of triangles that cover the whole target, back to front: every
+    fragment passes."""
+    quad = np.float32([[-1, -1], [1, -1], [-1, 1], [-1, 1], [1, -1], [1, 1]])
+    xyz = np.empty((n, 6, 3), dtype=np.float32)
+    xyz[:, :, :2] = quad
+    xyz[:, :, 2] = np.linspace(0.8, -0.8, n, dtype=np.float32)[:, None]
+    rec = np.zeros((6 * n, 16), dtype=np.uint8)
+    rec[:, 0:12] = xyz.reshape(-1, 3).view(np.uint8).reshape(-1, 12)
+    rec[:, 12:16] = scenes.uniform_u8(17, 24 * n, stream=3).reshape(-1, 4)
+    return scenes.build_from_vertex_records(ctx, rec, W, H, debug, shader_kw=dict(blend=blend))
+
+
+@pytest.mark.parametrize("size", [(1031, 40), (4100, 9), (20000, 9)])
+@pytest.mark.parametrize("blend", [A.SL_BLEND_OFF, A.SL_BLEND_ALPHA])
+def test_layers_over_wide_targets(gpu_lib, oracle_lib, size, blend):
+    g, o = render_both(gpu_lib, oracle_lib, _layers, W=size[0], H=size[1], debug=True, blend=blend)
+    assert_parity(g, o)
+
+
+def test_wide_fragments_cost_their_steps(gpu_lib):
+    """Eight layers over 2 M pixels: at 3,840 columns a fragment takes up to 960
+    steps, at 480 up to 120.  That costs the raster about three times as much;
+    a jump over the steps, which fragments past some distance once took, cost
+    it 29 times as much."""
+    ms = {}
+    for W, H in ((480, 4320), (3840, 540)):
+        ctx = A.SLContext(gpu_lib)
+        s = _layers(ctx, W, H)
+        s.render()
+        ctx.finish()
+        best = []
+        for _ in range(5):
+            ctx.reset_stats()
+            s.render()
+            ctx.finish()
+            best.append(ctx.stats()["ms_raster"])
+        ms[W] = min(best)
+        ctx.close()
+    assert ms[3840] < 9.0 * ms[480], ms
 
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 129])
