@@ -490,9 +490,10 @@ uint32_t split_parts(const Plan& p)
 // The heavy-tile split applies to a batch whose draws merge exactly
 // (RasterParams::splitClass): all unblended, one depth function, a float
 // depth target, and depth writes on with a min- or max-type function or off.
-uint32_t split_class(const Batch& B, const Plan& p, bool all)
+// partRecs 0: the split is off.
+uint32_t split_class(const Batch& B, const Plan& p, bool all, uint32_t partRecs)
 {
-    if (B.draws.empty() || p.dt->type != SL_COLOR_R_FLOAT) return kSplitNone;
+    if (partRecs == 0 || B.draws.empty() || p.dt->type != SL_COLOR_R_FLOAT) return kSplitNone;
     // by default only batches with point or line draws, whose records pile
     // onto few tiles (a distant mesh's vertices); wireframe batches when
     // asked.  Batches of filled triangles never split: k_raster_wave's waves
@@ -589,7 +590,7 @@ SetupParams setup_params(const Plan& p, const Batch& B, FrameRes& R)
     return sp;
 }
 
-RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool haveEntries, bool splitAll)
+RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool haveEntries, bool splitAll, uint32_t splitRecs)
 {
     RasterParams rp{};
     rp.draws = reinterpret_cast<const DrawDesc*>(R.draws.p);
@@ -648,7 +649,7 @@ RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool have
     rp.splitDtest = 0;
     if (haveEntries && R.items.p != nullptr && R.maxParts > 0)
     {
-        const uint32_t cls = split_class(B, p, splitAll);
+        const uint32_t cls = split_class(B, p, splitAll, splitRecs);
         if (cls != kSplitNone)
         {
             rp.items = reinterpret_cast<const RasterItem*>(R.items.p);
@@ -706,7 +707,7 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
                  hipEvent_t evBin0, hipEvent_t evBin1)
 {
     int rc;
-    RasterParams rp = raster_params(p, B, R, B.totalTris > 0 && entries > 0, c->splitAll);
+    RasterParams rp = raster_params(p, B, R, B.totalTris > 0 && entries > 0, c->splitAll, c->splitRecs);
     rp.wgPerCU = c->wgPerCU;
     if (evBin0) (void)hipEventRecord(evBin0, s);
     if (B.totalTris > 0)
@@ -716,7 +717,7 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
         {
             // with the heavy-tile split on, the tile scan also writes the
             // raster's work items
-            const uint32_t partRecs = std::max<uint32_t>(c->splitRecs, 1u);
+            const uint32_t partRecs = std::max<uint32_t>(c->splitRecs, 1u);   // (0: no items, not read)
             if ((rc = check(c, launch_binning(sp.pairKeys, sp.pairVals, sp.ctrl, R.pairCap, entries,
                                               reinterpret_cast<uint32_t*>(R.binCounts.p), reinterpret_cast<uint32_t*>(R.binTotals.p),
                                               reinterpret_cast<uint2*>(R.ranges.p), reinterpret_cast<uint32_t*>(R.sorted.p),
@@ -731,7 +732,7 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
         // heavy tiles: the grids cover the most work items the entries can
         // make (a split tile of n records, n > kSplitAboveParts * partRecs, has
         // at most n / partRecs + 1 parts); the counts stay on the device
-        const uint64_t partRecs = std::max<uint32_t>(c->splitRecs, 1u);
+        const uint64_t partRecs = c->splitRecs;
         const int parts = (int)std::min<uint64_t>(R.maxParts, (uint64_t)entries * (kSplitAboveParts + 1) / (kSplitAboveParts * partRecs) + 1);
         return check(c, launch_raster(rp, p.numTiles + parts, parts, p.cfg, p.debug, s), "raster");
     }
@@ -993,7 +994,7 @@ int execute_batch(sl_context* c, bool staticScratch = false)
     // flags first), and is run again with larger ones.  A batch whose heavy
     // tiles may split, or without triangles, reads the entry count first: its
     // raster's grids are sized by it.
-    const bool whole = B.totalTris > 0 && (staticScratch || c->splitRecs == 0 || split_class(B, p, c->splitAll) == kSplitNone);
+    const bool whole = B.totalTris > 0 && (staticScratch || split_class(B, p, c->splitAll, c->splitRecs) == kSplitNone);
     for (int attempt = 0; attempt < 4; ++attempt)
     {
         if (staticScratch)

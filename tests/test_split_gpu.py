@@ -151,3 +151,19 @@ def test_split_graph_replay(gpu_lib, oracle_lib):
     assert np.array_equal(g["last"], o["last"])
     assert np.array_equal(g["count"], o["count"])
     assert int(np.abs(g["color"].astype(int) - o["color"].astype(int)).max()) <= 1
+
+
+def test_split_turned_off_after_a_split_frame(gpu_lib, oracle_lib):
+    """With the split off a batch of lines is not split, whatever the frame
+    before it was: that frame's work items and part buffers are sized for its
+    own tiles, and this one has more tiles, of another size."""
+    def build(ctx):
+        small = scenes.build_random_lines(ctx, seed=9, nlines=3000, W=64, H=48)
+        ctx.set_raster_split(4)
+        small.render()
+        ctx.finish()
+        ctx.set_raster_split(0)
+        ctx.set_raster_config(11)
+        return scenes.build_random_lines(ctx, seed=10, nlines=4000, W=900, H=500, debug=True)
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
