@@ -239,10 +239,10 @@ int         sl_set_raster_config(sl_context* ctx, int config);
  * with more than 4 * partRecords records is split into parts of about
  * partRecords records (at most 1024 parts) rasterised by separate workgroups
  * and merged exactly.  By default batches with point or line draws split
- * with parts of 256 records; sl_set_raster_split(n > 0) splits these and
- * wireframe batches with parts of n records, 0 turns the split off.  Batches
- * of filled triangles alone never split (their raster's work items are 8x8
- * pixel blocks).  Results never depend on it. */
+ * with parts of 256 records; sl_set_raster_split(n > 0) splits every such
+ * batch with parts of n records, 0 turns the split off.  A batch of filled
+ * triangles alone splits a tile only if it holds more than 1/32 of the
+ * frame's bin entries.  Results never depend on it. */
 int         sl_set_raster_split(sl_context* ctx, uint32_t partRecords);
 #define SL_RASTER_SPLIT_DEFAULT 0xFFFFFFFFu   /* sl_set_raster_split: back to the default policy */
 /* Occupancy (no counterpart in the reference): caps the raster workgroups

@@ -341,7 +341,7 @@ struct FrameCtrl
     // reported after later replays succeed
     uint32_t sticky;
     uint32_t pairJobs;         // records whose bin entries the clip kernel's waves write (PairJob)
-    uint32_t pad;
+    uint32_t splitParts;       // parts of the heavy-tile split's tiles
     // Fragment counters, spread over kCounterSlots cache lines (a workgroup
     // adds to slot blockIdx % kCounterSlots): tens of thousands of atomics on
     // one address serialise, on 64 lines they do not.  Readers sum the slots.
@@ -422,6 +422,16 @@ enum : uint32_t { kSplitNone = 0, kSplitMin = 1, kSplitMax = 2, kSplitConst = 3 
 constexpr uint32_t kDefaultSplitRecords = 256;  // records per part of a split tile
 constexpr uint32_t kSplitAboveParts = 4;        // tiles of more than kSplitAboveParts parts' records split
 constexpr uint32_t kMaxTileParts = 1024;        // parts of one split tile at most
+
+// A tile of filled triangles is split (where asked for) only with more than
+// 1 / kFilledShare of the frame's entries: the tiles of a frame of many heavy
+// ones fill the chip by themselves, and a part knows nothing of the depths
+// before it, so it works out fragments that the whole list's bounds reject.
+// Whole frames in us, unsplit and in parts of 256, of so many 32x16 tiles alike:
+// 4,000 triangles of a few pixels a tile, GREATER: 4 tiles 457 / 277, 32
+// 569 / 366, 64 583 / 472; LESS: 4 272 / 216, 32 308 / 261, 64 319 / 326; about
+// 2,000 of some 30 pixels, GREATER: 4 774 / 720, 16 588 / 751, 256 800 / 1,472.
+constexpr uint32_t kFilledShare = 32;
 
 // A batch with at least one triangle per this many pixels of the target takes
 // the raster's instances whose small records queue their own fragments: at

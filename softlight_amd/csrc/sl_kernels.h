@@ -30,12 +30,14 @@ __host__ __device__ inline uint32_t bin_per(uint32_t entries)
 }
 // With items non-null the tile scan also writes the raster's work items of
 // the heavy-tile split (see RasterItem): tiles of more than splitAbove
-// records cut into parts of about partRecs records, at most maxParts parts.
-hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const FrameCtrl* ctrl, uint32_t cap,
+// records cut into parts of about partRecs records, at most maxParts parts;
+// filled (a batch of filled triangles): the parts alone, split tiles' ranges
+// left empty, and tiles with little of the frame not split (kFilledShare).
+hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, FrameCtrl* ctrl, uint32_t cap,
                           uint32_t entries, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items = nullptr,
                           uint32_t* itemCount = nullptr, uint32_t partRecs = 1,
-                          uint32_t splitAbove = 0, uint32_t maxParts = 0);
+                          uint32_t splitAbove = 0, uint32_t maxParts = 0, bool filled = false);
 // The raster of a batch: units workgroup shares, one per tile or (with
 // p.items) the most work items there can be, maxParts of them parts.
 hipError_t launch_raster(const RasterParams& p, int units, int maxParts, int cfg, bool debug, hipStream_t s);

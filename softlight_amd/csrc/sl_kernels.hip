@@ -1683,14 +1683,20 @@ __device__ __forceinline__ void block_excl_scan2(uint32_t& a, uint32_t& b, uint3
 // splitAbove records is cut into ceil(records / partRecs) parts (at most kMaxTileParts)
 // of equal length while the maxParts part slots last (in tile order); the
 // parts come first, then every tile in launch order, a split tile's entry
-// marked as nothing to do (parts == 0).  One workgroup; each thread owns up
-// to kTilesPerThread consecutive tiles.
+// marked as nothing to do (parts == 0).  With `filled` (a batch of filled
+// triangles) there are no items but the parts, whose number goes to
+// FrameCtrl::splitParts, and a split tile's range is left empty: the launch
+// over tiles passes it by; and only a tile with more than 1 / kFilledShare of
+// all entries is split.  One workgroup; each thread owns up to kTilesPerThread
+// consecutive tiles.
 constexpr int kTilesPerThread = 16;   // 16384 tiles at most
 struct SplitPlan
 {
     RasterItem* items;         // null: no work items
     uint32_t* itemCount;
     uint32_t partRecs, splitAbove, maxParts;
+    FrameCtrl* ctrl;
+    bool filled;
 };
 
 __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restrict__ totals, uint2* __restrict__ range,
@@ -1705,8 +1711,10 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
     uint32_t tot[kTilesPerThread];
 #pragma unroll
     for (int j = 0; j < kTilesPerThread; ++j) tot[j] = (j < per && t0 + j < numTiles) ? totals[t0 + j] : 0u;
+    uint32_t above = SP.splitAbove;
+    if (SP.items != nullptr && SP.filled) above = max(above, SP.ctrl->totalPairs / kFilledShare);
     auto wanted = [&](uint32_t n) -> uint32_t {
-        return (n > SP.splitAbove) ? min((n + SP.partRecs - 1u) / SP.partRecs, kMaxTileParts) : 1u;
+        return (n > above) ? min((n + SP.partRecs - 1u) / SP.partRecs, kMaxTileParts) : 1u;
     };
     uint32_t se = 0, sw = 0;
 #pragma unroll
@@ -1776,6 +1784,7 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
             if (j < per && t0 + j < numTiles && ((splitMask >> j) & 1u))
             {
                 const uint32_t n = tot[j], p = wanted(n);
+                if (SP.filled) range[t0 + j] = make_uint2(rb, rb);
                 for (uint32_t k = 0; k < p; ++k)
                 {
                     RasterItem it;
@@ -1814,8 +1823,9 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
     {
         if (SP.items != nullptr)
         {
-            SP.itemCount[0] = nParts + (uint32_t)numTiles;
+            SP.itemCount[0] = nParts + (SP.filled ? 0u : (uint32_t)numTiles);
             SP.itemCount[1] = nParts;
+            SP.ctrl->splitParts = nParts;
         }
     }
     __syncthreads();
@@ -1827,7 +1837,7 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
         {
             const uint32_t pos = atomicAdd(&sBucket[32 - __clz((int)tot[j])], 1u);
             order[pos] = (uint32_t)(t0 + j);
-            if (SP.items != nullptr)
+            if (SP.items != nullptr && !SP.filled)
             {
                 RasterItem it;
                 it.tile = (uint32_t)(t0 + j);
@@ -2071,12 +2081,12 @@ hipError_t launch_blit(const BlitParams& p, int srcType, int dstType, hipStream_
     return hipGetLastError();
 }
 
-hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, const FrameCtrl* ctrl, uint32_t cap,
+hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, FrameCtrl* ctrl, uint32_t cap,
                           uint32_t entries, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items, uint32_t* itemCount,
-                          uint32_t partRecs, uint32_t splitAbove, uint32_t maxParts)
+                          uint32_t partRecs, uint32_t splitAbove, uint32_t maxParts, bool filled)
 {
-    SplitPlan sp{items, itemCount, partRecs, splitAbove, maxParts};
+    SplitPlan sp{items, itemCount, partRecs, splitAbove, maxParts, ctrl, filled};
     (void)hipGetLastError();   // drop a stale error from an earlier call
     const size_t lds = sizeof(uint32_t) * (size_t)numTiles;
     const uint32_t blocks = std::min(kMaxBinBlocks, std::max(1u, (entries + kMinBinBlock - 1) / kMinBinBlock));
@@ -2102,8 +2112,9 @@ hipError_t launch_raster(const RasterParams& p, int units, int maxParts, int cfg
     int aux = (debug ? 1 : 0) | (p.vis != nullptr ? 2 : 0) | (p.extra ? 4 : 0) | (p.mrt ? 8 : 0);
     if (cf != 0 && (p.blend || debug || (p.mrt && p.extra))) aux |= 32;
     if (p.small && !p.extra) aux |= 64;
-    // visibility is built for RGBA32F colour, filled triangles and single
-    // outputs; several outputs need colour attachment 0
+    // visibility is built for RGBA32F colour, filled triangles (and the parts of
+    // their split tiles) and single outputs; several outputs need colour
+    // attachment 0
     switch (cf << 8 | aux)
     {
 #define SL_RASTER(CF, AUX) case CF << 8 | AUX: launch_raster_wave_cfg<CF, AUX>(p, units, maxParts, shx, shy, s); break
@@ -2112,6 +2123,7 @@ hipError_t launch_raster(const RasterParams& p, int units, int maxParts, int cfg
         SL_RASTER(2, 2); SL_RASTER(2, 34); SL_RASTER(2, 35);
         SL_RASTER(0, 4); SL_RASTER(1, 4); SL_RASTER(2, 4); SL_RASTER(1, 36); SL_RASTER(2, 36);
         SL_RASTER(0, 5); SL_RASTER(1, 37); SL_RASTER(2, 37);
+        SL_RASTER(2, 6); SL_RASTER(2, 39);
         SL_RASTER(1, 8); SL_RASTER(2, 8); SL_RASTER(1, 40); SL_RASTER(2, 40); SL_RASTER(1, 41); SL_RASTER(2, 41);
         SL_RASTER(1, 44); SL_RASTER(2, 44); SL_RASTER(1, 45); SL_RASTER(2, 45);
         SL_RASTER(0, 64); SL_RASTER(1, 64); SL_RASTER(2, 64); SL_RASTER(1, 96); SL_RASTER(2, 96);

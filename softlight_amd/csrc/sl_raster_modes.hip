@@ -8,5 +8,6 @@ template void launch_raster_wave_cfg<1, 4>(const RasterParams&, int, int, int, i
 template void launch_raster_wave_cfg<2, 4>(const RasterParams&, int, int, int, int, hipStream_t);
 template void launch_raster_wave_cfg<1, 36>(const RasterParams&, int, int, int, int, hipStream_t);
 template void launch_raster_wave_cfg<2, 36>(const RasterParams&, int, int, int, int, hipStream_t);
+template void launch_raster_wave_cfg<2, 6>(const RasterParams&, int, int, int, int, hipStream_t);
 
 }  // namespace slg

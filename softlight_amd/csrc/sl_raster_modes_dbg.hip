@@ -8,5 +8,6 @@ template void launch_raster_wave_cfg<1, 37>(const RasterParams&, int, int, int, 
 template void launch_raster_wave_cfg<2, 37>(const RasterParams&, int, int, int, int, hipStream_t);
 template void launch_raster_wave_cfg<1, 45>(const RasterParams&, int, int, int, int, hipStream_t);
 template void launch_raster_wave_cfg<2, 45>(const RasterParams&, int, int, int, int, hipStream_t);
+template void launch_raster_wave_cfg<2, 39>(const RasterParams&, int, int, int, int, hipStream_t);
 
 }  // namespace slg

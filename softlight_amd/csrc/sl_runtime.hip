@@ -268,7 +268,7 @@ struct sl_context
     unsigned numThreads = 1;
     int tileConfig = kDefaultTileConfig;
     uint32_t splitRecs = kDefaultSplitRecords;   // heavy-tile split: records per part (0: off)
-    bool splitAll = false;                       // split triangle-only batches too (sl_set_raster_split)
+    bool splitAll = false;                       // split triangle batches too, filled and wireframe (sl_set_raster_split)
     uint32_t wgPerCU = 0;                        // raster occupancy cap (sl_set_raster_occupancy; 0: none)
     uint32_t triSeq = 0;
     sl_frame_stats stats{};
@@ -495,16 +495,12 @@ uint32_t split_class(const Batch& B, const Plan& p, bool all, uint32_t partRecs)
 {
     if (partRecs == 0 || B.draws.empty() || p.dt->type != SL_COLOR_R_FLOAT) return kSplitNone;
     // by default only batches with point or line draws, whose records pile
-    // onto few tiles (a distant mesh's vertices); wireframe batches when
-    // asked.  Batches of filled triangles never split: k_raster_wave's waves
-    // are 8x8 blocks and it drops hidden records 64 at a time
-    bool prims = false, wire = false;
-    for (const DrawDesc& d : B.draws)
-    {
-        prims = prims || d.prim == kPrimPoint || d.prim == kPrimLine;
-        wire = wire || d.prim == kPrimWire;
-    }
-    if (!prims && !(all && wire)) return kSplitNone;
+    // onto few tiles (a distant mesh's vertices); triangle batches when asked
+    bool prims = false;
+    for (const DrawDesc& d : B.draws) prims = prims || d.prim == kPrimPoint || d.prim == kPrimLine;
+    if (!all && !prims) return kSplitNone;
+    // no tile can be heavy: a triangle yields at most kMaxFan records
+    if (B.totalTris * kMaxFan <= (uint64_t)kSplitAboveParts * partRecs) return kSplitNone;
     const DrawDesc& d0 = B.draws[0];
     for (const DrawDesc& d : B.draws)
         if (d.blend != SL_BLEND_OFF || d.dtest != d0.dtest || d.dmask != d0.dmask) return kSplitNone;
@@ -700,11 +696,21 @@ int enqueue_front(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, hip
     return SL_OK;
 }
 
+// The parts of a filled batch's split tiles, whose pixels the launch over the
+// tiles left as they were before the batch (or cleared): the instance with
+// work items takes them.
+int enqueue_parts(sl_context* c, const Plan& p, RasterParams rp, int parts, hipStream_t s)
+{
+    rp.extra = 1;
+    return check(c, launch_raster(rp, parts, parts, p.cfg, p.debug, s), "raster of split tiles");
+}
+
 // Binning and raster.  entries bounds the bin entries and sizes the grids (the
 // capacity, where the count has not been read back; the kernels read the
-// actual counts from the control block).
+// actual counts from the control block).  A filled batch's parts of split
+// tiles are left to enqueue_parts unless `withParts`.
 int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint32_t entries, hipStream_t s,
-                 hipEvent_t evBin0, hipEvent_t evBin1)
+                 hipEvent_t evBin0, hipEvent_t evBin1, bool withParts)
 {
     int rc;
     RasterParams rp = raster_params(p, B, R, B.totalTris > 0 && entries > 0, c->splitAll, c->splitRecs);
@@ -723,7 +729,7 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
                                               reinterpret_cast<uint2*>(R.ranges.p), reinterpret_cast<uint32_t*>(R.sorted.p),
                                               reinterpret_cast<uint32_t*>(R.order.p), p.numTiles, s,
                                               const_cast<RasterItem*>(rp.items), const_cast<uint32_t*>(rp.itemCount),
-                                              partRecs, kSplitAboveParts * partRecs, R.maxParts), "binning")) != SL_OK) return rc;
+                                              partRecs, kSplitAboveParts * partRecs, R.maxParts, rp.extra == 0), "binning")) != SL_OK) return rc;
         }
     }
     if (evBin1) (void)hipEventRecord(evBin1, s);
@@ -734,7 +740,11 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
         // at most n / partRecs + 1 parts); the counts stay on the device
         const uint64_t partRecs = c->splitRecs;
         const int parts = (int)std::min<uint64_t>(R.maxParts, (uint64_t)entries * (kSplitAboveParts + 1) / (kSplitAboveParts * partRecs) + 1);
-        return check(c, launch_raster(rp, p.numTiles + parts, parts, p.cfg, p.debug, s), "raster");
+        if (rp.extra) return check(c, launch_raster(rp, p.numTiles + parts, parts, p.cfg, p.debug, s), "raster");
+        RasterParams tiles = rp;
+        tiles.items = nullptr;
+        if ((rc = check(c, launch_raster(tiles, p.numTiles, 0, p.cfg, p.debug, s), "raster")) != SL_OK) return rc;
+        return withParts ? enqueue_parts(c, p, rp, parts, s) : SL_OK;
     }
     return check(c, launch_raster(rp, p.numTiles, 0, p.cfg, p.debug, s), "raster");
 }
@@ -991,10 +1001,12 @@ int execute_batch(sl_context* c, bool staticScratch = false)
 
     // The whole frame is queued at once and its flags are read after it: a
     // frame that outgrew its buffers touches no pixel (the raster reads the
-    // flags first), and is run again with larger ones.  A batch whose heavy
-    // tiles may split, or without triangles, reads the entry count first: its
-    // raster's grids are sized by it.
-    const bool whole = B.totalTris > 0 && (staticScratch || split_class(B, p, c->splitAll, c->splitRecs) == kSplitNone);
+    // flags first), and is run again with larger ones.  A batch of wireframe
+    // triangles, lines or points whose heavy tiles may split, or one without
+    // triangles, reads the entry count first: its raster's grids are sized by it.
+    bool filled = true;
+    for (const DrawDesc& d : B.draws) filled = filled && d.prim == kPrimFill;
+    const bool whole = B.totalTris > 0 && (staticScratch || filled || split_class(B, p, c->splitAll, c->splitRecs) == kSplitNone);
     for (int attempt = 0; attempt < 4; ++attempt)
     {
         if (staticScratch)
@@ -1022,7 +1034,7 @@ int execute_batch(sl_context* c, bool staticScratch = false)
         c->stats.setup_launches += 1;
         if (whole)
         {
-            if ((rc = enqueue_back(c, R, p, B, R.pairCap, s, c->ev[10], c->ev[4])) != SL_OK) return rc;
+            if ((rc = enqueue_back(c, R, p, B, R.pairCap, s, c->ev[10], c->ev[4], false)) != SL_OK) return rc;
             (void)hipEventRecord(c->ev[5], s);
         }
         if ((rc = check(c, hipMemcpyAsync(c->hCtrl, ctrl, sizeof(FrameCtrl), hipMemcpyDeviceToHost, s), "read ctrl")) != SL_OK) return rc;
@@ -1059,9 +1071,18 @@ int execute_batch(sl_context* c, bool staticScratch = false)
         totalPairs = c->hCtrl->totalPairs;
         jobs = c->hCtrl->clipJobs;
     }
-    if (!whole)
+    const bool split = whole && c->hCtrl->splitParts > 0;
+    if (!whole || split)
     {
-        if ((rc = enqueue_back(c, R, p, B, totalPairs, s, c->ev[10], c->ev[4])) != SL_OK) return rc;
+        // a filled batch's split tiles are drawn once the frame has shown that
+        // it has any: four launches that find nothing to do cost the others
+        // 18 us a frame
+        if (split)
+        {
+            const RasterParams rp = raster_params(p, B, R, true, c->splitAll, c->splitRecs);
+            if ((rc = enqueue_parts(c, p, rp, (int)c->hCtrl->splitParts, s)) != SL_OK) return rc;
+        }
+        else if ((rc = enqueue_back(c, R, p, B, totalPairs, s, c->ev[10], c->ev[4], true)) != SL_OK) return rc;
         (void)hipEventRecord(c->ev[5], s);
         if ((rc = check(c, hipMemcpyAsync(c->hCtrl, ctrl, sizeof(FrameCtrl), hipMemcpyDeviceToHost, s), "read ctrl")) != SL_OK) return rc;
         if ((rc = check(c, hipStreamSynchronize(s), "frame sync")) != SL_OK) return rc;
@@ -1156,7 +1177,7 @@ int graph_capture(sl_context* c)
         if ((rc = check(c, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "begin capture")) != SL_OK) { graph_release(c); return rc; }
         int rc1 = timed ? enqueue_front(c, G.res, p, B, s, c->gEv[0], c->gEv[1]) : enqueue_front(c, G.res, p, B, s);
         int rc2 = (rc1 == SL_OK) ? enqueue_back(c, G.res, p, B, G.res.pairCap, s, nullptr,
-                                                timed ? c->gEv[2] : nullptr) : rc1;
+                                                timed ? c->gEv[2] : nullptr, true) : rc1;
         if (rc2 == SL_OK && timed) rc2 = check(c, hipEventRecord(c->gEv[3], s), "event");
         int rc3 = (rc2 == SL_OK) ? check(c, hipMemcpyAsync(G.hCtrl, G.res.ctrl.p, sizeof(FrameCtrl), hipMemcpyDeviceToHost, s), "read ctrl") : rc2;
         hipGraph_t graph = nullptr;

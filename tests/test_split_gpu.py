@@ -167,3 +167,98 @@ def test_split_turned_off_after_a_split_frame(gpu_lib, oracle_lib):
         return scenes.build_random_lines(ctx, seed=10, nlines=4000, W=900, H=500, debug=True)
     g, o = render_both(gpu_lib, oracle_lib, build)
     assert_parity(g, o)
+
+
+def _pile(ctx, n=2500, W=64, H=48, dtest=A.SL_DEPTH_TEST_LESS_THAN, dmask=A.SL_DEPTH_MASK_ON, debug=True, color=True):
+    """n filled triangles of a few pixels piled on one tile, a tenth of them
+    repeated (ties), one in eight over the whole target."""
+    rec = scenes.random_triangle_vertices(71, n).copy()
+    xyz = rec[:, 0:12].copy().view(np.float32).reshape(-1, 3, 3)
+    k = np.arange(n)
+    xyz[k % 8 != 0, :, :2] = np.float32([-0.4, 0.3]) + 0.15 * xyz[k % 8 != 0, :, :2]
+    xyz[n // 2: n // 2 + n // 10] = xyz[: n // 10]
+    rec[:, 0:12] = xyz.reshape(-1, 3).view(np.uint8).reshape(-1, 12)
+    s = scenes.build_from_vertex_records(ctx, rec, W, H, debug, shader_kw=dict(depth_test=dtest, depth_mask=dmask))
+    if dtest in (A.SL_DEPTH_TEST_GREATER_THAN, A.SL_DEPTH_TEST_GREATER_EQUAL):
+        s.clear_depth = -1.0
+    return s
+
+
+@pytest.mark.parametrize("part", [1, 7, 100])
+@pytest.mark.parametrize("dtest,dmask", [
+    (A.SL_DEPTH_TEST_LESS_THAN, A.SL_DEPTH_MASK_ON), (A.SL_DEPTH_TEST_LESS_EQUAL, A.SL_DEPTH_MASK_ON),
+    (A.SL_DEPTH_TEST_GREATER_THAN, A.SL_DEPTH_MASK_ON), (A.SL_DEPTH_TEST_GREATER_EQUAL, A.SL_DEPTH_MASK_ON),
+    (A.SL_DEPTH_TEST_NOT_EQUAL, A.SL_DEPTH_MASK_OFF)], ids=["less", "lequal", "greater", "gequal", "nomask"])
+@pytest.mark.parametrize("debug", [True, False])
+def test_split_pile_of_filled_triangles(gpu_lib, oracle_lib, dtest, dmask, part, debug):
+    """One tile of 2,500 filled triangles among four: with and without the
+    debug buffers, drawn twice (the second time onto the first's depths)."""
+    def build(ctx):
+        s = _pile(ctx, dtest=dtest, dmask=dmask, debug=debug)
+        s.draws = s.draws * 2
+        return s
+    g, o = render_both(gpu_lib, oracle_lib, _with_split(build, part))
+    assert_parity(g, o)
+    def again(ctx):
+        s = _pile(ctx, dtest=dtest, dmask=dmask, debug=debug)
+        s.render()
+        ctx.finish()
+        render = s.render
+        s.render = lambda clear=False: render(clear=False)
+        return s
+    g, o = render_both(gpu_lib, oracle_lib, _with_split(again, part))
+    assert_parity(g, o)
+
+
+def test_split_pile_costs_less(gpu_lib):
+    """20,000 small triangles on one tile with a depth-raising test, whose
+    fragments nothing rejects: one wave per 8x8 block walks them all, parts of
+    256 share them out."""
+    ms = {}
+    for part in (0, 256):
+        ctx = A.SLContext(gpu_lib)
+        ctx.set_raster_split(part)
+        s = _pile(ctx, n=20_000, W=1280, H=720, dtest=A.SL_DEPTH_TEST_GREATER_THAN, debug=False)
+        vbo = np.asarray(scenes.random_triangle_vertices(72, 20_000)).copy()
+        xyz = vbo[:, 0:12].copy().view(np.float32)
+        xyz[:, 0:2] *= np.float32([0.012, 0.011])
+        vbo[:, 0:12] = xyz.view(np.uint8).reshape(-1, 12)
+        ctx.vbo_assign(0, vbo)
+        s.render()
+        ctx.finish()
+        best = []
+        for _ in range(5):
+            ctx.reset_stats()
+            s.render()
+            ctx.finish()
+            best.append(ctx.stats()["ms_raster"])
+        ms[part] = min(best)
+        ctx.close()
+    assert ms[256] < 0.7 * ms[0], ms
+
+
+@pytest.mark.parametrize("part", [2, 9])
+def test_split_filled_visibility_and_outputs(gpu_lib, oracle_lib, part):
+    """Two tiles: the visibility record (with the gradients it leads to) and the
+    four outputs of a G-buffer come out of the merge as from one list."""
+    from tests.test_mrt import FMTS, draw, gbuffer_scene
+    outs = []
+    for lib in (oracle_lib, gpu_lib):
+        ctx = A.SLContext(lib)
+        ctx.set_raster_split(part)
+        s = scenes.DiffScene(ctx, level=3, views=1, size=32, views_per_fbo=1, tex_size=16)
+        s.make_targets()
+        s.forward(); s.loss_grad_images(); s.backward()
+        sc = gbuffer_scene(ctx, 32, 32, FMTS, depth_type=A.SL_COLOR_R_FLOAT)
+        outs.append((s.visibility(), s.gradients(), draw(ctx, sc), ctx.texture_read(sc["depth"])))
+    (vo, go, (co, no), do), (vg, gg, (cg, ng), dg) = outs
+    np.testing.assert_array_equal(vo[0].view(np.uint32), vg[0].view(np.uint32))
+    assert (vo[0].view(np.uint32)[..., 0] != 0).sum() > 100
+    for ref, got in zip(go, gg):
+        assert float(np.abs(ref).max()) > 0
+        assert float(np.abs(ref - got).max()) <= 1e-4 * float(np.abs(ref).max())
+    np.testing.assert_array_equal(no, ng)
+    np.testing.assert_array_equal(do.view(np.uint32), dg.view(np.uint32))
+    assert no.sum() > 100
+    for a, b in zip(co, cg):
+        assert int(np.abs(a.astype(int) - b.astype(int)).max()) <= 1
