@@ -17,15 +17,16 @@ hipError_t launch_chunk_scan(const SetupParams& p, hipStream_t s);
 hipError_t launch_emit(const SetupParams& p, bool tris, bool prims, hipStream_t s);
 // The clip jobs, and the bin entries of records that cover many tiles.
 hipError_t launch_clip(const SetupParams& p, hipStream_t s);
-// Binning splits the entries into at most kMaxBinBlocks blocks of `per`
-// entries (a multiple of 64, at least kMinBinBlock).
+// Binning splits the entries into at most `rows` (kMaxBinBlocks where the
+// count matrix has room for them) blocks of `per` entries (a multiple of 64, at
+// least kMinBinBlock).
 constexpr uint32_t kMaxBinBlocks = 512;
 constexpr uint32_t kMinBinBlock = 256;   // (1,024: a frame of 1,000 .. 3,000 entries spent 13 us in a few waves of the scatter, now 5)
 // The kernels work out `per` from the device's entry count, so a launch needs
 // only an upper bound of the entries (blocks past the count end at once).
-__host__ __device__ inline uint32_t bin_per(uint32_t entries)
+__host__ __device__ inline uint32_t bin_per(uint32_t entries, uint32_t rows)
 {
-    const uint32_t per = (entries / kMaxBinBlocks + (entries % kMaxBinBlocks ? 1u : 0u) + 63u) / 64u * 64u;
+    const uint32_t per = (entries / rows + (entries % rows ? 1u : 0u) + 63u) / 64u * 64u;
     return per > kMinBinBlock ? per : kMinBinBlock;
 }
 // With items non-null the tile scan also writes the raster's work items of
@@ -34,7 +35,7 @@ __host__ __device__ inline uint32_t bin_per(uint32_t entries)
 // filled (a batch of filled triangles): the parts alone, split tiles' ranges
 // left empty, and tiles with little of the frame not split (kFilledShare).
 hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, FrameCtrl* ctrl, uint32_t cap,
-                          uint32_t entries, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
+                          uint32_t entries, uint32_t rows, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items = nullptr,
                           uint32_t* itemCount = nullptr, uint32_t partRecs = 1,
                           uint32_t splitAbove = 0, uint32_t maxParts = 0, bool filled = false);

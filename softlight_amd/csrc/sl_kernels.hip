@@ -1592,10 +1592,10 @@ __device__ __forceinline__ uint32_t bin_entries(const FrameCtrl* ctrl, uint32_t 
 
 // Block b of the binning kernels owns entries [b*per, (b+1)*per).
 __global__ __launch_bounds__(256) void k_bin_count(const uint32_t* __restrict__ keys, const FrameCtrl* __restrict__ ctrl,
-                                                   uint32_t cap, uint32_t* __restrict__ counts, int numTiles)
+                                                   uint32_t cap, uint32_t rows, uint32_t* __restrict__ counts, int numTiles)
 {
     extern __shared__ uint32_t sCnt[];
-    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n);
+    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n, rows);
     const uint32_t start = blockIdx.x * per;
     if (start >= n) return;
     const uint32_t end = min(start + per, n);
@@ -1618,14 +1618,14 @@ __global__ __launch_bounds__(256) void k_bin_count(const uint32_t* __restrict__ 
 constexpr int kColTiles = 32, kColParts = 32, kColRows = (int)kMaxBinBlocks / kColParts;
 static_assert(kMaxBinBlocks % kColParts == 0, "a part's rows");
 
-__global__ __launch_bounds__(kColTiles * kColParts) void k_bin_colscan(const FrameCtrl* __restrict__ ctrl, uint32_t cap,
+__global__ __launch_bounds__(kColTiles * kColParts) void k_bin_colscan(const FrameCtrl* __restrict__ ctrl, uint32_t cap, uint32_t binRows,
                                                                       uint32_t* __restrict__ counts, uint32_t* __restrict__ totals,
                                                                       int numTiles)
 {
     __shared__ uint32_t sPart[kColParts][kColTiles];
     const int tl = threadIdx.x % kColTiles, part = threadIdx.x / kColTiles;
     const int t = blockIdx.x * kColTiles + tl;
-    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n);
+    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n, binRows);
     const uint32_t blocks = (n + per - 1) / per;
     const uint32_t rpp = (blocks + kColParts - 1) / kColParts;   // kColRows at most
     const uint32_t r0 = min(blocks, part * rpp), rows = (t < numTiles) ? min(blocks - r0, rpp) : 0u;
@@ -1856,12 +1856,12 @@ __global__ __launch_bounds__(1024) void k_bin_tilescan(const uint32_t* __restric
 }
 
 __global__ __launch_bounds__(64) void k_bin_scatter(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                    const FrameCtrl* __restrict__ ctrl, uint32_t cap,
+                                                    const FrameCtrl* __restrict__ ctrl, uint32_t cap, uint32_t rows,
                                                     const uint32_t* __restrict__ counts, const uint2* __restrict__ range,
                                                     uint32_t* __restrict__ out, int numTiles)
 {
     extern __shared__ uint32_t sBase[];
-    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n);
+    const uint32_t n = bin_entries(ctrl, cap), per = bin_per(n, rows);
     const uint32_t start = blockIdx.x * per;
     if (start >= n) return;
     const uint32_t end = min(start + per, n);
@@ -2082,20 +2082,20 @@ hipError_t launch_blit(const BlitParams& p, int srcType, int dstType, hipStream_
 }
 
 hipError_t launch_binning(const uint32_t* keys, const uint32_t* vals, FrameCtrl* ctrl, uint32_t cap,
-                          uint32_t entries, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
+                          uint32_t entries, uint32_t rows, uint32_t* counts, uint32_t* totals, uint2* range, uint32_t* out,
                           uint32_t* order, int numTiles, hipStream_t s, RasterItem* items, uint32_t* itemCount,
                           uint32_t partRecs, uint32_t splitAbove, uint32_t maxParts, bool filled)
 {
     SplitPlan sp{items, itemCount, partRecs, splitAbove, maxParts, ctrl, filled};
     (void)hipGetLastError();   // drop a stale error from an earlier call
     const size_t lds = sizeof(uint32_t) * (size_t)numTiles;
-    const uint32_t blocks = std::min(kMaxBinBlocks, std::max(1u, (entries + kMinBinBlock - 1) / kMinBinBlock));
-    hipLaunchKernelGGL(k_bin_count, dim3(blocks), dim3(256), lds, s, keys, ctrl, cap, counts, numTiles);
+    const uint32_t blocks = std::min(rows, std::max(1u, entries / kMinBinBlock + (entries % kMinBinBlock ? 1u : 0u)));
+    hipLaunchKernelGGL(k_bin_count, dim3(blocks), dim3(256), lds, s, keys, ctrl, cap, rows, counts, numTiles);
     hipLaunchKernelGGL(k_bin_colscan, dim3((numTiles + kColTiles - 1) / kColTiles), dim3(kColTiles * kColParts), 0, s,
-                       ctrl, cap, counts, totals, numTiles);
+                       ctrl, cap, rows, counts, totals, numTiles);
     if (numTiles > 1024 * kTilesPerThread) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_bin_tilescan, dim3(1), dim3(1024), 0, s, totals, range, order, numTiles, sp);
-    hipLaunchKernelGGL(k_bin_scatter, dim3(blocks), dim3(64), lds, s, keys, vals, ctrl, cap, counts, range, out,
+    hipLaunchKernelGGL(k_bin_scatter, dim3(blocks), dim3(64), lds, s, keys, vals, ctrl, cap, rows, counts, range, out,
                        numTiles);
     return hipGetLastError();
 }

@@ -93,6 +93,7 @@ struct FrameRes
     // snapshots, the vertex pass's work table
     DevBuf draws, recs, vars, keys, vals, sorted, clip, status, ranges, ctrl, binCounts, binTotals, order;
     uint32_t recCap = 0, pairCap = 0, clipCap = 0;
+    uint32_t binRows = kMaxBinBlocks;   // rows of binCounts
     // heavy-tile split: work items, their counts, per part slot the first
     // pass's depths and the part results, per split tile and pixel the last
     // part with a pending fragment (absent: no split)
@@ -724,7 +725,7 @@ int enqueue_back(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, uint
             // with the heavy-tile split on, the tile scan also writes the
             // raster's work items
             const uint32_t partRecs = std::max<uint32_t>(c->splitRecs, 1u);   // (0: no items, not read)
-            if ((rc = check(c, launch_binning(sp.pairKeys, sp.pairVals, sp.ctrl, R.pairCap, entries,
+            if ((rc = check(c, launch_binning(sp.pairKeys, sp.pairVals, sp.ctrl, R.pairCap, entries, R.binRows,
                                               reinterpret_cast<uint32_t*>(R.binCounts.p), reinterpret_cast<uint32_t*>(R.binTotals.p),
                                               reinterpret_cast<uint2*>(R.ranges.p), reinterpret_cast<uint32_t*>(R.sorted.p),
                                               reinterpret_cast<uint32_t*>(R.order.p), p.numTiles, s,
@@ -904,8 +905,11 @@ int static_scratch(sl_context* c, uint8_t** out)
 
 size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
 
-// Bin count matrix rows for up to `pairs` entries (bin_plan never uses more).
-uint64_t bin_rows(uint64_t pairs) { return std::min<uint64_t>(kMaxBinBlocks, std::max<uint64_t>(1, (pairs + kMinBinBlock - 1) / kMinBinBlock)); }
+// Bin count matrix rows for up to `pairs` entries: one per 1,024, which leaves
+// the array to the records (one per kMinBinBlock would take up to four times as
+// much: 33 MB of the 64 at 16,200 tiles from 131k entries on).  Frames of fewer
+// entries than the rows are for still bin in blocks of kMinBinBlock.
+uint64_t bin_rows(uint64_t pairs) { return std::min<uint64_t>(kMaxBinBlocks, std::max<uint64_t>(1, (pairs + 1023) / 1024)); }
 
 // Bytes of the fixed part: control block, tile ranges and order, draw table,
 // uniform arena, setup chunk buffer, tile totals.
@@ -951,6 +955,7 @@ int bind_static(sl_context* c, uint8_t* base, FrameRes& R, const Plan& p, const 
     R.recCap = (uint32_t)recs;
     R.pairCap = (uint32_t)pairs;
     R.clipCap = (uint32_t)clips;
+    R.binRows = (uint32_t)bin_rows(pairs);
     return SL_OK;
 }
 

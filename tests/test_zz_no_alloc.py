@@ -86,3 +86,25 @@ def test_static_draw_refuses_frames_beyond_the_array(gpu_lib):
     small = A.sl_mesh(mesh.vaoId, 0, 3000, mesh.mode, 0)
     ctx.draw_static(small, s.shader, s.fbo)
     ctx.close()
+
+
+@pytest.mark.parametrize("config,n", [(3, 170_000), (2, 235_000), (0, 268_000)])
+def test_static_draw_holds_large_frames_of_small_tiles(gpu_lib, config, n):
+    """Small triangles at 1080p on 16x8, 16x16 and 32x16 tiles, whose bin counts
+    take a row of 16,200, 8,160 and 4,080 tiles per 1,024 entries of the array:
+    frames near the largest that fit it draw as sl_draw draws them."""
+    from tests.test_capacity_gpu import small_triangles
+    outs = []
+    for static in (False, True):
+        ctx = A.SLContext(gpu_lib)
+        ctx.set_raster_config(config)
+        s = small_triangles(ctx, n=n, W=1920, H=1080)
+        ctx.clear_framebuffer(s.fbo, 0, s.clear_rgba, s.clear_depth)
+        (ctx.draw_static if static else ctx.draw)(s.draws[0][1], s.shader, s.fbo)
+        out = s.read()
+        st = ctx.stats()
+        out["stats"] = {k: st[k] for k in STATS}
+        outs.append(out)
+        ctx.close()
+    assert outs[0]["stats"]["triangles_binned"] > 0.9 * n
+    _same(*outs)
