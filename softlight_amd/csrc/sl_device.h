@@ -554,7 +554,7 @@ struct SmoothParams
     // between rows y and y + 1 with its sign bit set when row y receives; NaN
     // where there is no boundary
     float2* bounds;
-    uint32_t* clippedTiles;    // per block of the boundary pass: it holds a clipped winner
+    uint32_t* clippedRows;     // per row of the boundary pass's blocks: its pixels that a clipped winner bounds
 };
 
 struct BackwardParams

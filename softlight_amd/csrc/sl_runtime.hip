@@ -288,7 +288,7 @@ struct sl_context
     hipEvent_t bwdEv[2] = {};                      // first / last backward since the last collection
     hipEvent_t gEv[4] = {};                        // graph replays: setup start/end, raster start/end
     uint64_t bwdPending = 0;
-    DevBuf smoothBounds;                           // the smoothing passes' per-pixel boundary weights (float2) and clipped blocks
+    DevBuf smoothBounds;                           // the smoothing passes' per-pixel boundary weights (float2) and clipped pixels
     uint64_t visCounter = 0;                       // generations of visibility recordings
 };
 
@@ -2263,9 +2263,9 @@ int smooth_setup(sl_context* c, size_t fbo, size_t srcTex, size_t dstTex, float 
     if (sp.sigma > 0.f)
     {
         const size_t pixels = (size_t)vis->w * vis->h;
-        if ((rc = ensure(c, c->smoothBounds, sizeof(float2) * pixels + sizeof(uint32_t) * smooth_tiles(vis->w, vis->h))) != SL_OK) return rc;
+        if ((rc = ensure(c, c->smoothBounds, sizeof(float2) * pixels + sizeof(uint32_t) * smooth_rows(vis->w, vis->h))) != SL_OK) return rc;
         sp.bounds = reinterpret_cast<float2*>(c->smoothBounds.p);
-        sp.clippedTiles = reinterpret_cast<uint32_t*>(sp.bounds + pixels);
+        sp.clippedRows = reinterpret_cast<uint32_t*>(sp.bounds + pixels);
     }
     return SL_OK;
 }

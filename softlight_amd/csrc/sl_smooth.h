@@ -6,8 +6,8 @@
 namespace slg {
 
 // Each launcher runs the boundary pass first (p.bounds: W * H float2;
-// p.clippedTiles: smooth_tiles(W, H) words).
-size_t smooth_tiles(int W, int H);
+// p.clippedRows: smooth_rows(W, H) words).
+size_t smooth_rows(int W, int H);
 hipError_t launch_smooth(const SmoothParams& p, hipStream_t s);
 hipError_t launch_smooth_backward(const SmoothParams& p, hipStream_t s);
 

@@ -435,15 +435,19 @@ __device__ __forceinline__ float4 add_scaled_diff(float4 o, float w, float4 a, f
 // fetched and transformed once; a boundary used to fetch its two by itself,
 // which made up to four a pixel, each a chain of a search over the draws,
 // indices, attributes and matrices (a wave takes its draws one after the
-// other, so that these come through scalar registers).  Blocks with a clipped
-// winner are marked and left to launches of their own (k_smooth_bounds_clipped,
-// k_smooth_scatter_clipped), whose pixels fetch their winners themselves: the
-// polygons' registers and scratch would cost these kernels their occupancy.
+// other, so that these come through scalar registers).  Pixels with a clipped
+// winner on a boundary are marked and left to launches of their own
+// (k_smooth_bounds_clipped, k_smooth_scatter_clipped), which fetch their winners
+// themselves: the polygons' registers and scratch would cost these kernels
+// their occupancy.
 // Measured per 2048x1024 framebuffer (eight views of eight spheres, triangles
 // of a pixel or two, so nearly every pixel is a boundary): boundary pass 142 ->
 // 107 us and 5 for the clipped launch, adjoint 267 -> 185 and 4 (half its gain
 // from add_position's pairing; the rest of it is position atomics and the
-// latency of the winners' fetches).
+// latency of the winners' fetches).  Where the frustum cuts many triangles
+// (eight views from among four spheres) the clipped launches take most of the
+// time: 1,258 us a pass with a fetch per boundary, 1,331 with whole blocks left
+// to them, up to eight a workgroup, now 1,128 (1,235 without marks by pixel).
 // ---------------------------------------------------------------------------
 constexpr int kShapeW = 32, kShapeH = 8;
 constexpr int kShapeCols = kShapeW + 1, kShapeEntries = kShapeCols * (kShapeH + 1);
@@ -478,7 +482,7 @@ __device__ __forceinline__ SVert tile_vert(const SmoothParams& P, const ShapeTil
 
 // Fills T for the block at (x0, y0); every thread of the workgroup calls it.
 // What it holds (the same for all of them): kShapeNone where no two
-// neighbours' winners differ, kShapeClipped where one that bounds another is
+// neighbours' winners differ, kShapeClipped where some that bounds another is
 // clipped.
 __device__ __forceinline__ uint32_t load_shapes(const SmoothParams& P, ShapeTile& T, int x0, int y0)
 {
@@ -530,6 +534,7 @@ __device__ __forceinline__ uint32_t load_shapes(const SmoothParams& P, ShapeTile
         for (int j = 0; j < 3; ++j) pos[j] = mat_mul(D.scissor, pos[j]);
         const int status = clip_status(pos[0], pos[1], pos[2]);
         clipped = status == 1;
+        if (clipped) T.kind[i] = kShapeClipped;
         if (status != 3) continue;
         T.kind[i] = kShapeTri;
         T.draw[i] = cur;
@@ -543,6 +548,14 @@ __device__ __forceinline__ uint32_t load_shapes(const SmoothParams& P, ShapeTile
         }
     }
     return __syncthreads_or(clipped) ? kShapeClipped : kShapeTri;
+}
+
+// A clipped winner bounds the pixel of tile entry i, to its left or below it.
+__device__ __forceinline__ bool tile_clipped(const SmoothParams& P, const ShapeTile& T, int i, int x, int y)
+{
+    const bool here = T.kind[i] == kShapeClipped;
+    return (x > 0 && T.seq[i - 1] != T.seq[i] && (here || T.kind[i - 1] == kShapeClipped)) ||
+           (y + 1 < P.H && T.seq[i] != T.seq[i + kShapeCols] && (here || T.kind[i + kShapeCols] == kShapeClipped));
 }
 
 // boundary_x / boundary_y of the pixel of tile entry i, its winners from the tile.
@@ -611,14 +624,24 @@ __device__ __forceinline__ bool tile_pixel(const SmoothParams& P, int& x0, int& 
 __global__ __launch_bounds__(kShapeThreads) void k_smooth_bounds(SmoothParams P)
 {
     __shared__ ShapeTile T;
+    __shared__ uint32_t sLeft[kShapeH];
     int x0, y0, x, y, e;
     const bool mine = tile_pixel(P, x0, y0, x, y, e);
     const uint32_t kind = load_shapes(P, T, x0, y0);
-    if (threadIdx.x == 0) P.clippedTiles[blockIdx.x] = kind == kShapeClipped ? 1u : 0u;
-    if (!mine || kind == kShapeClipped) return;
+    bool left = false;
+    if (kind == kShapeClipped)
+    {
+        left = mine && tile_clipped(P, T, e, x, y);
+        if (threadIdx.x < kShapeH) sLeft[threadIdx.x] = 0u;
+        __syncthreads();
+        if (left) atomicOr(&sLeft[y - y0], 1u << (x - x0));
+        __syncthreads();
+    }
+    if (threadIdx.x < kShapeH) P.clippedRows[kShapeH * blockIdx.x + threadIdx.x] = kind == kShapeClipped ? sLeft[threadIdx.x] : 0u;
+    if (!mine || left) return;
     const float none = __builtin_nanf("");
     float wx = none, wy = none;
-    if (kind == kShapeTri)
+    if (kind != kShapeNone)
     {
         const Bnd Bx = tile_boundary_x(P, T, e, x, y);
         if (Bx.ok) wx = bnd_weight(Bx, P.sigma);
@@ -632,27 +655,30 @@ __global__ __launch_bounds__(kShapeThreads) void k_smooth_bounds(SmoothParams P)
     P.bounds[(uint64_t)y * P.W + x] = make_float2(wx, wy);
 }
 
-// The boundaries of the blocks marked as holding clipped winners, one block a
-// workgroup at a time.
+// Block b's pixel of this lane (a workgroup of kShapeW x kShapeH) was marked.
+__device__ __forceinline__ bool left_to_clipped(const SmoothParams& P, int b)
+{
+    static_assert(kShapeW == 32, "a word per row");
+    return ((P.clippedRows[kShapeH * b + (int)threadIdx.x / kShapeW] >> (threadIdx.x % kShapeW)) & 1u) != 0u;
+}
+
+// The boundaries of the pixels marked as bounded by clipped winners, a lane per
+// pixel of the block.
 __global__ __launch_bounds__(kShapeW * kShapeH) void k_smooth_bounds_clipped(SmoothParams P)
 {
-    const int bxN = (P.W + kShapeW - 1) / kShapeW, n = bxN * ((P.H + kShapeH - 1) / kShapeH);
-    for (int b = (int)blockIdx.x; b < n; b += (int)gridDim.x)
+    const int bxN = (P.W + kShapeW - 1) / kShapeW, b = (int)blockIdx.x;
+    if (!left_to_clipped(P, b)) return;
+    const int x = (b % bxN) * kShapeW + (int)threadIdx.x % kShapeW, y = (b / bxN) * kShapeH + (int)threadIdx.x / kShapeW;
+    const Bnd Bx = boundary_x(P, x, y);
+    const Bnd By = boundary_y(P, x, y);
+    const float wx = Bx.ok ? bnd_weight(Bx, P.sigma) : __builtin_nanf("");
+    float wy = __builtin_nanf("");
+    if (By.ok)
     {
-        if (P.clippedTiles[b] == 0u) continue;
-        const int x = (b % bxN) * kShapeW + (int)threadIdx.x % kShapeW, y = (b / bxN) * kShapeH + (int)threadIdx.x / kShapeW;
-        if (x >= P.W || y >= P.H) continue;
-        const Bnd Bx = boundary_x(P, x, y);
-        const Bnd By = boundary_y(P, x, y);
-        const float wx = Bx.ok ? bnd_weight(Bx, P.sigma) : __builtin_nanf("");
-        float wy = __builtin_nanf("");
-        if (By.ok)
-        {
-            const float w = bnd_weight(By, P.sigma);
-            wy = By.recvLow ? -w : w;
-        }
-        P.bounds[(uint64_t)y * P.W + x] = make_float2(wx, wy);
+        const float w = bnd_weight(By, P.sigma);
+        wy = By.recvLow ? -w : w;
     }
+    P.bounds[(uint64_t)y * P.W + x] = make_float2(wx, wy);
 }
 
 // A stored boundary: present, its weight and (column pass) whether row y receives.
@@ -802,7 +828,7 @@ __global__ __launch_bounds__(kShapeThreads) void k_smooth_backward(SmoothParams 
         if (mine) P.out[i] = P.grad[i];
         return;
     }
-    const bool shapes = P.posGrad != nullptr && P.clippedTiles[blockIdx.x] == 0u && load_shapes(P, T, x0, y0) == kShapeTri;
+    const bool shapes = P.posGrad != nullptr && load_shapes(P, T, x0, y0) != kShapeNone;
     float4 gx = make_float4(0.f, 0.f, 0.f, 0.f);
     StoredBnd Sx{false, false, 0.f};
     if (mine)
@@ -822,9 +848,10 @@ __global__ __launch_bounds__(kShapeThreads) void k_smooth_backward(SmoothParams 
     if (!shapes) return;
     // this pixel's row-pass boundary (x - 1 | x) and the column-pass
     // boundary (y | y + 1), rebuilt for their edges' vertices
+    const bool here = mine && !tile_clipped(P, T, e, x, y);
     Bnd B = no_bnd();
     float d = 0.f;
-    if (mine && Sx.ok)
+    if (here && Sx.ok)
     {
         B = tile_boundary_x(P, T, e, x, y);
         d = dL_dd(B, P.sigma, row_dLdw(P, i, gx));
@@ -832,7 +859,7 @@ __global__ __launch_bounds__(kShapeThreads) void k_smooth_backward(SmoothParams 
     scatter_position(P, B, d, true);
     B = no_bnd();
     d = 0.f;
-    if (mine && stored_y(P, i).ok)
+    if (here && stored_y(P, i).ok)
     {
         B = tile_boundary_y(P, T, e, x, y);
         d = dL_dd(B, P.sigma, col_dLdw(P, i, x, y, B.recvLow));
@@ -840,33 +867,30 @@ __global__ __launch_bounds__(kShapeThreads) void k_smooth_backward(SmoothParams 
     scatter_position(P, B, d, false);
 }
 
-// The position gradients of the blocks with clipped winners.
+// The position gradients of the pixels bounded by clipped winners.
 __global__ __launch_bounds__(kShapeW * kShapeH) void k_smooth_scatter_clipped(SmoothParams P)
 {
-    const int bxN = (P.W + kShapeW - 1) / kShapeW, n = bxN * ((P.H + kShapeH - 1) / kShapeH);
-    for (int b = (int)blockIdx.x; b < n; b += (int)gridDim.x)
+    const int bxN = (P.W + kShapeW - 1) / kShapeW, b = (int)blockIdx.x;
+    const bool mine = left_to_clipped(P, b);
+    if (__ballot(mine) == 0) return;
+    const int x = (b % bxN) * kShapeW + (int)threadIdx.x % kShapeW, y = (b / bxN) * kShapeH + (int)threadIdx.x / kShapeW;
+    const uint64_t i = mine ? (uint64_t)y * P.W + x : 0;
+    Bnd B = no_bnd();
+    float d = 0.f;
+    if (mine && stored_x(P, i).ok)
     {
-        if (P.clippedTiles[b] == 0u) continue;
-        const int x = (b % bxN) * kShapeW + (int)threadIdx.x % kShapeW, y = (b / bxN) * kShapeH + (int)threadIdx.x / kShapeW;
-        const bool mine = x < P.W && y < P.H;
-        const uint64_t i = mine ? (uint64_t)y * P.W + x : 0;
-        Bnd B = no_bnd();
-        float d = 0.f;
-        if (mine && stored_x(P, i).ok)
-        {
-            B = boundary_x(P, x, y);
-            d = dL_dd(B, P.sigma, row_dLdw(P, i, grad_x_image(P, x, y)));
-        }
-        scatter_position(P, B, d, true);
-        B = no_bnd();
-        d = 0.f;
-        if (mine && stored_y(P, i).ok)
-        {
-            B = boundary_y(P, x, y);
-            d = dL_dd(B, P.sigma, col_dLdw(P, i, x, y, B.recvLow));
-        }
-        scatter_position(P, B, d, false);
+        B = boundary_x(P, x, y);
+        d = dL_dd(B, P.sigma, row_dLdw(P, i, grad_x_image(P, x, y)));
     }
+    scatter_position(P, B, d, true);
+    B = no_bnd();
+    d = 0.f;
+    if (mine && stored_y(P, i).ok)
+    {
+        B = boundary_y(P, x, y);
+        d = dL_dd(B, P.sigma, col_dLdw(P, i, x, y, B.recvLow));
+    }
+    scatter_position(P, B, d, false);
 }
 
 static unsigned tile_grid(const SmoothParams& p)
@@ -881,13 +905,10 @@ static unsigned smooth_grid(const SmoothParams& p)
     return (unsigned)(g > 65536 ? 65536 : (g == 0 ? 1 : g));
 }
 
-// Blocks of the clipped launches: they look through the marks of all blocks.
-static unsigned clipped_grid(const SmoothParams& p) { return std::min(tile_grid(p), 1024u); }
-
 static void launch_bounds(const SmoothParams& p, hipStream_t s)
 {
     hipLaunchKernelGGL(k_smooth_bounds, dim3(tile_grid(p)), dim3(kShapeThreads), 0, s, p);
-    hipLaunchKernelGGL(k_smooth_bounds_clipped, dim3(clipped_grid(p)), dim3(kShapeW * kShapeH), 0, s, p);
+    hipLaunchKernelGGL(k_smooth_bounds_clipped, dim3(tile_grid(p)), dim3(kShapeW * kShapeH), 0, s, p);
 }
 
 hipError_t launch_smooth(const SmoothParams& p, hipStream_t s)
@@ -906,13 +927,13 @@ hipError_t launch_smooth_backward(const SmoothParams& p, hipStream_t s)
     if (p.sigma > 0.f) launch_bounds(p, s);
     hipLaunchKernelGGL(k_smooth_backward, dim3(tile_grid(p)), dim3(kShapeThreads), 0, s, p);
     if (p.sigma > 0.f && p.posGrad != nullptr)
-        hipLaunchKernelGGL(k_smooth_scatter_clipped, dim3(clipped_grid(p)), dim3(kShapeW * kShapeH), 0, s, p);
+        hipLaunchKernelGGL(k_smooth_scatter_clipped, dim3(tile_grid(p)), dim3(kShapeW * kShapeH), 0, s, p);
     return hipGetLastError();
 }
 
-size_t smooth_tiles(int W, int H)
+size_t smooth_rows(int W, int H)
 {
-    return (size_t)((W + kShapeW - 1) / kShapeW) * (size_t)((H + kShapeH - 1) / kShapeH);
+    return (size_t)((W + kShapeW - 1) / kShapeW) * (size_t)((H + kShapeH - 1) / kShapeH) * kShapeH;
 }
 
 }  // namespace slg

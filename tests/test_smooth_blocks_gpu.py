@@ -1,8 +1,8 @@
 """The smoothing passes' blocks (32x8 pixels and their halo) at the sizes
 where they can go wrong, against the oracle: framebuffers of one block, one
-pixel past it and ragged, with winners clipped by the frustum in some blocks
-(left to launches of their own) and not in others, and more draws than are
-searched in LDS.  Tolerances as the suite's batched smoothing check: 1e-5 for
+pixel past it and ragged, with winners clipped by the frustum bounding some
+pixels of a block (left to launches of their own) and not others, and more
+draws than are searched in LDS.  Tolerances as the suite's batched smoothing check: 1e-5 for
 images, 1e-4 of the largest for gradients."""
 import numpy as np
 import pytest
@@ -33,6 +33,7 @@ def _run(lib, sigma, kw):
     dict(meshes=3, views=1, size=32, views_per_fbo=1),
     dict(meshes=4, views=2, size=33, views_per_fbo=1),
     dict(meshes=8, views=9, size=41, views_per_fbo=9),
+    dict(meshes=4, views=4, size=100, views_per_fbo=4),
 ])
 def test_blocks_match_oracle(gpu_lib, oracle_lib, kw, distance):
     kw = dict(kw, min_tris=60, max_tris=400, tex_size=16, distance=distance)
