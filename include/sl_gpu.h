@@ -226,9 +226,10 @@ int         sl_set_scissor(sl_context* ctx, int32_t x, int32_t y, int32_t w, int
 
 /* Raster tile configuration (no counterpart in the reference, whose raster
  * splits scanlines across CPU threads, SL_ScanlineBounds.hpp:31-50).
- * Configurations 0..11 select the screen tile each GPU workgroup owns (8x8
- * to 64x64) and how many column segments a tile row is split into; see
- * sl_get_raster_config.  Configuration 11 (64x64) falls back to 7 (32x32)
+ * Configurations 0..11 select the screen tile that primitives are binned to
+ * (8x8 to 64x64); configurations that sl_get_raster_config reports with the
+ * same tile are alike, whatever their column segments (which the raster no
+ * longer uses).  Configuration 11 (64x64) falls back to 7 (32x32)
  * for a batch with an RGBA32F colour target or a visibility attachment.
  * sl_get_raster_config(ctx, -1, ...) reports the current one and returns its
  * index; results do not depend on the configuration. */

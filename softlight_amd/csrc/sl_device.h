@@ -21,32 +21,34 @@ namespace slg {
 constexpr int kSetupBlock = 256;       // triangles per setup workgroup (one per lane)
 constexpr int kMaxFan = 7;             // a 9-gon from 6-plane clipping fans into 7 triangles
 
-// Tile raster configurations.  A workgroup owns one tileW x tileH screen
-// tile; lane = (row, column segment, x-phase): each lane walks the pixels
-// x = xMin + phase + 4k of its row that fall in its segment of tileW/segs
-// columns (the reference steps its barycentrics in groups of 4 pixels).
+// Tile raster configurations: the screen tile that a record list is built for.
+// Its pixels are rasterised in 8x8 blocks, a wave each, four waves a workgroup
+// (fewer where a tile has fewer blocks).  `segs`, the column segments of a row,
+// plays no part in that: configurations that differ in it alone are the same
+// launch, kept so that the indices and what sl_get_raster_config reports stay.
 struct TileConfig { int tileW, tileH, segs; };
 constexpr int kNumTileConfigs = 12;
 constexpr TileConfig kTileConfigs[kNumTileConfigs] = {
-    {32, 16, 1},   // 0: 1 wave
-    {32, 8, 2},    // 1: 1 wave
-    {16, 16, 1},   // 2: 1 wave
-    {16, 8, 2},    // 3: 1 wave
-    {16, 8, 4},    // 4: 2 waves x 4 rows
-    {16, 16, 4},   // 5: 4 waves x 4 rows
-    {32, 16, 4},   // 6: 4 waves x 4 rows
-    {32, 32, 2},   // 7: 4 waves x 8 rows
-    {32, 8, 4},    // 8: 2 waves x 4 rows
-    {32, 8, 8},    // 9: 4 waves x 2 rows
+    {32, 16, 1},   // 0: 8 waves
+    {32, 8, 2},    // 1: 4 waves
+    {16, 16, 1},   // 2: 4 waves
+    {16, 8, 2},    // 3: 2 waves
+    {16, 8, 4},    // 4: as 3
+    {16, 16, 4},   // 5: as 2
+    {32, 16, 4},   // 6: as 0
+    {32, 32, 2},   // 7: 16 waves
+    {32, 8, 4},    // 8: as 1
+    {32, 8, 8},    // 9: as 1
     {8, 8, 2},     // 10: 1 wave
-    {64, 64, 1},   // 11: 4 waves x 16 rows
+    {64, 64, 1},   // 11: 64 waves
 };
 constexpr int kDefaultTileConfig = 0;
 
-// Configuration 11 (64x64) gives each 8x8 block a list four times as long as
-// 32x32 does; a batch with an RGBA32F target or the visibility attachment,
-// whose pixels hold more registers per wave, is rasterised on configuration 7
-// instead.
+// A batch with an RGBA32F target or the visibility attachment is rasterised on
+// configuration 7 (32x32) instead of 11 (64x64), whose lists are four times as
+// long for every 8x8 block: raster kernel on 7 / 11 of 64 spheres at 1080p 54 /
+// 103 us, of 8 views of 512x512 46 / 64, of 4,096 overlapping triangles at
+// 640x480 122 / 127.
 constexpr int kLargeTileConfig = 11, kLargeTileFallback = 7;
 SL_HD constexpr int effective_tile_config(int cfg, bool floatColor, bool vis)
 {
@@ -433,11 +435,15 @@ constexpr uint32_t kMaxTileParts = 1024;        // parts of one split tile at mo
 // 2,000 of some 30 pixels, GREATER: 4 774 / 720, 16 588 / 751, 256 800 / 1,472.
 constexpr uint32_t kFilledShare = 32;
 
-// A batch with at least one triangle per this many pixels of the target takes
-// the raster's instances whose small records queue their own fragments: at
-// 5 .. 26 pixels a triangle (sphere and mesh scenes) these take the raster from
-// 65 to 34 us, 120 to 72 and 313 to 246; at 48 .. 400 (overlapping triangles of a
-// tenth of the target) their extra registers cost it 8 - 12% (116 -> 125 us).
+// A batch with at least one submitted triangle per this many pixels of the
+// target takes the raster's instances whose small records queue their own
+// fragments: at 5 .. 26 pixels a triangle (sphere and mesh scenes) these take the
+// raster from 70 to 40 us, 120 to 72 and 350 to 318; at 48 .. 400 (overlapping
+// triangles of a tenth of the target) their extra registers cost it 9 - 16% (118
+// -> 130 us, blended 86 -> 99).  The host knows the triangles' number and not
+// their size: culled ones beside large ones and many layers count as small, at
+// that cost (16 layers of 16-pixel triangles 368 -> 415 us, blended 552 -> 665; of
+// 4-pixel ones 968 -> 609 and 1,233 -> 952).
 constexpr uint64_t kSmallTrianglePixels = 40;
 
 // One raster workgroup's work: a whole tile (parts == 1) or part `part` of
