@@ -47,7 +47,8 @@ def test_gradients_match_oracle(gpu_lib, oracle_lib, kw):
 
 def test_several_meshes_in_a_block(gpu_lib, oracle_lib):
     """Eight overlapping spheres, each with a colour gradient of its own, in
-    views of 48x48 pixels: most blocks hold several destination buffers."""
+    views of 48x48 pixels: most blocks hold several destination buffers (all
+    eight meshes and the texture get gradients)."""
     outs = []
     for lib in (gpu_lib, oracle_lib):
         ctx = A.SLContext(lib)
@@ -59,4 +60,5 @@ def test_several_meshes_in_a_block(gpu_lib, oracle_lib):
         outs.append([ctx.vbo_read(g, sc.pos[m].shape[0] * 16, dtype=np.float32) for m, g in enumerate(sc.grad_vbos)] +
                     [ctx.texture_read(sc.grad_tex)])
     for got, ref in zip(*outs):
+        assert float(np.abs(ref).max()) > 0.0
         assert float(np.abs(ref - got).max()) <= 1e-4 * float(np.abs(ref).max())

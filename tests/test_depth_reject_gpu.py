@@ -1,17 +1,18 @@
-"""Depth rejection (sl_set_raster_depth_reject): a wave of a tile with 64 or
-more records skips the filled triangles whose depth provably fails a LESS /
-LESS_EQUAL test at every pixel it owns, and only counts their depth tests.
-With it on, coverage, depth, per-pixel primitive order and the
-tested/shaded/binned counts equal the oracle's exactly and equal the
-output with it off: on random triangles (every tile ~2,300 records), on
-every tile configuration, with depth-raising draws (GREATER, test off with
-writes) between LESS draws of one batch, with heavy-tile splitting, blended
-batches and R16F depth (where the variant rejects nothing)."""
+"""Depth rejection: the raster drops the filled triangles whose depth provably
+fails a LESS / LESS_EQUAL test at every pixel of an 8x8 block, and only counts
+their depth tests.  Coverage, depth, per-pixel primitive order and the
+tested/shaded/binned counts equal the oracle's exactly: on random triangles
+(every tile ~1,200 records), on every tile configuration, with depth-raising
+draws (GREATER, test off with writes) between LESS draws of one batch, with
+heavy tiles split, in blended batches, with R16F depth and for triangles whose
+planes are not finite.  sl_set_raster_depth_reject chooses nothing: it is set
+here both ways and the output must be the same."""
 import numpy as np
 import pytest
 
 from softlight_amd import api as A
 from softlight_amd import scenes
+from tests.geometry import build_screen_triangles
 from tests.parity import assert_parity, render_both
 
 pytestmark = pytest.mark.gpu
@@ -112,6 +113,59 @@ def test_depth_raising_draws_in_one_batch(gpu_lib, oracle_lib):
 
 @pytest.mark.parametrize("part", [3, 64])
 def test_with_heavy_tile_split(gpu_lib, oracle_lib, part):
+    """Twelve tiles of some 500 records each."""
     g, o = render_both(gpu_lib, oracle_lib, _reject(scenes.build_random_triangles, split=part), seed=6, ntri=1500,
-                       W=200, H=150, debug=True)
+                       W=96, H=64, debug=True)
+    assert_parity(g, o)
+    assert g["stats"]["tile_pairs"] > 4 * part * 12
+
+
+def _lines_and_slivers(W, H, n=2400):
+    """n triangles by integer corners, and which of them are flat: every third
+    an ordinary one, one whose corners lie on one line, and the like with a
+    corner moved by a pixel."""
+    rng = np.random.default_rng(19)
+    tris, flat = [], []
+    for k in range(n):
+        flat.append(k % 3 == 1)
+        if k % 3 == 0:
+            tris.append([tuple(int(v) for v in rng.integers(0, [W + 1, H + 1])) for _ in range(3)])
+            continue
+        while True:                                    # a direction whose multiples stay inside
+            a, d, m = rng.integers(0, [W - 1, H - 1]), rng.integers(-9, 10, size=2), int(rng.integers(2, 12))
+            b, c = a + d * int(rng.integers(1, m)), a + d * m
+            if (d != 0).all() and (c >= 0).all() and c[0] <= W and c[1] <= H:
+                break
+        if k % 3 == 2:
+            c = np.clip(c + rng.integers(-1, 2, size=2), 0, [W, H])
+        tris.append([tuple(int(v) for v in (a, b, c)[j]) for j in rng.permutation(3)])
+    return tris, np.array(flat), rng
+
+
+@pytest.mark.parametrize("depth_test,blend", [
+    (A.SL_DEPTH_TEST_LESS_THAN, A.SL_BLEND_OFF), (A.SL_DEPTH_TEST_LESS_EQUAL, A.SL_BLEND_ALPHA),
+    (A.SL_DEPTH_TEST_GREATER_EQUAL, A.SL_BLEND_OFF), (A.SL_DEPTH_TEST_EQUAL, A.SL_BLEND_OFF)],
+    ids=["less", "lequal_blended", "gequal", "equal"])
+@pytest.mark.parametrize("size", [(97, 61), (640, 480)])
+def test_planes_that_are_not_finite(gpu_lib, oracle_lib, size, depth_test, blend):
+    """Triangles whose three snapped corners lie on one line: their planes are
+    infinite or NaN, and the rounding of their edges still covers some pixels.
+    With slivers and ordinary triangles around them; on the small target a batch
+    of small triangles by its number, on the large one not.  A NaN depth passes
+    no ordered test, and no bound may decide otherwise."""
+    W, H = size
+    tris, flat, rng = _lines_and_slivers(W, H)
+    zs = rng.uniform(-0.9, 0.9, size=len(tris)).astype(np.float32)
+    colors = rng.integers(0, 256, size=(len(tris), 3, 4))
+    o = A.SLContext(oracle_lib)
+    build_screen_triangles(o, [t for t, f in zip(tris, flat) if f], W, H, z=list(zs[flat]), colors=colors[flat].reshape(-1, 4),
+                           depth_mask=A.SL_DEPTH_MASK_OFF).render()
+    o.finish()
+    assert o.stats()["fragments_tested"] >= 10          # of the flat ones alone
+    def build(ctx):
+        s = build_screen_triangles(ctx, tris, W, H, z=list(zs), colors=colors.reshape(-1, 4), depth_test=depth_test, blend=blend)
+        if depth_test == A.SL_DEPTH_TEST_GREATER_EQUAL:
+            s.clear_depth = -1.0
+        return s
+    g, o = render_both(gpu_lib, oracle_lib, build)
     assert_parity(g, o)

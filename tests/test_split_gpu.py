@@ -3,10 +3,13 @@ cut into parts rasterised by separate workgroups and merged must give the
 frame the unsplit raster and the oracle give -- depth, colour, per-pixel
 last primitive and depth-pass count, counters -- for every depth-function
 class that splits (LESS / LESS_EQUAL and GREATER / GREATER_EQUAL with depth
-writes, any function without them), with ties, for points, lines and
-wireframe triangles, with the visibility attachment, and on the full-size
-benchmark frames.  Batches that do not split (blending, mixed functions)
-are unchanged."""
+writes, any function without them), with ties, for points, lines, wireframe
+and filled triangles, on every tile shape, in captured frames, with the
+visibility attachment and several outputs.  A tile of points, lines or
+wireframe triangles splits above four parts' records, one of filled triangles
+also needs more than 1/32 of the frame's entries: the cases that mean to split
+check that some tile must.  Batches that do not split (blending, mixed
+functions, filled triangles spread over many tiles) are unchanged."""
 import numpy as np
 import pytest
 
@@ -33,7 +36,19 @@ def _same(a, b):
         assert a["stats"][k] == b["stats"][k], k
 
 
-def _overlapping(ctx, n=400, W=96, H=64, seed=3, z="random", **kw):
+def _must_split(out, part, W, H, tile=(32, 16), filled=False):
+    """Some tile holds more records than four parts by the mean over the tiles,
+    and (filled) that mean is more than a 32nd of all."""
+    tiles = -(-W // tile[0]) * -(-H // tile[1])
+    assert out["stats"]["tile_pairs"] > 4 * part * tiles
+    assert not filled or tiles < 32
+
+
+MODES = {"filled": A.RENDER_MODE_TRIANGLES, "wire": A.RENDER_MODE_TRI_WIRE, "lines": A.RENDER_MODE_LINES,
+         "points": A.RENDER_MODE_POINTS}
+
+
+def _overlapping(ctx, n=400, W=96, H=64, seed=3, z="random", mode="filled", **kw):
     """n random triangles over a small target, so every tile holds far more
     records than a part."""
     rng = np.random.default_rng(seed)
@@ -43,7 +58,9 @@ def _overlapping(ctx, n=400, W=96, H=64, seed=3, z="random", **kw):
     else:
         zs = [[float(z)] * 3] * n                     # every fragment at one depth: ties everywhere
     cols = rng.integers(0, 256, size=(3 * n, 4))
-    return build_screen_triangles(ctx, tris, W, H, z=zs, colors=cols, **kw)
+    s = build_screen_triangles(ctx, tris, W, H, z=zs, colors=cols, **kw)
+    s.draws[0][1].mode = MODES[mode]                  # the same vertices as lines or points
+    return s
 
 
 @pytest.mark.parametrize("dtest,dmask,z", [
@@ -59,9 +76,10 @@ def _overlapping(ctx, n=400, W=96, H=64, seed=3, z="random", **kw):
 ], ids=["less", "lequal", "less_ties", "lequal_ties", "greater", "gequal_ties", "less_nomask", "off_nomask",
         "notequal_nomask"])
 @pytest.mark.parametrize("part", [1, 5])
-def test_split_matches_unsplit_and_oracle(gpu_lib, oracle_lib, dtest, dmask, z, part):
+@pytest.mark.parametrize("mode", list(MODES))
+def test_split_matches_unsplit_and_oracle(gpu_lib, oracle_lib, mode, dtest, dmask, z, part):
     def build(ctx, **kw):
-        s = _overlapping(ctx, z=z, depth_test=dtest, depth_mask=dmask)
+        s = _overlapping(ctx, z=z, mode=mode, depth_test=dtest, depth_mask=dmask)
         if dtest in (A.SL_DEPTH_TEST_GREATER_THAN, A.SL_DEPTH_TEST_GREATER_EQUAL):
             s.clear_depth = -1.0
         return s
@@ -69,7 +87,8 @@ def test_split_matches_unsplit_and_oracle(gpu_lib, oracle_lib, dtest, dmask, z, 
     g_whole, _ = render_both(gpu_lib, oracle_lib, _with_split(build, 0))
     assert_parity(g_split, o)
     _same(g_split, g_whole)
-    assert g_split["stats"]["fragments_tested"] > 50_000
+    _must_split(g_split, part, 96, 64, filled=mode == "filled")
+    assert g_split["stats"]["fragments_tested"] > {"filled": 50_000, "points": 1_000}.get(mode, 10_000)
 
 
 @pytest.mark.parametrize("part", [1, 3, 64])
@@ -83,6 +102,25 @@ def test_split_render_modes(gpu_lib, oracle_lib, kind, part):
         build = lambda ctx, **kw: scenes.build_random_triangles(ctx, seed=2, ntri=600, W=160, H=120, debug=True, wire=True)
     g, o = render_both(gpu_lib, oracle_lib, _with_split(build, part))
     assert_parity(g, o)
+    if part < 64:
+        _must_split(g, part, 160, 120)
+
+
+TILES = {0: (32, 16), 1: (32, 8), 2: (16, 16), 3: (16, 8), 7: (32, 32), 10: (8, 8), 11: (64, 64)}
+
+
+@pytest.mark.parametrize("mode", ["wire", "lines", "points"])
+@pytest.mark.parametrize("config", list(TILES))
+def test_split_modes_on_every_tile_shape(gpu_lib, oracle_lib, config, mode):
+    """The tiles of every size, some past the target's edges, all of them split."""
+    def build(ctx, **kw):
+        ctx.set_raster_config(config)
+        ctx.set_raster_split(2)
+        n = {"wire": 500, "lines": 1500, "points": 2500}[mode]
+        return _overlapping(ctx, n=n, W=150, H=101, seed=12, mode=mode, depth_test=A.SL_DEPTH_TEST_LESS_EQUAL)
+    g, o = render_both(gpu_lib, oracle_lib, build)
+    assert_parity(g, o)
+    _must_split(g, 2, 150, 101, TILES[config])
 
 
 @pytest.mark.parametrize("config", [0, 2, 5, 7, 9, 10, 11])
@@ -97,7 +135,8 @@ def test_split_on_every_tile_shape(gpu_lib, oracle_lib, config):
 
 
 def test_split_with_visibility_and_gradients(gpu_lib, oracle_lib):
-    """The differentiable views split: visibility bit-exact, gradients as the oracle's."""
+    """Asking for the split leaves views spread over many tiles as they are:
+    visibility bit-exact, gradients as the oracle's."""
     outs = []
     for lib, part in ((oracle_lib, 0), (gpu_lib, 2)):
         ctx = A.SLContext(lib)
@@ -127,12 +166,51 @@ def test_blended_batches_do_not_split(gpu_lib, oracle_lib):
 ])
 @pytest.mark.parametrize("part", [16, 64])
 def test_split_full_size_frames(gpu_lib, oracle_lib, name, build, kw, part):
+    """The benchmark's frames of filled triangles, spread over the target, with
+    the split asked for."""
     g, o = render_both(gpu_lib, oracle_lib, _with_split(build, part), debug=True, **kw)
     assert_parity(g, o)
 
 
+@pytest.mark.parametrize("mode,dtest,dmask", [
+    ("lines", A.SL_DEPTH_TEST_LESS_THAN, A.SL_DEPTH_MASK_ON), ("points", A.SL_DEPTH_TEST_GREATER_THAN, A.SL_DEPTH_MASK_ON),
+    ("wire", A.SL_DEPTH_TEST_OFF, A.SL_DEPTH_MASK_OFF), ("filled", A.SL_DEPTH_TEST_LESS_EQUAL, A.SL_DEPTH_MASK_ON)],
+    ids=["lines", "points_greater", "wire_nomask", "filled"])
+def test_split_modes_graph_replay(gpu_lib, oracle_lib, mode, dtest, dmask):
+    """Every replay of a captured frame with split tiles gives the oracle's image,
+    with eager frames of the same context between them."""
+    def build(ctx):
+        s = _overlapping(ctx, n=700, seed=5, mode=mode, depth_test=dtest, depth_mask=dmask)
+        if dtest == A.SL_DEPTH_TEST_GREATER_THAN:
+            s.clear_depth = -1.0
+        return s
+    so = build(A.SLContext(oracle_lib))
+    so.render()
+    o = so.read()
+    ctx = A.SLContext(gpu_lib)
+    ctx.set_raster_split(3)
+    s = build(ctx)
+    other = _overlapping(ctx, n=90, seed=6, W=200, H=40, mode="lines")
+    s.render()
+    ctx.frame_graph_capture()
+    ctx.finish()
+    for _ in range(4):
+        ctx.texture_set_texels(s.color, np.zeros((64, 96, 4), dtype=np.uint8))
+        ctx.reset_stats()
+        ctx.frame_graph_launch()
+        g = s.read()
+        assert np.array_equal(g["depth"].view(np.uint32), o["depth"].view(np.uint32))
+        assert np.array_equal(g["last"], o["last"])
+        assert np.array_equal(g["count"], o["count"])
+        assert int(np.abs(g["color"].astype(int) - o["color"].astype(int)).max()) <= 1
+        other.render()
+        ctx.finish()
+    assert int(o["count"].sum()) > 1000
+
+
 def test_split_graph_replay(gpu_lib, oracle_lib):
-    """A captured frame with split tiles replays to the oracle's image."""
+    """A captured frame replays to the oracle's image with the split asked for
+    (its spheres are spread over too many tiles to split)."""
     ctx = A.SLContext(gpu_lib)
     ctx.set_raster_split(8)
     s = scenes.build_sphere_scene(ctx, seed=4, n_instances=10, stacks=40, sectors=40, W=400, H=240, tex_size=64, debug=True)
