@@ -338,7 +338,7 @@ struct FrameCtrl
     uint32_t error;            // the emitting pass found a survivor that yields no record
     uint32_t emptyRecs;        // records that passed push_bin's tests but cover no pixel (not binned)
     // overflow | error << 1 of every earlier frame since the host last reset
-    // it: the per-frame reset (k_ctrl_reset) folds them in here before it
+    // it: the per-frame reset (k_frame_reset) folds them in here before it
     // clears them, so a replayed graph frame that overflowed is still
     // reported after later replays succeed
     uint32_t sticky;

@@ -8,8 +8,7 @@ namespace slg {
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
 hipError_t launch_vertex(const SetupParams& p, hipStream_t s);
 // Clears the control block before a frame, keeping (and adding the last
-// frame's overflow / error flags to) FrameCtrl::sticky, and na words of a and
-// nb of b.
+// frame's overflow / error flags to) FrameCtrl::sticky, and na words of a.
 hipError_t launch_frame_reset(FrameCtrl* ctrl, uint32_t* a, uint32_t na, hipStream_t s);
 hipError_t launch_setup(const SetupParams& p, uint64_t chunks, hipStream_t s);
 hipError_t launch_chunk_scan(const SetupParams& p, hipStream_t s);

@@ -319,11 +319,10 @@ __device__ __forceinline__ void write_pair_jobs(const SetupParams& P, uint32_t w
 //
 // k_setup runs the position part of the vertex programs, classification and
 // bin reservation for one triangle per lane and leaves, per chunk of
-// kSetupBlock triangles, the mask of triangles that yield records and the
-// chunk's packed (bin entries << kRecBits | records) total, which it also adds
-// to its group and super-group sums.  Nothing waits on another workgroup.
-// k_emit then turns the sums into each group's global offsets and writes the
-// records in submission order.
+// kSetupBlock triangles, a staging word per triangle that yields records and the
+// chunk's packed (bin entries << kRecBits | records) total.  Nothing waits on
+// another workgroup.  k_chunk_scan turns the totals into the chunks' offsets and
+// k_emit writes the records there, in submission order.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ unsigned long long wave_incl_scan(unsigned long long v)
 {

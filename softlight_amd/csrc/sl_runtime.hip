@@ -471,8 +471,9 @@ int make_plan(sl_context* c, const Batch& B, Plan& p)
 }
 
 // Setup's per-chunk buffer: ChunkInfo per chunk, kSetupBlock staging words
-// per chunk, the block sums (packed totals, then survivors; zeroed before
-// every frame) and the first chunk of every block of kSetupBlock survivors.
+// per chunk, the block sums (packed totals, then survivors; k_chunk_sums writes
+// them where there is more than one block, else nothing reads them) and the
+// chunk of every survivor.
 uint64_t chunk_blocks(uint64_t chunks) { return (chunks + kScanBlock - 1) / kScanBlock; }
 size_t chunk_buffer_bytes(uint64_t chunks)
 {
@@ -481,7 +482,9 @@ size_t chunk_buffer_bytes(uint64_t chunks)
 }
 
 // Part slots of the heavy-tile split: the per-slot buffers (first-pass
-// depths and part results, 28 B per tile pixel) kept within 64 MB.
+// depths and part results, 28 B per tile pixel) kept within 64 MB.  The split
+// tiles' winners (partWin, 4 B per pixel of at most a fifth as many tiles) come
+// on top.
 uint32_t split_parts(const Plan& p)
 {
     const size_t pix = (size_t)p.tc.tileW * p.tc.tileH;
@@ -661,7 +664,7 @@ RasterParams raster_params(const Plan& p, const Batch& B, FrameRes& R, bool have
     return rp;
 }
 
-// Control-block reset, block-sum reset and the setup passes: counting (the
+// The frame's reset and the setup passes: counting (the
 // events bracket it), chunk scan, emitting, clipping.
 int enqueue_front(sl_context* c, FrameRes& R, const Plan& p, const Batch& B, hipStream_t s,
                   hipEvent_t evSetup0 = nullptr, hipEvent_t evSetup1 = nullptr, hipEvent_t evClip0 = nullptr,
