@@ -1188,8 +1188,8 @@ __global__ __launch_bounds__(kSetupBlock, 7) void k_setup(SetupParams P)
 // k_chunk_scan: exclusive prefixes of the chunk totals and survivor counts.
 // Workgroup b owns chunks [b * kScanBlock, (b + 1) * kScanBlock): its offset is
 // the sum of the earlier blocks' totals (k_chunk_sums), the rest a workgroup
-// scan.  Also records, for every block of kSetupBlock survivors,
-// the chunk that holds its first survivor, and the frame totals.
+// scan.  Also writes the frame totals and, of few chunks, the survivors' chunks
+// (else k_surv_map does).
 __device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long v, unsigned long long* sRed)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -1325,10 +1325,8 @@ __global__ __launch_bounds__(64 * kSurvMapChunks) void k_surv_map(SetupParams P)
 }
 
 // k_emit: one workgroup per block of kEmitBlock survivors (grid-stride).  A
-// lane finds its survivor's chunk by searching the chunks' survivor prefixes
-// (kEmitBlock chunks per window in LDS, starting from the block's first
-// chunk), reads the staging word for its lane and offsets within the chunk,
-// re-fetches and re-classifies the triangle (the vertex programs are pure, so
+// lane reads its survivor's chunk from the map (survChunk) and the staging word
+// for its lane and offsets within the chunk, re-fetches and re-classifies the triangle (the vertex programs are pure, so
 // this gives the counting pass's bits) and writes its record, varyings and
 // bin entries at the chunk's prefix plus those offsets.  Straddling triangles
 // become clip jobs with their slots reserved.

@@ -125,7 +125,7 @@ def test_batched_meshes_1080p(gpu_lib, oracle_lib):
 
 # ---------------------------------------------------------------------------
 # The raster kernels the benchmark times: no debug attachments (so the
-# non-debug k_raster instances run) and the tuned tile of each workload.
+# non-debug k_raster_wave instances run) and the tuned tile of each workload.
 # ---------------------------------------------------------------------------
 TUNED = {
     "random": ("random:640x480:4096", scenes.build_random_triangles, dict(seed=0, ntri=4096, W=640, H=480)),
